@@ -55,9 +55,7 @@ typedef struct albd_counters {
     int heur_choice;                   /* the reference heuristic's choice     */
     float features[12];                /* selector features of the next level  */
     int persist_levels;                /* levels run by the small-frontier kernel */
-    int persist_in_queue;              /* 1: its last frontier is in st.queue   */
     int persist_error;                 /* 1: its grid barrier gave up           */
-    int pad_;
     unsigned int seq;                  /* host mailbox: sequence of the copy    */
     unsigned int pad2_;
     /* Unvisited-word list lengths, slot level % 3: built by that level's
@@ -72,11 +70,19 @@ typedef struct albd_counters {
 /* levels one small-frontier call may run (st.level_log holds 4 per level) */
 #define ALBD_PERSIST_LEVELS 4096
 
+/* most workgroups of the small-frontier kernel */
+#define ALBD_PERSIST_BLOCKS 256
+
 /* grid state of the small-frontier kernel, zeroed before each launch */
 typedef struct albd_persist {
-    unsigned long long barrier;      /* arrivals at the grid barrier        */
+    unsigned long long reserve;      /* found-list entries reserved         */
     unsigned int error;              /* a workgroup gave up waiting         */
     unsigned int pad_;
+    unsigned long long pad8_[6];     /* the slots start a cache line        */
+    /* arrivals at the grid barrier, by level parity: found vertices, their
+     * out-edges and the vertices put on the shared queue of each workgroup,
+     * each word with the level's tag in its top 16 bits                    */
+    unsigned long long slot[2][3][ALBD_PERSIST_BLOCKS];
 } albd_persist;
 
 /* Policy inputs of the select kernel. */
@@ -136,7 +142,7 @@ typedef struct albd_state {
     int32_t *active_next;       /* [nwords]  */
     albd_counters *ctr;         /* device counters */
     albd_slot *slots;           /* [ALBD_NSLOT] per-level counter slots */
-    int64_t *level_log;         /* [4*ALBD_PERSIST_LEVELS] found, edges, queue per level */
+    int64_t *level_log;         /* [4*ALBD_PERSIST_LEVELS] found, edges, shared queue per level */
     unsigned long long *pkey;   /* [npos] small-frontier (level, parent) keys, all ones at rest */
     albd_persist *persist;      /* small-frontier grid state */
 } albd_state;
@@ -302,8 +308,8 @@ ALBD_HIDDEN int albd_push_finalize(albd_ctx *c, const albd_graph *g, const albd_
  * while the new frontier has at most edge_cap out-edges and vertex_cap
  * vertices, at most max_levels levels.
  * On return the state is that of one finished push level: st.next holds the
- * last frontier's bitmap, its queue is in st.queue_next (ctr->persist_in_queue
- * = 0) or st.queue (= 1), ctr->qnext_len its length, the slots its counts;
+ * last frontier's bitmap, its queue is in st.queue_next, ctr->qnext_len its
+ * length (zero before the launch), the slots its counts;
  * ctr->persist_levels levels ran, st.level_log holds their sizes.  A grid
  * barrier that waits more than spin_limit polls sets ctr->persist_error and
  * the kernel ends early (the keys in st.pkey must then be refilled). */

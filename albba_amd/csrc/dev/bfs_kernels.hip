@@ -585,8 +585,8 @@ __global__ __launch_bounds__(kSelectBlock) void k_select(albd_graph g, albd_stat
 
 // Zero st.next (the select kernel has moved the counters and zeroed the
 // slots).  LB_SLOTS: zero the slots too (trial runs of one level);
-// LB_SMALL: the small-frontier kernel follows; zero its grid state, level
-// 0's counters and the error flag here instead of in launches of their own.
+// LB_SMALL: the small-frontier kernel follows; zero its grid state, its
+// levels' counters and the error flag here instead of in launches of their own.
 enum { LB_SLOTS = 1, LB_SMALL = 8 };
 
 __global__ __launch_bounds__(kBlock) void k_level_begin(albd_state st, int32_t nwords, int flags)
@@ -600,17 +600,17 @@ __global__ __launch_bounds__(kBlock) void k_level_begin(albd_state st, int32_t n
              i < (int64_t)(ALBD_NSLOT * sizeof(albd_slot) / 8); i += (int64_t)gridDim.x * kBlock)
             slots[i] = 0;
     }
-    if (blockIdx.x == 0) {
-        if (threadIdx.x == 0) {
-            if (flags & LB_SMALL) {
-                st.persist->barrier = 0;
-                st.persist->error = 0;
-                for (int f = 0; f < 4; ++f) st.level_log[f] = 0;
-                st.ctr->persist_error = 0;
-                // the levels run inside that kernel skip the select kernels
-                // that clear the list-count slots
-                for (int k = 0; k < 3; ++k) st.ctr->list_cnt[k] = 0;
-            }
+    if (flags & LB_SMALL) {
+        const int64_t i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x, step = (int64_t)gridDim.x * kBlock;
+        unsigned long long *p = reinterpret_cast<unsigned long long *>(st.persist);
+        static_assert(sizeof(albd_persist) % 8 == 0, "cleared by word");
+        for (int64_t i = i0; i < (int64_t)(sizeof(albd_persist) / 8); i += step) p[i] = 0;
+        for (int64_t i = i0; i < 4 * ALBD_PERSIST_LEVELS; i += step) st.level_log[i] = 0;
+        if (i0 == 0) {
+            st.ctr->persist_error = 0;
+            // the levels run inside that kernel skip the select kernels
+            // that clear the list-count slots
+            for (int k = 0; k < 3; ++k) st.ctr->list_cnt[k] = 0;
         }
     }
 }
@@ -1072,9 +1072,9 @@ __global__ __launch_bounds__(kBlock) void k_push_expand(albd_graph g, albd_state
 // High-diameter graphs spend thousands of levels with a few thousand
 // frontier vertices; a launch sequence and a host round trip per level would
 // dominate, and one workgroup alone is bound by its CU's gather rate.  A
-// grid of G co-resident workgroups runs the push levels back to
-// back with one grid barrier per level, until the next frontier has more
-// than edge_cap out-edges or more than vertex_cap vertices.
+// grid of G co-resident workgroups runs the push levels back to back with
+// one grid barrier per level, until the next frontier has more than edge_cap
+// out-edges or more than vertex_cap vertices.
 //
 // Exactness without a second barrier per level: every position p has a
 // 64-bit key, all ones outside this kernel.  An edge u -> v at level L does
@@ -1088,16 +1088,47 @@ __global__ __launch_bounds__(kBlock) void k_push_expand(albd_graph g, albd_state
 // launch: the vertices it finds get their level/parent words, visited bits
 // and keys back to all ones when it ends.
 //
-// Cross-workgroup data (found list, queues, keys, counters) moves through
-// device-coherent loads, stores and atomics; every wave waits for its own
-// memory operations before the barrier.
+// What bounds a level is its chain of dependent memory round trips, so
+// everything that is not the atomic or the barrier is off that chain:
+//   - a workgroup keeps the vertices it finds as its own part of the next
+//     frontier, as a list of their edges in LDS (no queue in memory between
+//     levels); vertices with more than kSmallDeg out-edges, and those beyond
+//     the list's kSmallEdges, go to a queue in memory that the workgroups
+//     share evenly at the next level;
+//   - the edges' columns, filters, degrees and vertex ids -- data that no
+//     level changes, but for the keys, which are only a filter -- are loaded
+//     while the workgroup waits at the barrier;
+//   - the barrier itself carries the level's counts: every workgroup stores
+//     its three counts, tagged with the level, into slots of its own, and
+//     three waves of every workgroup poll everybody's slots and sum them.
+// The slots alternate between two sets: a set is written again only two
+// levels later, when every workgroup has passed the barrier after reading it.
+// Cross-workgroup data (slots, shared queue, keys, found list) moves through
+// device-coherent loads, stores and atomics; a wave that wrote to the shared
+// queue waits for its stores before the barrier.
+//
+// A workgroup whose list grew past twice its part of the level's edges keeps
+// half a part of what it finds next and shares the rest.  Without that a
+// search stays with the workgroup that holds its root until the list is full:
+// one workgroup carried the first 4 096 levels of a 4 096 x 4 096 grid alone
+// and the kernel took 8.2 us per level instead of 5.5.
+//
+// Measured on grids of 0.6, 4.2 and 16.8 M vertices: 4.0, 4.6 and 5.5 us per
+// level, where a queue in memory between the levels, with its reservations
+// and a counting barrier, took 11.8, 12.3 and 13.6.  Of the 4 us about 1.3
+// are the atomic and the appends, 2.0 the loads behind the barrier (two
+// dependent misses) and 0.7 what the barrier waits beyond them.  Keeping all
+// workgroups on one XCD changed nothing at 0.6 M vertices (4.1 us) and cost at
+// 16.8 M (8.3 us with 32 workgroups): the misses go to memory either way.
 
-constexpr int kSmallBlock = 1024;
+constexpr int kSmallBlock = 512;
 constexpr int kSmallWaves = kSmallBlock / 64;
-
-constexpr int kSmallChunk = kSmallBlock;      // queue entries staged per pass
-constexpr int kSmallPer = 4;                  // edges per thread per window
-constexpr int kSmallWin = kSmallPer * kSmallBlock;
+constexpr int kSmallPer = 2;                           // edges per thread per window
+constexpr int kSmallEdges = kSmallPer * kSmallBlock;   // edges per window, and of the LDS list
+constexpr int kSmallDeg = 32;                          // most out-edges of a listed vertex
+constexpr int kSmallSlack = 64, kSmallKeep = 32;       // see the levels' end
+constexpr int kSmallFound = 1024;                      // found-list entries reserved at a time
+static_assert(kSmallFound >= kSmallEdges, "a window finds at most one reservation more");
 
 struct SmallArgs {
     albd_graph g;
@@ -1109,211 +1140,366 @@ struct SmallArgs {
     uint32_t spin_limit;
 };
 
+struct SmallLds {
+    // the next level's own edges: entry in push_col (-1: none) and source id
+    int32_t ecol[kSmallEdges];
+    uint32_t eou[kSmallEdges];
+    // a staged part of the shared queue
+    int64_t pre[kSmallBlock], start[kSmallBlock];
+    uint32_t ou[kSmallBlock];
+    int64_t scan[kSmallWaves];
+    // per level parity: listed edges << 32 | found; their out-edges; spilled
+    unsigned long long cnt[2], edges[2], spill[2];
+    unsigned long long tot[3]; // the grid's sums of found, edges, spilled
+    int64_t chunk[2];          // found-list reservations in use, by number & 1
+    int64_t reserved;          // reservations made so far
+    int ok;
+};
+
+// One edge of a lane: target position, its row and id, the source's id and
+// the filters.
+struct SmallEdge {
+    bool act;
+    int32_t v, start, deg;
+    uint32_t ou, ro;
+    uint64_t vis;
+    unsigned long long pk;
+};
+
+__device__ __forceinline__ void small_target(const albd_graph &g, const albd_state &st, SmallEdge &e)
+{
+    e.vis = e.act ? st.visited[e.v >> 6] : ~0ull;
+    e.pk = e.act ? st.pkey[e.v] : 0ull;
+    const int64_t a = e.act ? g.push_ptr[e.v] : 0, b = e.act ? g.push_ptr[e.v + 1] : 0;
+    e.start = (int32_t)a;
+    e.deg = (int32_t)(b - a);
+    e.ro = e.act ? (uint32_t)g.row_order[e.v] : 0u;
+}
+
+// Relax a window of edges (every lane of the wave calls): won lanes are their
+// vertices' discoverers; f gets their numbers among the level's found.
+__device__ __forceinline__ void small_relax(SmallLds &S, const albd_state &st, const SmallEdge (&e)[kSmallPer],
+                                            uint32_t lvl, int par, int cap, unsigned long long *spill_ctr,
+                                            int32_t *qb, bool (&won)[kSmallPer], uint32_t (&f)[kSmallPer], bool &spilled)
+{
+    const int lane = lane_id();
+#pragma unroll
+    for (int i = 0; i < kSmallPer; ++i) {
+        won[i] = false;
+        // unvisited at the launch and not found at an earlier level of it
+        if (e[i].act && !((e[i].vis >> (e[i].v & 63)) & 1ull) && (uint32_t)(e[i].pk >> 32) >= lvl)
+            won[i] = atomicMin(&st.pkey[e[i].v], ((unsigned long long)lvl << 32) | e[i].ou) == ~0ull;
+    }
+#pragma unroll
+    for (int i = 0; i < kSmallPer; ++i) {
+        const uint64_t m = __ballot(won[i]);
+        f[i] = 0;
+        if (m == 0) continue; // wave-uniform
+        const int32_t deg = won[i] ? e[i].deg : 0;
+        const bool listed = deg > 0 && deg <= kSmallDeg;
+        // exclusive prefix of the listed degrees, bit by bit
+        uint32_t pre = 0, tot = 0;
+#pragma unroll
+        for (int b = 0; b < 6; ++b) {
+            const uint64_t mb = __ballot(listed && ((deg >> b) & 1));
+            pre += (uint32_t)__popcll(mb & lanemask_lt(lane)) << b;
+            tot += (uint32_t)__popcll(mb) << b;
+        }
+        static_assert(kSmallDeg < 64, "six bits hold a listed degree");
+        const unsigned long long es = wave_sum((unsigned long long)(uint32_t)deg);
+        unsigned long long base = 0;
+        if (lane == 0) {
+            base = atomicAdd(&S.cnt[par], ((unsigned long long)tot << 32) | (unsigned long long)__popcll(m));
+            if (es) atomicAdd(&S.edges[par], es);
+        }
+        base = __shfl(base, 0, 64);
+        f[i] = (uint32_t)base + (uint32_t)__popcll(m & lanemask_lt(lane));
+        const unsigned long long e0 = (base >> 32) + pre;
+        const bool fits = listed && e0 + (unsigned long long)deg <= (unsigned long long)cap;
+        if (listed)
+            for (int k = 0; k < deg; ++k) {
+                if (e0 + k >= (unsigned long long)cap) break;
+                S.ecol[e0 + k] = fits ? e[i].start + k : -1;
+                S.eou[e0 + k] = e[i].ro;
+            }
+        const bool sp = deg > 0 && !fits;
+        const uint64_t ms = __ballot(sp);
+        if (ms) {
+            unsigned long long q = 0;
+            if (lane == 0) {
+                q = atomicAdd(spill_ctr, (unsigned long long)__popcll(ms));
+                atomicAdd(&S.spill[par], (unsigned long long)__popcll(ms));
+            }
+            q = __shfl(q, 0, 64);
+            if (sp) st_coherent(&qb[q + __popcll(ms & lanemask_lt(lane))], e[i].v);
+            spilled = true;
+        }
+    }
+}
+
+// the workgroup's found vertices of one window -> its reservations; F: found
+// before this level
+__device__ __forceinline__ void small_store_found(const SmallLds &S, int32_t *found,
+                                                  const SmallEdge (&e)[kSmallPer], const bool (&won)[kSmallPer],
+                                                  const uint32_t (&f)[kSmallPer], int64_t F)
+{
+#pragma unroll
+    for (int i = 0; i < kSmallPer; ++i)
+        if (won[i]) {
+            const int64_t at = F + f[i];
+            st_coherent(&found[S.chunk[(at / kSmallFound) & 1] + at % kSmallFound], e[i].v);
+        }
+}
+
+// room for a window's found vertices after the first `at` (thread 0)
+__device__ __forceinline__ void small_reserve(SmallLds &S, albd_persist *P, int64_t at)
+{
+    while (S.reserved < at / kSmallFound + 2) {
+        S.chunk[S.reserved & 1] = (int64_t)atomicAdd(&P->reserve, (unsigned long long)kSmallFound);
+        ++S.reserved;
+    }
+}
+
+// arrival: the workgroup's counts of a level (three lanes of one wave)
+__device__ __forceinline__ void small_arrive(const SmallLds &S, albd_persist *P, int par, unsigned int tag)
+{
+    const int lane = lane_id();
+    if (lane < 3) {
+        const unsigned long long x = lane == 0 ? (S.cnt[par] & 0xffffffffull) : (lane == 1 ? S.edges[par] : S.spill[par]);
+        st_coherent(&P->slot[tag & 1][lane][blockIdx.x], ((unsigned long long)tag << 48) | x);
+    }
+}
+
+// wait for every workgroup's arrival with `tag`; the wave sums word `k`
+__device__ __forceinline__ void small_poll(SmallLds &S, albd_persist *P, int k, unsigned int tag,
+                                           uint32_t spin_limit)
+{
+    const int lane = lane_id();
+    const unsigned int G = gridDim.x;
+    const unsigned long long *slot = P->slot[tag & 1][k];
+    unsigned long long sum = 0;
+    bool ok = true;
+    for (uint32_t spins = 0;; ++spins) {
+        bool all = true;
+        sum = 0;
+        for (unsigned int i = lane; i < G; i += 64) {
+            const unsigned long long x = ld_coherent(&slot[i]);
+            all = all && (x >> 48) == tag;
+            sum += x & ((1ull << 48) - 1);
+        }
+        if (__ballot(!all) == 0) break;
+        if (spins >= spin_limit || ((spins & 63) == 63 && ld_coherent(&P->error) != 0)) {
+            ok = false;
+            break;
+        }
+    }
+    sum = wave_sum(sum);
+    if (lane == 0) {
+        S.tot[k] = sum;
+        if (!ok) {
+            atomicOr(&P->error, 1u);
+            S.ok = 0;
+        }
+    }
+}
+
 __global__ __launch_bounds__(kSmallBlock) void k_push_small(SmallArgs a)
 {
     const albd_graph &g = a.g;
     const albd_state &st = a.st;
-    __shared__ int64_t s_pre[kSmallChunk];
-    __shared__ int64_t s_start[kSmallChunk];
-    __shared__ uint32_t s_ou[kSmallChunk];
-    __shared__ int64_t s_scan[kSmallWaves];
-    __shared__ int32_t s_found[kSmallWin];
-    __shared__ int32_t s_queue[kSmallWin];
-    __shared__ unsigned int s_nf, s_nq;
-    __shared__ unsigned long long s_bf, s_bq, s_sum;
-    __shared__ int s_ok;
+    __shared__ SmallLds S;
     albd_persist *P = st.persist;
-    // cumulative list of the vertices this launch finds, level after level
+    // every vertex this launch finds, in reservations of kSmallFound entries
     int32_t *found = reinterpret_cast<int32_t *>(st.prefix);
+    const int64_t found_cap = 2 * (g.npos + 1);
     int32_t *qa = st.queue, *qb = st.queue_next;
-    int64_t qlen = (int64_t)st.ctr->queue_len;
-    const int tid = threadIdx.x, lane = lane_id();
+    const int tid = threadIdx.x, lane = lane_id(), wid = tid >> 6;
     const unsigned int G = gridDim.x, w = blockIdx.x;
-    const int64_t gtid = (int64_t)w * kSmallBlock + tid, gthreads = (int64_t)G * kSmallBlock;
-    if (tid == 0) {
-        s_nf = 0;
-        s_nq = 0;
-        s_sum = 0;
+    // the waves that poll the slots: the last ones, which hold the fewest edges
+    const int poll = wid - (kSmallWaves - 3);
+    if (tid < 2) {
+        S.cnt[tid] = S.edges[tid] = S.spill[tid] = 0;
+        S.chunk[tid] = 0;
     }
-    __syncthreads();
-    int64_t fo = 0; // found[0, fo): the earlier levels of this launch
+    if (tid == 0) {
+        S.ok = 1;
+        S.reserved = 0;
+        small_reserve(S, P, 0);
+    }
+    int64_t ns = (int64_t)st.ctr->queue_len; // the shared queue's length
+    int64_t F = 0;                           // found by this workgroup before the level
+    SmallEdge e[kSmallPer];
+#pragma unroll
+    for (int i = 0; i < kSmallPer; ++i) e[i].act = false;
+    int cap = kSmallEdges; // edges the list takes at this level
     bool ok = true;
-    for (int k = 0; ok; ++k) {
-        const uint32_t lvl = (uint32_t)(a.level0 + k + 1);
-        // found, edges, queue entries of level k, and the level's count in
-        // the found list (appends go to found[fo + ...]).  Per level: a
-        // workgroup past the barrier may already append for the next level
-        // while another still reads this level's counts.
-        int64_t *cnt = st.level_log + 4 * k;
-        // expansion: workgroup w takes queue entries [q0, q1)
-        const int64_t per = (qlen + G - 1) / G;
-        const int64_t q0 = (int64_t)w * per, q1 = q0 + per < qlen ? q0 + per : qlen;
-        unsigned long long my_edges = 0;
-        for (int64_t base = q0; base < q1; base += kSmallChunk) { // uniform in the workgroup
-            const int cnt_e = (int)(q1 - base < kSmallChunk ? q1 - base : kSmallChunk);
-            int64_t a0 = 0, e0 = 0;
-            uint32_t o0 = 0;
-            if (tid < cnt_e) {
-                const int32_t u = ld_coherent(&qa[base + tid]);
-                a0 = g.push_ptr[u];
-                e0 = g.push_ptr[u + 1];
-                o0 = (uint32_t)g.row_order[u];
+    __syncthreads();
+    int k = 0;
+    uint32_t lvl = 0;
+    for (;; ++k) {
+        lvl = (uint32_t)(a.level0 + k + 1);
+        const int par = k & 1;
+        unsigned long long *spill_ctr = reinterpret_cast<unsigned long long *>(&st.level_log[4 * k + 2]);
+        if (tid == 0) S.cnt[par ^ 1] = S.edges[par ^ 1] = S.spill[par ^ 1] = 0;
+        bool won[kSmallPer], spilled = false;
+        uint32_t f[kSmallPer];
+        // the workgroup's own edges, loaded while it waited
+        small_relax(S, st, e, lvl, par, cap, spill_ctr, qb, won, f, spilled);
+        if (ns > 0) {
+            // its share of the queue in memory: entries [q0, q1)
+            small_store_found(S, found, e, won, f, F);
+            const int64_t per = (ns + G - 1) / G;
+            const int64_t q0 = (int64_t)w * per, q1 = q0 + per < ns ? q0 + per : ns;
+            for (int64_t base = q0; base < q1; base += kSmallBlock) { // uniform in the workgroup
+                const int cnt_e = (int)(q1 - base < kSmallBlock ? q1 - base : kSmallBlock);
+                int64_t a0 = 0, a1 = 0;
+                uint32_t o0 = 0;
+                if (tid < cnt_e) {
+                    const int32_t u = ld_coherent(&qa[base + tid]);
+                    a0 = g.push_ptr[u];
+                    a1 = g.push_ptr[u + 1];
+                    o0 = (uint32_t)g.row_order[u];
+                }
+                int64_t T;
+                const int64_t ex = block_scan_excl<kSmallBlock>(a1 - a0, &T, S.scan);
+                S.pre[tid] = ex;
+                S.start[tid] = a0;
+                S.ou[tid] = o0;
+                for (int64_t wb = 0; wb < T; wb += kSmallEdges) { // uniform
+                    // every found of the earlier windows has its place
+                    __syncthreads();
+                    if (tid == 0) small_reserve(S, P, F + (int64_t)(S.cnt[par] & 0xffffffffull));
+                    __syncthreads();
+                    SmallEdge x[kSmallPer];
+#pragma unroll
+                    for (int i = 0; i < kSmallPer; ++i) {
+                        const int64_t en = wb + i * kSmallBlock + tid;
+                        x[i].act = en < T;
+                        x[i].v = 0;
+                        x[i].ou = 0;
+                        if (x[i].act) {
+                            int lo = 0, hi = cnt_e;
+                            while (hi - lo > 1) {
+                                const int mid = (lo + hi) >> 1;
+                                if (S.pre[mid] <= en) lo = mid;
+                                else hi = mid;
+                            }
+                            x[i].v = g.push_col[S.start[lo] + (en - S.pre[lo])];
+                            x[i].ou = S.ou[lo];
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < kSmallPer; ++i) small_target(g, st, x[i]);
+                    bool xw[kSmallPer];
+                    uint32_t xf[kSmallPer];
+                    small_relax(S, st, x, lvl, par, cap, spill_ctr, qb, xw, xf, spilled);
+                    small_store_found(S, found, x, xw, xf, F);
+                }
+                __syncthreads(); // the staged entries are replaced
             }
-            int64_t T;
-            const int64_t ex = block_scan_excl<kSmallBlock>(e0 - a0, &T, s_scan);
-            s_pre[tid] = ex;
-            s_start[tid] = a0;
-            s_ou[tid] = o0;
-            __syncthreads();
-            for (int64_t wb = 0; wb < T; wb += kSmallWin) { // uniform
-                int64_t e = wb + (int64_t)tid * kSmallPer;
-                const int64_t e_end = e + kSmallPer < T ? e + kSmallPer : T;
-                int lo = 0;
-                if (e < e_end) {
-                    int hi = cnt_e;
-                    while (hi - lo > 1) {
-                        const int mid = (lo + hi) >> 1;
-                        if (s_pre[mid] <= e) lo = mid;
-                        else hi = mid;
-                    }
-                }
-                int32_t v[kSmallPer];
-                uint32_t ou[kSmallPer];
-                bool okv[kSmallPer];
-#pragma unroll
-                for (int i = 0; i < kSmallPer; ++i) {
-                    okv[i] = e < e_end;
-                    v[i] = 0;
-                    ou[i] = 0;
-                    if (okv[i]) {
-                        while (lo + 1 < cnt_e && s_pre[lo + 1] <= e) ++lo;
-                        v[i] = g.push_col[s_start[lo] + (e - s_pre[lo])];
-                        ou[i] = s_ou[lo];
-                        ++e;
-                    }
-                }
-                uint64_t vis[kSmallPer];
-                unsigned long long pk[kSmallPer];
-                int64_t d0[kSmallPer], d1[kSmallPer];
-                // the filters and the out-degree together: one round trip
-                // ahead of the atomic instead of one after it
-#pragma unroll
-                for (int i = 0; i < kSmallPer; ++i) {
-                    vis[i] = okv[i] ? st.visited[v[i] >> 6] : ~0ull;
-                    pk[i] = okv[i] ? st.pkey[v[i]] : 0ull;
-                    d0[i] = okv[i] ? g.push_ptr[v[i]] : 0;
-                    d1[i] = okv[i] ? g.push_ptr[v[i] + 1] : 0;
-                }
-                bool won[kSmallPer];
-#pragma unroll
-                for (int i = 0; i < kSmallPer; ++i) {
-                    won[i] = false;
-                    // unvisited at the launch and not found at an earlier
-                    // level of it
-                    if (!((vis[i] >> (v[i] & 63)) & 1ull) && (uint32_t)(pk[i] >> 32) >= lvl) {
-                        const unsigned long long key =
-                            ((unsigned long long)lvl << 32) | (unsigned long long)ou[i];
-                        const unsigned long long old = atomicMin(&st.pkey[v[i]], key);
-                        won[i] = old == ~0ull;
-                    }
-                }
-                int64_t dv[kSmallPer];
-#pragma unroll
-                for (int i = 0; i < kSmallPer; ++i)
-                    dv[i] = won[i] ? d1[i] - d0[i] : 0;
-#pragma unroll
-                for (int i = 0; i < kSmallPer; ++i) {
-                    const unsigned int pf = wave_append(&s_nf, won[i]);
-                    if (won[i]) s_found[pf] = v[i];
-                    const unsigned int pq = wave_append(&s_nq, dv[i] > 0);
-                    if (dv[i] > 0) s_queue[pq] = v[i];
-                    my_edges += (unsigned long long)dv[i];
-                }
-                __syncthreads();
-                // flush the window's lists: one reservation per list
-                const unsigned int nf = s_nf, nq = s_nq;
-                if (tid == 0) {
-                    s_bf = nf ? atomicAdd(reinterpret_cast<unsigned long long *>(&cnt[3]), (unsigned long long)nf)
-                              : 0;
-                    s_bq = nq ? atomicAdd(reinterpret_cast<unsigned long long *>(&cnt[2]),
-                                          (unsigned long long)nq)
-                              : 0;
-                }
-                __syncthreads();
-                const unsigned long long bf = s_bf, bq = s_bq;
-                for (unsigned int i = tid; i < nf; i += kSmallBlock) st_coherent(&found[fo + bf + i], s_found[i]);
-                for (unsigned int i = tid; i < nq; i += kSmallBlock) st_coherent(&qb[bq + i], s_queue[i]);
-                __syncthreads();
-                if (tid == 0) {
-                    s_nf = 0;
-                    s_nq = 0;
-                }
-            }
-            __syncthreads(); // s_pre and friends are restaged
         }
-        my_edges = wave_sum(my_edges);
-        if (lane == 0 && my_edges) atomicAdd(&s_sum, my_edges);
+        // the shared queue's entries are in place before the arrival
+        if (spilled) __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        if (tid == 0) {
-            if (s_sum) atomicAdd(reinterpret_cast<unsigned long long *>(&cnt[1]), s_sum);
-            s_sum = 0;
-            // the next level's counters, unused until after the barrier
-            if (w == 0 && k + 1 < a.max_levels)
-                for (int f = 0; f < 4; ++f) st_coherent(&cnt[4 + f], (int64_t)0);
+        if (poll == 0) small_arrive(S, P, par, (unsigned int)(k + 1));
+        // off the chain: the found list, and everything about the next
+        // level's own edges but the atomic
+        if (ns == 0) small_store_found(S, found, e, won, f, F);
+        const unsigned long long mine = S.cnt[par];
+        F += (int64_t)(mine & 0xffffffffull);
+        const int T = (int)((mine >> 32) < (unsigned long long)cap ? (mine >> 32) : (unsigned long long)cap);
+#pragma unroll
+        for (int i = 0; i < kSmallPer; ++i) {
+            const int en = i * kSmallBlock + tid;
+            const int32_t at = en < T ? S.ecol[en] : -1;
+            e[i].act = at >= 0;
+            e[i].ou = e[i].act ? S.eou[en] : 0;
+            e[i].v = e[i].act ? g.push_col[at] : 0;
         }
-        ok = team_sync(&P->barrier, &P->error, G, a.spin_limit, &s_ok);
+#pragma unroll
+        for (int i = 0; i < kSmallPer; ++i) small_target(g, st, e[i]);
+        if (poll >= 0) small_poll(S, P, poll, (unsigned int)(k + 1), a.spin_limit);
+        __syncthreads();
+        ok = S.ok != 0;
         if (!ok) break;
-        const int64_t na = ld_coherent(&cnt[3]);
-        const int64_t total = fo + na;
-        const int64_t edges = ld_coherent(&cnt[1]);
-        const int64_t nq = ld_coherent(&cnt[2]);
-        if (w == 0 && tid == 0) st_coherent(&cnt[0], na);
-        const bool last = na == 0 || edges > a.edge_cap || na > a.vertex_cap ||
-                          k + 1 >= a.max_levels;
-        if (last) {
-            // this level's vertices: level, parent, visited and next bits;
-            // then every key set by this launch goes back to all ones
-            unsigned long long my_words = 0;
-            for (int64_t i = fo + gtid; i < total; i += gthreads) {
-                const int32_t v = ld_coherent(&found[i]);
-                const unsigned long long key = ld_coherent(&st.pkey[v]);
-                st.lp[v] = key;
-                const uint64_t bit = 1ull << (v & 63);
-                atomicOr(reinterpret_cast<unsigned long long *>(&st.visited[v >> 6]), bit);
-                const unsigned long long old =
-                    atomicOr(reinterpret_cast<unsigned long long *>(&st.next[v >> 6]), bit);
-                my_words += old == 0 ? 1 : 0;
-                st.pkey[v] = ~0ull;
-            }
-            // the earlier levels' vertices: level, parent and visited too
-            for (int64_t i = gtid; i < fo; i += gthreads) {
-                const int32_t v = ld_coherent(&found[i]);
-                st.lp[v] = ld_coherent(&st.pkey[v]); // the same (level, parent) packing
-                atomicOr(reinterpret_cast<unsigned long long *>(&st.visited[v >> 6]), 1ull << (v & 63));
-                st.pkey[v] = ~0ull;
-            }
-            my_words = wave_sum(my_words);
-            if (lane == 0 && my_words) atomicAdd(&st.slots[1 + (w % (ALBD_NSLOT - 1))].next_words, my_words);
-            if (w == 0 && tid == 0) {
-                st.slots[0].next_count = (unsigned long long)na;
-                st.slots[0].next_edges = (unsigned long long)edges;
-                st.ctr->qnext_len = (unsigned long long)nq;
-                st.ctr->persist_levels = k + 1;
-                st.ctr->persist_in_queue = qb == st.queue ? 1 : 0;
-            }
-            break;
+        const int64_t na = (int64_t)S.tot[0], edges = (int64_t)S.tot[1];
+        ns = (int64_t)S.tot[2];
+        if (w == 0 && tid == 0) {
+            st.level_log[4 * k] = na;
+            st.level_log[4 * k + 1] = edges;
         }
+        if (na == 0 || edges > a.edge_cap || na > a.vertex_cap || k + 1 >= a.max_levels) break;
         // an intermediate level: the select kernel sees only the last one,
         // so these counts go straight into the running totals
         if (w == 0 && tid == 0) {
             st.ctr->reached += (unsigned long long)na;
             st.ctr->reached_edges += (unsigned long long)edges;
         }
-        fo = total;
+        if (tid == 0) small_reserve(S, P, F);
+        // a workgroup that holds more than twice its part of the edges keeps
+        // half a part of what it finds next and shares the rest
+        const int64_t part = edges / G;
+        cap = (int64_t)(mine >> 32) > 2 * part + kSmallSlack
+                  ? (int)(part / 2 < kSmallKeep ? kSmallKeep : (part / 2 > kSmallEdges ? kSmallEdges : part / 2))
+                  : kSmallEdges;
         int32_t *t = qa;
         qa = qb;
         qb = t;
-        qlen = nq;
+    }
+    if (ok) {
+        const unsigned long long na = S.tot[0], edges = S.tot[1];
+        // the unused ends of the reservations hold no vertex
+        for (int64_t j = F + tid; j < S.reserved * kSmallFound; j += kSmallBlock) {
+            const int64_t at = S.chunk[(j / kSmallFound) & 1] + j % kSmallFound;
+            if (at < found_cap) st_coherent(&found[at], (int32_t)-1);
+        }
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        // (the counts of this arrival are not used)
+        if (poll == 0) small_arrive(S, P, k & 1, (unsigned int)(k + 2));
+        if (poll >= 0) small_poll(S, P, poll, (unsigned int)(k + 2), a.spin_limit);
+        __syncthreads();
+        ok = S.ok != 0;
+        if (ok) {
+            // level, parent and visited of every vertex found, and its key
+            // back to all ones; the last level's also into the next frontier
+            // and its queue
+            int64_t total = (int64_t)ld_coherent(&P->reserve);
+            if (total > found_cap) total = found_cap;
+            unsigned long long my_words = 0;
+            for (int64_t b = ((int64_t)w * kSmallWaves + wid) * 64; b < total;
+                 b += (int64_t)G * kSmallBlock) { // uniform in the wave
+                const int64_t i = b + lane;
+                const int32_t v = i < total ? ld_coherent(&found[i]) : -1;
+                bool queued = false;
+                if (v >= 0) {
+                    const unsigned long long key = ld_coherent(&st.pkey[v]);
+                    st.lp[v] = key; // the same (level, parent) packing
+                    const uint64_t bit = 1ull << (v & 63);
+                    atomicOr(reinterpret_cast<unsigned long long *>(&st.visited[v >> 6]), bit);
+                    st.pkey[v] = ~0ull;
+                    if ((uint32_t)(key >> 32) == lvl) {
+                        my_words +=
+                            atomicOr(reinterpret_cast<unsigned long long *>(&st.next[v >> 6]), bit) == 0 ? 1 : 0;
+                        queued = g.push_ptr[v + 1] > g.push_ptr[v];
+                    }
+                }
+                const uint64_t mq = __ballot(queued);
+                if (mq) {
+                    unsigned long long q = 0;
+                    if (lane == 0) q = atomicAdd(&st.ctr->qnext_len, (unsigned long long)__popcll(mq));
+                    q = __shfl(q, 0, 64);
+                    if (queued) st.queue_next[q + __popcll(mq & lanemask_lt(lane))] = v;
+                }
+            }
+            my_words = wave_sum(my_words);
+            if (lane == 0 && my_words) atomicAdd(&st.slots[1 + (w % (ALBD_NSLOT - 1))].next_words, my_words);
+            if (w == 0 && tid == 0) {
+                st.slots[0].next_count = na;
+                st.slots[0].next_edges = edges;
+                st.ctr->persist_levels = k + 1;
+            }
+        }
     }
     if (!ok && tid == 0) st.ctr->persist_error = 1;
 }
@@ -1597,11 +1783,20 @@ int albd_push_small(albd_ctx *c, const albd_graph *g, const albd_state *st, int3
     // after spin_limit polls (ctr->persist_error), never hang.
     int per_cu = 0;
     HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_push_small, kSmallBlock, 0));
-    const int cap = per_cu * albd_num_cus(c);
-    if (blocks <= 0) blocks = 64;
-    if (blocks > cap) blocks = cap;
-    if (blocks < 1) return albd_set_error_msg(ALBBA_EHIP, "small-frontier kernel cannot be resident");
-    // level 0's counters, the grid state and the error flag were zeroed by
+    int64_t cap = (int64_t)per_cu * albd_num_cus(c);
+    if (cap < 1) return albd_set_error_msg(ALBBA_EHIP, "small-frontier kernel cannot be resident");
+    if (cap > ALBD_PERSIST_BLOCKS) cap = ALBD_PERSIST_BLOCKS;
+    // the found list (2 (npos + 1) entries) holds every vertex and the up to
+    // two unfilled reservations of every workgroup
+    if (cap > g->npos / (2 * kSmallFound)) cap = g->npos / (2 * kSmallFound);
+    if (cap < 1) cap = 1;
+    // More workgroups shorten each one's part of a level but lengthen the
+    // barrier: measured us per level with 16, 32 and 64 workgroups on grids
+    // of 0.6, 4.2 and 16.8 M vertices: 4.04, 4.30, 4.65; 6.22, 4.91, 4.64;
+    // 9.43, 6.84, 5.56 (96 workgroups: 5.12, 4.96, 5.42).
+    if (blocks <= 0) blocks = g->n < (1 << 20) ? 16 : (g->n < (1 << 21) ? 32 : 64);
+    if (blocks > cap) blocks = (int32_t)cap;
+    // the grid state, the levels' counters and the error flag were zeroed by
     // the level-begin kernel (LB_SMALL)
     SmallArgs a{*g, *st, level0, max_levels, edge_cap, vertex_cap, spin_limit};
     hipLaunchKernelGGL(k_push_small, dim3(blocks), dim3(kSmallBlock), 0, albd_stream(c), a);

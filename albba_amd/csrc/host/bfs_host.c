@@ -900,13 +900,6 @@ static int run_small(albba_graph *G, const loop_state *ls, int32_t level, int64_
         return albba_fail(ALBBA_EHIP, "small-frontier kernel: grid barrier timed out");
     }
     *nlev = hc->persist_levels;
-    if (hc->persist_in_queue) {
-        /* the last frontier's queue is in st.queue: swap so that it is in
-         * queue_next, where a finished push level leaves it */
-        int32_t *q = G->st.queue;
-        G->st.queue = G->st.queue_next;
-        G->st.queue_next = q;
-    }
     return 0;
 }
 
@@ -1040,6 +1033,10 @@ static int script_at(const albba_graph *G, const albba_bfs_opts *o, int32_t leve
     return choice_ok(G, o->script[level]) ? o->script[level] : -1;
 }
 
+/* small levels that did not double before the learned policy's BFS goes on
+ * in the small-frontier kernel */
+#define SLOW_LEVELS 4
+
 static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs_opts *opts_in,
                    albba_bfs_stats *stats, bfs_events ev)
 {
@@ -1083,6 +1080,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
          : (script_at(G, &opts, (L) + 1) == ALBBA_CHOICE_PUSH ? INT64_MAX : (int64_t)-1))
     loop_state ls = {1, 0, 0, 0, 0};
     int small_streak = 0; /* consecutive plain push levels that stayed small */
+    int slow_streak = 0;  /* consecutive small levels that did not double */
     int32_t level = 0;
     int rc;
     /* The heuristic, learned and scripted policies prepare every level
@@ -1172,12 +1170,25 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
          * (high-diameter graphs), which the streak detects, not on the one or
          * two small levels of a power-law BFS. */
         const int64_t first_edges = (int64_t)hc->frontier_edges;
-        const int small_ok = choice == ALBBA_CHOICE_PUSH && opts.small_frontier_edges > 0 &&
-                             (policy == ALBBA_SWITCH_HEURISTIC || policy == ALBBA_SWITCH_LEARNED) &&
-                             first_edges <= opts.small_frontier_edges && frontier <= push_vertex_cap;
+        const int size_ok = opts.small_frontier_edges > 0 &&
+                            (policy == ALBBA_SWITCH_HEURISTIC || policy == ALBBA_SWITCH_LEARNED) &&
+                            first_edges <= opts.small_frontier_edges && frontier <= push_vertex_cap;
+        /* The learned selector ranks one level's kernels and does not know the
+         * persistent one, so on a small high-diameter graph it may pull level
+         * after level (a 601 x 1009 grid: all but two of 1 429 levels, 22 us
+         * each against 4 us in the persistent kernel).  After SLOW_LEVELS
+         * small levels in a row that did not double, its BFS goes on in the
+         * persistent kernel whatever it ranks first; the few small levels at
+         * either end of a power-law or random graph's BFS are fewer than that
+         * or grow faster. */
+        slow_streak = size_ok && frontier <= 2 * frontier_prev ? slow_streak + 1 : 0;
+        const int slow = policy == ALBBA_SWITCH_LEARNED && slow_streak > SLOW_LEVELS && !queued_push &&
+                         queued_pull < 0;
+        if (slow) choice = ALBBA_CHOICE_PUSH;
+        const int small_ok = choice == ALBBA_CHOICE_PUSH && size_ok;
         /* (never with push kernels queued: they are queued only while
          * small_streak < 2) */
-        const int small = small_ok && small_streak >= 2 && !queued_push;
+        const int small = slow || (small_ok && small_streak >= 2 && !queued_push);
         small_streak = small_ok && !small ? small_streak + 1 : 0;
         int nlev = 1;
         int queue_built = 1;
@@ -1222,7 +1233,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
              * large frontiers.  The kernels read the choice themselves and
              * return at once if it differs; the host then queues the chosen
              * kernels behind them.  Not with per-level events, which must
-             * bracket the chosen kernels, and no push while the
+             * bracket the chosen kernels, and nothing while the
              * small-frontier kernel may take the next level. */
             queued_pull = -1;
             queued_push = 0;
@@ -1234,6 +1245,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
                 else if (small_streak >= 2)
                     guess = -1;
             }
+            if (policy == ALBBA_SWITCH_LEARNED && slow_streak >= SLOW_LEVELS) guess = -1;
             if (sel.forced >= 0) {
                 /* a scripted level is known: queue it, except a push that
                  * would need the queue listed from the bitmap first */
@@ -1315,7 +1327,8 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
         }
         if (!spec) commit_pointers(G, &ls, choice, 1);
         commit_counts(&ls, choice, &sums);
-        frontier_prev = frontier;
+        /* (a run of levels says nothing about the growth at its end) */
+        frontier_prev = small ? (int64_t)hc->frontier : frontier;
         frontier = (int64_t)hc->frontier;
         level += nlev;
     }

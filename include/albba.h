@@ -219,7 +219,9 @@ typedef struct albba_bfs_opts {
      * growing frontier), the following levels run inside one persistent push
      * kernel (one grid barrier per level, no host round trip) until the
      * frontier outgrows the cap or the heuristic's push threshold (0
-     * disables; default 65536).  Results are identical either way. */
+     * disables; default 65536).  The learned policy enters it too after five
+     * such frontiers in a row that did not double, whatever it would choose.
+     * Results are identical either way. */
     int64_t small_frontier_edges;
     int32_t small_frontier_blocks; /* workgroups of that kernel (0: default)    */
     int32_t reserved_;
