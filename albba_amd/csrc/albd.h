@@ -385,14 +385,13 @@ ALBD_HIDDEN int albd_batch_scratch(albd_ctx *c, void **ptr, size_t *bytes);
 ALBD_HIDDEN double albd_clock_ticks_per_ms(albd_ctx *c);
 
 /* ---- selector MLP (mlp.hip); every pointer is device memory ---- */
-#define ALBD_MLP_SCRATCH_PER_SAMPLE (32 + 32 + 4 + 32 + 32 + 1)
 /* samples per partial sum of the gradient */
 #define ALBD_MLP_CHUNK 64
-/* floats of scratch albd_mlp_loss_grad needs for ns samples: the per-sample
- * activations and errors, then one partial gradient (+ loss) per chunk */
-#define ALBD_MLP_SCRATCH_FLOATS(ns)                                                                \
-    ((size_t)(ns) * ALBD_MLP_SCRATCH_PER_SAMPLE +                                                  \
-     (((size_t)(ns) + ALBD_MLP_CHUNK - 1) / ALBD_MLP_CHUNK) * (ALBBA_MLP_NPARAM + 1))
+/* floats of one chunk's partial gradient and loss (rows of 16-byte multiples) */
+#define ALBD_MLP_PARTIAL ((ALBBA_MLP_NPARAM + 1 + 3) / 4 * 4)
+/* floats of scratch the gradient of ns samples needs: one partial per chunk */
+#define ALBD_MLP_SCRATCH_FLOATS(ns) \
+    ((((size_t)(ns) + ALBD_MLP_CHUNK - 1) / ALBD_MLP_CHUNK) * ALBD_MLP_PARTIAL)
 /* out[ns*4] = MLP(x[ns*12]) */
 ALBD_HIDDEN int albd_mlp_forward(albd_ctx *c, const float *params, const float *x, int32_t ns,
                                  float *out);
@@ -401,8 +400,11 @@ ALBD_HIDDEN int albd_mlp_forward(albd_ctx *c, const float *params, const float *
 ALBD_HIDDEN int albd_mlp_loss_grad(albd_ctx *c, const float *params, const float *x,
                                    const float *t, int32_t ns, float *scratch, float *grad,
                                    float *loss);
-ALBD_HIDDEN int albd_mlp_adam(albd_ctx *c, float *params, const float *grad, float *m, float *v,
-                              int32_t np, float lr, float b1, float b2, float eps, int32_t step);
+/* one training step: the gradient as above, then Adam on params (m, v: its
+ * moments; step counts from 1) */
+ALBD_HIDDEN int albd_mlp_train_step(albd_ctx *c, float *params, const float *x, const float *t, int32_t ns,
+                                    float *scratch, float *grad, float *loss, float *m, float *v, float lr,
+                                    float b1, float b2, float eps, int32_t step);
 
 #ifdef __cplusplus
 }

@@ -5,12 +5,12 @@
 // Parameter layout (1604 floats): W1[32][12], b1[32], W2[32][32], b2[32],
 // W3[4][32], b3[4]; W[j][i] multiplies input i into unit j.
 //
-// The gradient is computed in deterministic passes without atomics: one
-// thread per sample stores activations and back-propagated errors; a block
-// per chunk of 64 samples stages them in LDS and sums every parameter's
-// contributions over its chunk in sample order; one thread per parameter then
-// adds the chunks' partial sums in chunk order.  A run reproduces bit for bit
-// and can be compared with a CPU restatement.
+// The gradient is computed in two deterministic passes without atomics: a
+// block per chunk of 64 samples runs them forward and backward in LDS and sums
+// every parameter's contributions over its chunk in sample order; then the
+// chunks' partial sums are added in chunk order, and a training step updates
+// the parameters in the same pass.  A run reproduces bit for bit and can be
+// compared with a CPU restatement.
 #include "dev_common.h"
 #include "../../../include/albba.h"
 
@@ -60,123 +60,259 @@ __global__ __launch_bounds__(256) void k_forward(const float *params, const floa
     for (int k = 0; k < NO; ++k) out[(size_t)s * NO + k] = y[k];
 }
 
-// scratch layout per sample block: h1[ns][32] h2[ns][32] dy[ns][4] dh1[ns][32]
-// dh2[ns][32] lossv[ns]
-__global__ __launch_bounds__(256) void k_sample_pass(const float *params, const float *x,
-                                                     const float *t, int32_t ns, float *scratch)
+// Loss and gradient of a chunk of CH samples, one block each: partial[c][p]
+// for every parameter p, partial[c][NP] the chunk's squared errors.
+//
+// Activations and errors stay in LDS, unit-major (a unit's samples are
+// consecutive), so that a thread works on one unit and four samples, or on two
+// weights and four samples at a time, with 16-byte LDS reads; every sum
+// runs in the order of the forward above and, over the samples, in sample
+// order.  The rows are padded against bank conflicts: activations to CH + 4
+// (rows stay 16-byte aligned), weights to an odd length.  Writing the
+// activations to memory for a second kernel, one thread per sample with its
+// vectors in scratch memory, took 23 + 13 us at 9 000 samples (141 chunks);
+// this takes 10.2 us there with 512 threads and 13.4 with 256, latency of LDS
+// and barriers: the arithmetic is 0.6 us.
+constexpr int CH = ALBD_MLP_CHUNK;
+constexpr int PS = ALBD_MLP_PARTIAL; // floats per chunk's partial sums
+constexpr int LS = CH + 4;
+constexpr int S1 = NI + 1, S2 = H1 + 1, S3 = H2 + 1;
+static_assert(CH == 64 && H1 == 32 && H2 == 32 && NO == 4 && NI % 4 == 0, "the block's work split");
+static_assert(PS >= NP + 1, "a chunk's sums");
+
+struct ChunkLds {
+    float w1[H1 * S1], b1[H1], w2[H2 * S2], b2[H2], w3[NO * S3], b3[NO];
+    alignas(16) float x[NI * LS], h1[H1 * LS], h2[H2 * LS], e[NO * LS], dy[NO * LS], d1[H1 * LS], d2[H2 * LS],
+        lv[LS];
+};
+
+constexpr int GT = 512;                // threads per block
+constexpr int U = CH * 32 / GT;        // samples per thread
+static_assert(U % 4 == 0, "16-byte reads");
+
+// acc[u] += w * v[u]
+__device__ __forceinline__ void fma_samples(float (&acc)[U], float w, const float *v)
 {
-    __shared__ float sp[NP];
-    load_params(params, sp);
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= ns) return;
-    float *H1s = scratch, *H2s = H1s + (size_t)ns * H1, *DY = H2s + (size_t)ns * H2,
-          *DH1 = DY + (size_t)ns * NO, *DH2 = DH1 + (size_t)ns * H1, *LV = DH2 + (size_t)ns * H2;
-    float xi[NI], h1[H1], h2[H2], y[NO], dy[NO], dh2[H2];
-    for (int i = 0; i < NI; ++i) xi[i] = x[(size_t)s * NI + i];
-    forward_one(sp, xi, h1, h2, y);
-    const float scale = 2.0f / ((float)ns * (float)NO);
-    float l = 0.f;
-    for (int k = 0; k < NO; ++k) {
-        const float e = y[k] - t[(size_t)s * NO + k];
-        l = fmaf(e, e, l);
-        dy[k] = scale * e;
-        DY[(size_t)s * NO + k] = dy[k];
-    }
-    LV[s] = l;
-    for (int i = 0; i < H2; ++i) {
-        float a = 0.f;
-        for (int k = 0; k < NO; ++k) a = fmaf(sp[OW3 + k * H2 + i], dy[k], a);
-        dh2[i] = h2[i] > 0.f ? a : 0.f;
-        DH2[(size_t)s * H2 + i] = dh2[i];
-        H2s[(size_t)s * H2 + i] = h2[i];
-    }
-    for (int i = 0; i < H1; ++i) {
-        float a = 0.f;
-        for (int j = 0; j < H2; ++j) a = fmaf(sp[OW2 + j * H1 + i], dh2[j], a);
-        DH1[(size_t)s * H1 + i] = h1[i] > 0.f ? a : 0.f;
-        H1s[(size_t)s * H1 + i] = h1[i];
+#pragma unroll
+    for (int u = 0; u < U; u += 4) {
+        const float4 p = *reinterpret_cast<const float4 *>(v + u);
+        acc[u] = fmaf(w, p.x, acc[u]);
+        acc[u + 1] = fmaf(w, p.y, acc[u + 1]);
+        acc[u + 2] = fmaf(w, p.z, acc[u + 2]);
+        acc[u + 3] = fmaf(w, p.w, acc[u + 3]);
     }
 }
 
-constexpr int CH = ALBD_MLP_CHUNK;
-
-// Partial sums of chunk blockIdx.x (samples [CH*c, CH*c + m)): partial[c][p]
-// for every parameter p, partial[c][NP] the chunk's squared errors.
-__global__ __launch_bounds__(256) void k_param_partial(const float *x, int32_t ns, const float *scratch,
-                                                       float *partial)
+// sum over the chunk's samples, in order, of a[q] * b[q]
+__device__ __forceinline__ float dot_samples(const float *a, const float *b)
 {
-    __shared__ float sh1[CH * H1], sh2[CH * H2], sdy[CH * NO], sdh1[CH * H1], sdh2[CH * H2], sx[CH * NI],
-        slv[CH];
-    const float *H1s = scratch, *H2s = H1s + (size_t)ns * H1, *DY = H2s + (size_t)ns * H2,
-                *DH1 = DY + (size_t)ns * NO, *DH2 = DH1 + (size_t)ns * H1, *LV = DH2 + (size_t)ns * H2;
-    const int c = blockIdx.x;
+    float g = 0.f;
+#pragma unroll
+    for (int q = 0; q < CH; q += 4) {
+        const float4 u = *reinterpret_cast<const float4 *>(a + q), v = *reinterpret_cast<const float4 *>(b + q);
+        g = fmaf(u.x, v.x, g);
+        g = fmaf(u.y, v.y, g);
+        g = fmaf(u.z, v.z, g);
+        g = fmaf(u.w, v.w, g);
+    }
+    return g;
+}
+
+__device__ __forceinline__ float sum_samples(const float *a)
+{
+    float g = 0.f;
+#pragma unroll
+    for (int q = 0; q < CH; q += 4) {
+        const float4 u = *reinterpret_cast<const float4 *>(a + q);
+        g += u.x;
+        g += u.y;
+        g += u.z;
+        g += u.w;
+    }
+    return g;
+}
+
+__global__ __launch_bounds__(GT) void k_chunk_grad(const float *params, const float *x, const float *t, int32_t ns,
+                                                    float *partial)
+{
+    __shared__ ChunkLds S;
+    const int tid = threadIdx.x, c = blockIdx.x;
     const size_t s0 = (size_t)c * CH;
     const int m = (int)((size_t)ns - s0 < (size_t)CH ? (size_t)ns - s0 : (size_t)CH);
-    for (int i = threadIdx.x; i < m * H1; i += blockDim.x) {
-        sh1[i] = H1s[s0 * H1 + i];
-        sdh1[i] = DH1[s0 * H1 + i];
-    }
-    for (int i = threadIdx.x; i < m * H2; i += blockDim.x) {
-        sh2[i] = H2s[s0 * H2 + i];
-        sdh2[i] = DH2[s0 * H2 + i];
-    }
-    for (int i = threadIdx.x; i < m * NO; i += blockDim.x) sdy[i] = DY[s0 * NO + i];
-    for (int i = threadIdx.x; i < m * NI; i += blockDim.x) sx[i] = x[s0 * NI + i];
-    for (int i = threadIdx.x; i < m; i += blockDim.x) slv[i] = LV[s0 + i];
+    // samples past the last one stay zero in every array, so that they add
+    // nothing to the sums
+    for (int i = tid; i < CH * NI; i += GT) S.x[(i % NI) * LS + i / NI] = i < m * NI ? x[s0 * NI + i] : 0.f;
+    for (int i = tid; i < H1 * NI; i += GT) S.w1[(i / NI) * S1 + i % NI] = params[OW1 + i];
+    for (int i = tid; i < H2 * H1; i += GT) S.w2[(i / H1) * S2 + i % H1] = params[OW2 + i];
+    for (int i = tid; i < NO * H2; i += GT) S.w3[(i / H2) * S3 + i % H2] = params[OW3 + i];
+    if (tid < H1) S.b1[tid] = params[OB1 + tid];
+    else if (tid < H1 + H2) S.b2[tid - H1] = params[OB2 + tid - H1];
+    else if (tid < H1 + H2 + NO) S.b3[tid - H1 - H2] = params[OB3 + tid - H1 - H2];
     __syncthreads();
-    float *out = partial + (size_t)c * (NP + 1);
-    for (int p = threadIdx.x; p <= NP; p += blockDim.x) {
-        float g = 0.f;
-        if (p == NP) {
-            for (int q = 0; q < m; ++q) g += slv[q];
-        } else if (p < OB1) {
-            const int j = (p - OW1) / NI, i = (p - OW1) % NI;
-            for (int q = 0; q < m; ++q) g = fmaf(sdh1[q * H1 + j], sx[q * NI + i], g);
-        } else if (p < OW2) {
-            const int j = p - OB1;
-            for (int q = 0; q < m; ++q) g += sdh1[q * H1 + j];
-        } else if (p < OB2) {
-            const int j = (p - OW2) / H1, i = (p - OW2) % H1;
-            for (int q = 0; q < m; ++q) g = fmaf(sdh2[q * H2 + j], sh1[q * H1 + i], g);
-        } else if (p < OW3) {
-            const int j = p - OB2;
-            for (int q = 0; q < m; ++q) g += sdh2[q * H2 + j];
-        } else if (p < OB3) {
-            const int k = (p - OW3) / H2, i = (p - OW3) % H2;
-            for (int q = 0; q < m; ++q) g = fmaf(sdy[q * NO + k], sh2[q * H2 + i], g);
-        } else {
-            const int k = p - OB3;
-            for (int q = 0; q < m; ++q) g += sdy[q * NO + k];
+    const int j = tid & 31, q0 = (tid >> 5) * U; // this thread's unit and samples
+    float acc[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc[u] = S.b1[j];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) fma_samples(acc, S.w1[j * S1 + i], &S.x[i * LS + q0]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) S.h1[j * LS + q0 + u] = q0 + u < m && acc[u] > 0.f ? acc[u] : 0.f;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc[u] = S.b2[j];
+#pragma unroll 8
+    for (int i = 0; i < H1; ++i) fma_samples(acc, S.w2[j * S2 + i], &S.h1[i * LS + q0]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) S.h2[j * LS + q0 + u] = q0 + u < m && acc[u] > 0.f ? acc[u] : 0.f;
+    __syncthreads();
+    if (tid < CH * NO) {
+        const int q = tid >> 2, k = tid & 3;
+        float a = S.b3[k];
+#pragma unroll 8
+        for (int i = 0; i < H2; ++i) a = fmaf(S.w3[k * S3 + i], S.h2[i * LS + q], a);
+        const float scale = 2.0f / ((float)ns * (float)NO);
+        const float e = q < m ? a - t[(s0 + q) * NO + k] : 0.f;
+        S.e[k * LS + q] = e;
+        S.dy[k * LS + q] = q < m ? scale * e : 0.f;
+    }
+    __syncthreads();
+    if (tid < CH) {
+        float l = 0.f;
+#pragma unroll
+        for (int k = 0; k < NO; ++k) l = fmaf(S.e[k * LS + tid], S.e[k * LS + tid], l);
+        S.lv[tid] = l;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc[u] = 0.f;
+#pragma unroll
+    for (int k = 0; k < NO; ++k) fma_samples(acc, S.w3[k * S3 + j], &S.dy[k * LS + q0]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        S.d2[j * LS + q0 + u] = q0 + u < m && S.h2[j * LS + q0 + u] > 0.f ? acc[u] : 0.f;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc[u] = 0.f;
+#pragma unroll 8
+    for (int i = 0; i < H2; ++i) fma_samples(acc, S.w2[i * S2 + j], &S.d2[i * LS + q0]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        S.d1[j * LS + q0 + u] = q0 + u < m && S.h1[j * LS + q0 + u] > 0.f ? acc[u] : 0.f;
+    __syncthreads();
+    float *out = partial + (size_t)c * PS;
+    {
+        // W2[jj][ii .. ii + WU - 1]
+        constexpr int WU = H2 * H1 / GT;
+        const int jj = tid / (H1 / WU), ii = tid % (H1 / WU) * WU;
+        float g[WU];
+#pragma unroll
+        for (int u = 0; u < WU; ++u) g[u] = 0.f;
+#pragma unroll 4
+        for (int q = 0; q < CH; q += 4) {
+            const float4 d = *reinterpret_cast<const float4 *>(&S.d2[jj * LS + q]);
+#pragma unroll
+            for (int u = 0; u < WU; ++u) {
+                const float4 h = *reinterpret_cast<const float4 *>(&S.h1[(ii + u) * LS + q]);
+                g[u] = fmaf(d.x, h.x, g[u]);
+                g[u] = fmaf(d.y, h.y, g[u]);
+                g[u] = fmaf(d.z, h.z, g[u]);
+                g[u] = fmaf(d.w, h.w, g[u]);
+            }
         }
-        out[p] = g;
+#pragma unroll
+        for (int u = 0; u < WU; ++u) out[OW2 + jj * H1 + ii + u] = g[u];
+    }
+    constexpr int N1 = H1 * NI, N3 = NO * H2;
+    for (int p = tid; p < N1 + N3 + H1 + H2 + NO + 1; p += GT) {
+        int r = p;
+        if (r < N1) {
+            out[OW1 + r] = dot_samples(&S.d1[(r / NI) * LS], &S.x[(r % NI) * LS]);
+        } else if ((r -= N1) < N3) {
+            out[OW3 + r] = dot_samples(&S.dy[(r / H2) * LS], &S.h2[(r % H2) * LS]);
+        } else if ((r -= N3) < H1) {
+            out[OB1 + r] = sum_samples(&S.d1[r * LS]);
+        } else if ((r -= H1) < H2) {
+            out[OB2 + r] = sum_samples(&S.d2[r * LS]);
+        } else if ((r -= H2) < NO) {
+            out[OB3 + r] = sum_samples(&S.dy[r * LS]);
+        } else {
+            out[NP] = sum_samples(S.lv);
+        }
     }
 }
 
-// grad[p] = the chunks' partial sums in chunk order; loss = the mean of the
-// squared errors
-__global__ __launch_bounds__(256) void k_param_reduce(const float *partial, int32_t nchunks, int32_t ns,
-                                                      float *grad, float *loss)
+struct AdamArgs {
+    float *params, *m, *v; // params null: no update
+    float lr, b1, b2, eps, c1, c2;
+};
+
+// grad[p] = the chunks' partial sums in chunk order, loss = the mean of the
+// squared errors, and with A.params the Adam step on the gradient.
+//
+// A sum has one addition per chunk, in order; what must not wait in turn are
+// its loads.  A block takes 64 parameters: its 16 waves load the partial sums
+// of 256 chunks into LDS, 16 loads in flight each, and one wave adds them.
+// One thread per parameter walking the chunks took 33 us at 141 chunks, and
+// Adam its own launch 5 us; this takes 4.3.  A step at 200, 9 000 and 33 000
+// samples: 36, 72 and 172 us before, 12, 14 and 26 now, with the same bits.
+constexpr int RT = 256; // chunks per tile
+
+__global__ __launch_bounds__(1024) void k_reduce_adam(const float *partial, int32_t nchunks, int32_t ns, float *grad,
+                                                      float *loss, AdamArgs A)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p > NP) return;
+    __shared__ float tile[RT * 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane;
     float g = 0.f;
-    for (int c = 0; c < nchunks; ++c) g += partial[(size_t)c * (NP + 1) + p];
-    if (p == NP) *loss = g / ((float)ns * (float)NO);
-    else grad[p] = g;
+    for (int c0 = 0; c0 < nchunks; c0 += RT) {
+        float r[RT / 16];
+#pragma unroll
+        for (int k = 0; k < RT / 16; ++k) {
+            const int c = c0 + wave + 16 * k;
+            r[k] = c < nchunks && p <= NP ? partial[(size_t)c * PS + p] : 0.f;
+        }
+#pragma unroll
+        for (int k = 0; k < RT / 16; ++k) tile[(wave + 16 * k) * 64 + lane] = r[k];
+        __syncthreads();
+        if (wave == 0) {
+            const int cnt = nchunks - c0 < RT ? nchunks - c0 : RT;
+            int c = 0;
+            for (; c + 16 <= cnt; c += 16) {
+                float v[16];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) v[k] = tile[(c + k) * 64 + lane];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) g += v[k];
+            }
+            for (; c < cnt; ++c) g += tile[c * 64 + lane];
+        }
+        __syncthreads(); // the tile is loaded again
+    }
+    if (wave != 0 || p > NP) return;
+    if (p == NP) {
+        *loss = g / ((float)ns * (float)NO);
+        return;
+    }
+    grad[p] = g;
+    if (A.params) {
+        const float mm = A.b1 * A.m[p] + (1.f - A.b1) * g;
+        const float vv = A.b2 * A.v[p] + (1.f - A.b2) * g * g;
+        A.m[p] = mm;
+        A.v[p] = vv;
+        A.params[p] -= A.lr * (mm / A.c1) / (sqrtf(vv / A.c2) + A.eps);
+    }
 }
 
-__global__ __launch_bounds__(256) void k_adam(float *params, const float *grad, float *m, float *v,
-                                              int32_t np, float lr, float b1, float b2, float eps,
-                                              float c1, float c2)
+int loss_grad(albd_ctx *c, const float *params, const float *x, const float *t, int32_t ns, float *scratch,
+              float *grad, float *loss, const AdamArgs &A)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= np) return;
-    const float g = grad[p];
-    const float mm = b1 * m[p] + (1.f - b1) * g;
-    const float vv = b2 * v[p] + (1.f - b2) * g * g;
-    m[p] = mm;
-    v[p] = vv;
-    params[p] -= lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+    if (ns <= 0) return albd_set_error_msg(ALBBA_EINVAL, "mlp: no samples");
+    hipStream_t s = albd_stream(c);
+    const int32_t nchunks = (int32_t)(((int64_t)ns + CH - 1) / CH);
+    hipLaunchKernelGGL(k_chunk_grad, dim3(nchunks), dim3(GT), 0, s, params, x, t, ns, scratch);
+    HIPCHK(hipGetLastError());
+    hipLaunchKernelGGL(k_reduce_adam, dim3((NP + 1 + 63) / 64), dim3(1024), 0, s, scratch, nchunks, ns, grad, loss, A);
+    HIPCHK(hipGetLastError());
+    return 0;
 }
 
 } // namespace
@@ -194,28 +330,15 @@ int albd_mlp_forward(albd_ctx *c, const float *params, const float *x, int32_t n
 int albd_mlp_loss_grad(albd_ctx *c, const float *params, const float *x, const float *t, int32_t ns,
                        float *scratch, float *grad, float *loss)
 {
-    if (ns <= 0) return albd_set_error_msg(ALBBA_EINVAL, "mlp: no samples");
-    hipStream_t s = albd_stream(c);
-    hipLaunchKernelGGL(k_sample_pass, dim3((ns + 255) / 256), dim3(256), 0, s, params, x, t, ns, scratch);
-    HIPCHK(hipGetLastError());
-    const int32_t nchunks = (ns + CH - 1) / CH;
-    float *partial = scratch + (size_t)ns * ALBD_MLP_SCRATCH_PER_SAMPLE;
-    hipLaunchKernelGGL(k_param_partial, dim3(nchunks), dim3(256), 0, s, x, ns, scratch, partial);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_param_reduce, dim3((NP + 1 + 255) / 256), dim3(256), 0, s, partial, nchunks, ns, grad,
-                       loss);
-    HIPCHK(hipGetLastError());
-    return 0;
+    return loss_grad(c, params, x, t, ns, scratch, grad, loss, AdamArgs{});
 }
 
-int albd_mlp_adam(albd_ctx *c, float *params, const float *grad, float *m, float *v, int32_t np,
-                  float lr, float b1, float b2, float eps, int32_t step)
+int albd_mlp_train_step(albd_ctx *c, float *params, const float *x, const float *t, int32_t ns, float *scratch,
+                        float *grad, float *loss, float *m, float *v, float lr, float b1, float b2, float eps,
+                        int32_t step)
 {
-    const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-    hipLaunchKernelGGL(k_adam, dim3((np + 255) / 256), dim3(256), 0, albd_stream(c), params, grad, m, v,
-                       np, lr, b1, b2, eps, c1, c2);
-    HIPCHK(hipGetLastError());
-    return 0;
+    const AdamArgs A{params, m, v, lr, b1, b2, eps, 1.f - powf(b1, (float)step), 1.f - powf(b2, (float)step)};
+    return loss_grad(c, params, x, t, ns, scratch, grad, loss, A);
 }
 
 } // extern "C"

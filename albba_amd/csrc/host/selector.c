@@ -188,10 +188,9 @@ int albba_selector_train(albba_selector *s, const float *x, const float *t, int3
     if (!rc) rc = albd_h2d(d, b.t, t, sizeof(float) * (size_t)ns * ALBBA_MLP_OUT);
     if (!rc) rc = albd_fill_u32(d, b.m, 0, ALBBA_MLP_NPARAM);
     if (!rc) rc = albd_fill_u32(d, b.v, 0, ALBBA_MLP_NPARAM);
-    for (int32_t it = 1; !rc && it <= steps; ++it) {
-        rc = albd_mlp_loss_grad(d, s->dparams, b.x, b.t, ns, b.scratch, b.grad, b.loss);
-        if (!rc) rc = albd_mlp_adam(d, s->dparams, b.grad, b.m, b.v, ALBBA_MLP_NPARAM, lr, 0.9f, 0.999f, 1e-8f, it);
-    }
+    for (int32_t it = 1; !rc && it <= steps; ++it)
+        rc = albd_mlp_train_step(d, s->dparams, b.x, b.t, ns, b.scratch, b.grad, b.loss, b.m, b.v, lr, 0.9f, 0.999f,
+                                 1e-8f, it);
     /* loss of the final parameters */
     if (!rc) rc = albd_mlp_loss_grad(d, s->dparams, b.x, b.t, ns, b.scratch, b.grad, b.loss);
     if (!rc && final_loss) rc = albd_d2h(d, final_loss, b.loss, sizeof(float));
