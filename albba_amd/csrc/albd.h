@@ -155,6 +155,9 @@ ALBD_HIDDEN int albd_ctx_create(int device, albd_ctx **out);
 ALBD_HIDDEN void albd_ctx_destroy(albd_ctx *c);
 ALBD_HIDDEN int albd_ctx_device(const albd_ctx *c);
 ALBD_HIDDEN int albd_num_cus(const albd_ctx *c);
+/* freed blocks are kept for later allocations of the context, at most
+ * ALBD_KEEP_BYTES of them, and given back with it or when memory runs out */
+#define ALBD_KEEP_BYTES ((size_t)4 << 30)
 ALBD_HIDDEN int albd_malloc(albd_ctx *c, size_t bytes, void **p);
 ALBD_HIDDEN void albd_free(albd_ctx *c, void *p);
 ALBD_HIDDEN int albd_h2d(albd_ctx *c, void *dst, const void *src, size_t bytes);
@@ -170,13 +173,25 @@ ALBD_HIDDEN int albd_read_counters(albd_ctx *c, const albd_state *st); /* sync *
 #define ALBD_NEVENTS 10
 ALBD_HIDDEN int albd_event_record(albd_ctx *c, int idx);
 ALBD_HIDDEN int albd_event_elapsed(albd_ctx *c, int a, int b, float *ms); /* syncs b */
-ALBD_HIDDEN int albd_event_wait(albd_ctx *c, int idx); /* host waits for the event */
 
 /* ---- pinned host staging ---- */
+/* The context's stages: ALBD_STAGES pinned buffers of ALBD_STAGE_BYTES each,
+ * allocated at the first use and given back with the context.  albd_stages
+ * takes them for the calling thread (other threads' transfers on the context
+ * wait), albd_stages_release gives them back; _mark records that the stream's
+ * copies so far have used stage k, _wait waits for that. */
+#define ALBD_STAGES 4
+#define ALBD_STAGE_BYTES ((size_t)4 << 20)
+ALBD_HIDDEN int albd_stages(albd_ctx *c, void *stage[ALBD_STAGES]);
+ALBD_HIDDEN void albd_stages_release(albd_ctx *c);
+ALBD_HIDDEN int albd_stage_mark(albd_ctx *c, int k);
+ALBD_HIDDEN int albd_stage_wait(albd_ctx *c, int k);
 ALBD_HIDDEN int albd_pinned_alloc(albd_ctx *c, size_t bytes, void **p);
 ALBD_HIDDEN void albd_pinned_free(albd_ctx *c, void *p);
 /* host -> device copy on the context's stream, not waited for */
 ALBD_HIDDEN int albd_h2d_async(albd_ctx *c, void *dst, const void *src, size_t bytes);
+/* device -> pinned host memory on the context's stream, not waited for */
+ALBD_HIDDEN int albd_d2h_async(albd_ctx *c, void *dst, const void *src, size_t bytes);
 
 /* ---- fills (kernels, safe under graph capture) ---- */
 ALBD_HIDDEN int albd_fill_u32(albd_ctx *c, void *p, uint32_t v, size_t count);
@@ -186,19 +201,17 @@ ALBD_HIDDEN int albd_copy_u64(albd_ctx *c, void *dst, const void *src, size_t co
 
 /* ---- SELL-C-sigma build on the device ---- */
 typedef struct albd_build_input {
-    const int64_t *row_ptr; /* CSR (validated by the caller: row_ptr[0] = 0,
-                               non-decreasing, row_ptr[n] = nnz), host memory
-                               unless on_device                               */
+    const int64_t *row_ptr; /* CSR in device memory (validated by the caller:
+                               row_ptr[0] = 0, non-decreasing, row_ptr[n] =
+                               nnz)                                          */
     const int32_t *col;
     int64_t nnz;
     int32_t n, C, sigma, pad;
     int32_t symmetric;      /* 1: the push CSR is the layout's own rows      */
-    int32_t on_device;      /* 1: row_ptr/col are device pointers (no upload) */
     int32_t sort_first;     /* 1: first-column order before the window sort
                                (ALBBA_SELL_SORT_FIRST_COL)                   */
 } albd_build_input;
 typedef struct albd_build_report {
-    float upload_ms;        /* CSR host -> device                            */
     float build_ms;         /* every build step on the device                */
     int32_t rows_sorted;    /* 1: every row was already in ascending order   */
     int32_t pad_;
@@ -241,9 +254,8 @@ ALBD_HIDDEN int albd_gen_csr(albd_ctx *c, const albd_gen_spec *spec, const int32
 ALBD_HIDDEN int albd_build_haslen(albd_ctx *c, const albd_graph *g, uint64_t *haslen);
 /* row_off from row_order (g->win at most 65 536) */
 ALBD_HIDDEN int albd_build_row_off(albd_ctx *c, const albd_graph *g, uint16_t *row_off);
-/* reset every state array and seed the root (position rp, vertex id ro) */
-ALBD_HIDDEN int albd_bfs_init(albd_ctx *c, const albd_graph *g, const albd_state *st,
-                              int32_t rp, int32_t ro);
+/* reset every state array and seed the root (a vertex id) */
+ALBD_HIDDEN int albd_bfs_init(albd_ctx *c, const albd_graph *g, const albd_state *st, int32_t root);
 /* level/parent from position order (st->lp) to vertex order */
 /* if_done: queued before the host knew the BFS had ended; the kernel runs only
  * if the last select kernel found the frontier empty */

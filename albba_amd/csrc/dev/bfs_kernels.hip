@@ -390,7 +390,7 @@ __global__ __launch_bounds__(kBlock) void k_haslen(const int32_t *row_len, uint6
     if (lane_id() == 0 && w < nwords) haslen[w] = m;
 }
 
-// The state of a BFS from position rp (vertex ro) in one launch: the bitmaps
+// The state of a BFS from vertex ro in one launch: the bitmaps
 // and the slot and counter blocks zeroed, except what the root sets -- its
 // visited and frontier bits, its level/parent entry, the queue holding it
 // (when it has out-edges), and slot 0 seeded as the frontier of "level -1",
@@ -405,8 +405,9 @@ __global__ __launch_bounds__(kBlock) void k_row_off(albd_graph g, uint16_t *row_
     if (p < g.n) row_off[p] = (uint16_t)(g.row_order[p] - (int32_t)((p / g.win) * g.win));
 }
 
-__global__ __launch_bounds__(kBlock) void k_bfs_reset(albd_graph g, albd_state st, int32_t rp, int32_t ro)
+__global__ __launch_bounds__(kBlock) void k_bfs_reset(albd_graph g, albd_state st, int32_t ro)
 {
+    const int32_t rp = g.pos_of[ro];
     const int64_t deg = g.push_ptr[rp + 1] - g.push_ptr[rp];
     const int32_t rw = rp >> 6;
     const uint64_t bit = 1ull << (rp & 63);
@@ -1600,13 +1601,13 @@ int albd_build_haslen(albd_ctx *c, const albd_graph *g, uint64_t *haslen)
     return 0;
 }
 
-int albd_bfs_init(albd_ctx *c, const albd_graph *g, const albd_state *st, int32_t rp, int32_t ro)
+int albd_bfs_init(albd_ctx *c, const albd_graph *g, const albd_state *st, int32_t root)
 {
     hipStream_t s = albd_stream(c);
     int64_t blocks = ((int64_t)g->nwords + kBlock - 1) / kBlock;
     int64_t cap = (int64_t)albd_num_cus(c) * 16;
     hipLaunchKernelGGL(k_bfs_reset, dim3((unsigned)(blocks < 1 ? 1 : (blocks > cap ? cap : blocks))), dim3(kBlock),
-                       0, s, *g, *st, rp, ro);
+                       0, s, *g, *st, root);
     HIPCHK(hipGetLastError());
     return 0;
 }

@@ -583,7 +583,6 @@ int albba_batch_results(albba_batch *b, int32_t i, int32_t *level, int32_t *pare
     if (!b || i < 0 || i >= b->count) return albba_fail(ALBBA_EINVAL, "batch_results: bad instance");
     const size_t n = (size_t)b->items[i].g.n;
     int rc = 0;
-    if (level) rc = albd_d2h(b->ctx->d, level, b->items[i].level, 4 * n);
-    if (!rc && parent) rc = albd_d2h(b->ctx->d, parent, b->items[i].parent, 4 * n);
+    rc = albba_d2h_pair(b->ctx->d, level, b->items[i].level, parent, b->items[i].parent, 4 * n);
     return rc ? albba_fail(rc, "batch_results: %s", albd_error()) : ALBBA_OK;
 }

@@ -112,7 +112,7 @@ static int upload_padded_i64(albba_ctx *c, int64_t *dst, const int64_t *src, int
     if (!tmp) return ALBBA_ENOMEM;
     memcpy(tmp, src, sizeof(int64_t) * (size_t)n_src);
     for (int64_t i = n_src; i < n_dst; ++i) tmp[i] = src[n_src - 1];
-    int rc = albd_h2d(c->d, dst, tmp, sizeof(int64_t) * (size_t)n_dst);
+    int rc = albba_h2d(c->d, dst, tmp, sizeof(int64_t) * (size_t)n_dst);
     free(tmp);
     return rc;
 }
@@ -124,7 +124,7 @@ static int upload_padded_i32(albba_ctx *c, int32_t *dst, const int32_t *src, int
     if (!tmp) return ALBBA_ENOMEM;
     memcpy(tmp, src, sizeof(int32_t) * (size_t)n_src);
     for (int64_t i = n_src; i < n_dst; ++i) tmp[i] = fill;
-    int rc = albd_h2d(c->d, dst, tmp, sizeof(int32_t) * (size_t)n_dst);
+    int rc = albba_h2d(c->d, dst, tmp, sizeof(int32_t) * (size_t)n_dst);
     free(tmp);
     return rc;
 }
@@ -170,7 +170,6 @@ void albba_graph_free(albba_graph *G)
     albd_free(d, G->st.persist);
     albd_free(d, G->scratch_visited);
     albd_free(d, G->scratch_ctr);
-    free(G->pos_of);
     free(G->host_log);
     free(G->word_entries);
     free(G->list_copy);
@@ -178,8 +177,8 @@ void albba_graph_free(albba_graph *G)
 }
 
 /* The BFS state of a graph whose layout arrays are on the device (shapes
- * from G->g): allocate, build haslen, fill the keys, and keep the host copy
- * of pos_of.  Sets the error message on failure. */
+ * from G->g): allocate, build haslen and fill the keys.  Sets the error
+ * message on failure. */
 static int graph_state_alloc(albba_graph *G)
 {
     albd_graph *g = &G->g;
@@ -220,11 +219,8 @@ static int graph_state_alloc(albba_graph *G)
         (rc = albd_fill_u32(G->ctx->d, st->pmin, 0xFFFFFFFFu, (size_t)npos)) ||
         (rc = albd_sync(G->ctx->d)))
         return albba_fail(rc, "%s", albd_error());
-    G->pos_of = (int32_t *)albba_malloc(sizeof(int32_t) * (size_t)n);
     G->host_log = (int64_t *)albba_malloc(sizeof(int64_t) * 4 * ALBD_PERSIST_LEVELS);
-    if (!G->pos_of || !G->host_log) return albba_fail(ALBBA_ENOMEM, "host arrays");
-    if ((rc = albd_d2h(G->ctx->d, G->pos_of, g->pos_of, sizeof(int32_t) * (size_t)n)))
-        return albba_fail(rc, "%s", albd_error());
+    if (!G->host_log) return albba_fail(ALBBA_ENOMEM, "host arrays");
     return ALBBA_OK;
 }
 
@@ -283,15 +279,15 @@ int albba_graph_upload(albba_ctx *ctx, const albba_sellcs *s, albba_graph **out)
     if ((rc = upload_padded_i64(ctx, (int64_t *)g->slice_ptr, s->slice_pointers, s->nslices + 1, ns_alloc + 1)) ||
         (rc = upload_padded_i32(ctx, (int32_t *)g->slice_width, s->slice_widths, s->nslices, ns_alloc, 0)) ||
         (rc = upload_padded_i64(ctx, (int64_t *)g->vop_ptr, s->vop_pointers, s->nslices + 1, ns_alloc + 1)) ||
-        (rc = albd_h2d(ctx->d, (void *)g->vop_len, s->vop_lengths, (size_t)s->nvops)) ||
-        (rc = albd_h2d(ctx->d, (void *)g->colidx, s->column_indices, sizeof(int32_t) * (size_t)s->padded_nnz)) ||
+        (rc = albba_h2d(ctx->d, (void *)g->vop_len, s->vop_lengths, (size_t)s->nvops)) ||
+        (rc = albba_h2d(ctx->d, (void *)g->colidx, s->column_indices, sizeof(int32_t) * (size_t)s->padded_nnz)) ||
         (rc = upload_padded_i32(ctx, (int32_t *)g->row_order, s->row_order, s->n, npos, -1)) ||
         (rc = upload_padded_i32(ctx, (int32_t *)g->row_len, s->row_lengths, npos_raw, npos, 0)) ||
         (rc = upload_padded_i64(ctx, (int64_t *)g->push_ptr, s->push_ptr, npos_raw + 1, npos + 1)) ||
-        (rc = albd_h2d(ctx->d, (void *)g->push_col, s->push_col, sizeof(int32_t) * (size_t)s->nnz)) ||
+        (rc = albba_h2d(ctx->d, (void *)g->push_col, s->push_col, sizeof(int32_t) * (size_t)s->nnz)) ||
         (s->pull_ptr && (rc = upload_padded_i64(ctx, (int64_t *)g->pull_ptr, s->pull_ptr, npos_raw + 1, npos + 1))) ||
-        (s->pull_ptr && (rc = albd_h2d(ctx->d, (void *)g->pull_col, s->pull_col, sizeof(int32_t) * (size_t)s->nnz))) ||
-        (rc = albd_h2d(ctx->d, (void *)g->pos_of, s->pos_of, sizeof(int32_t) * (size_t)s->n))) {
+        (s->pull_ptr && (rc = albba_h2d(ctx->d, (void *)g->pull_col, s->pull_col, sizeof(int32_t) * (size_t)s->nnz))) ||
+        (rc = albba_h2d(ctx->d, (void *)g->pos_of, s->pos_of, sizeof(int32_t) * (size_t)s->n))) {
         char buf[512];
         snprintf(buf, sizeof buf, "%s", rc == ALBBA_ENOMEM ? "host staging buffer" : albd_error());
         albba_graph_free(G);
@@ -350,10 +346,19 @@ int albba_graph_build_ex(albba_ctx *ctx, const albba_csr *cg, int C, int sigma, 
     G->nnz = cg->nnz;
     G->sigma = sigma;
     G->order_flags = flags;
+    albd_ctx *d = ctx->d;
+    const double t0 = albba_now_ms();
+    int64_t *rp = NULL;
+    int32_t *col = NULL;
+    int rc = albd_malloc(d, sizeof(int64_t) * ((size_t)cg->n + 1), (void **)&rp);
+    if (!rc) rc = albd_malloc(d, sizeof(int32_t) * (size_t)(cg->nnz > 0 ? cg->nnz : 1), (void **)&col);
+    if (!rc) rc = albba_h2d(d, rp, cg->row_ptr, sizeof(int64_t) * ((size_t)cg->n + 1));
+    if (!rc) rc = albba_h2d(d, col, cg->col, sizeof(int32_t) * (size_t)cg->nnz);
+    const double t1 = albba_now_ms();
     albd_build_input in;
     memset(&in, 0, sizeof in);
-    in.row_ptr = cg->row_ptr;
-    in.col = cg->col;
+    in.row_ptr = rp;
+    in.col = col;
     in.sort_first = (flags & ALBBA_SELL_SORT_FIRST_COL) != 0;
     in.nnz = cg->nnz;
     in.n = cg->n;
@@ -363,7 +368,9 @@ int albba_graph_build_ex(albba_ctx *ctx, const albba_csr *cg, int C, int sigma, 
     in.symmetric = cg->symmetric == 1;
     albd_build_report r;
     memset(&r, 0, sizeof r);
-    int rc = albd_build_graph(ctx->d, &in, &G->g, build_alloc, G, &r);
+    if (!rc) rc = albd_build_graph(d, &in, &G->g, build_alloc, G, &r);
+    albd_free(d, rp);
+    albd_free(d, col);
     if (rc) {
         char buf[512];
         snprintf(buf, sizeof buf, "%s", albd_error());
@@ -377,33 +384,13 @@ int albba_graph_build_ex(albba_ctx *ctx, const albba_csr *cg, int C, int sigma, 
         return albba_fail(rc, "graph_build: %s", buf);
     }
     if (report) {
-        report->upload_ms = r.upload_ms;
+        report->upload_ms = (float)(t1 - t0);
         report->build_ms = r.build_ms;
         report->rows_sorted = r.rows_sorted;
         report->reserved_ = 0;
     }
     *out = G;
     return ALBBA_OK;
-}
-
-/* Stream `bytes` of f (from its current offset) into device memory at dst
- * through two pinned buffers: reading one while the other's copy runs. */
-#define LOAD_CHUNK ((size_t)64 << 20)
-static int stream_to_device(albd_ctx *d, FILE *f, void *dst, size_t bytes, void *buf[2])
-{
-    size_t done = 0;
-    int k = 0, rc;
-    while (done < bytes) {
-        const size_t len = bytes - done < LOAD_CHUNK ? bytes - done : LOAD_CHUNK;
-        /* the copy that last used this buffer must have finished */
-        if ((rc = albd_event_wait(d, 4 + k))) return rc;
-        if (fread(buf[k], 1, len, f) != len) return albba_fail(ALBBA_EIO, "graph_load: short read");
-        if ((rc = albd_h2d_async(d, (char *)dst + done, buf[k], len)) || (rc = albd_event_record(d, 4 + k)))
-            return rc;
-        done += len;
-        k ^= 1;
-    }
-    return 0;
 }
 
 int albba_graph_load(albba_ctx *ctx, const char *path, int C, int sigma, int pad, albba_graph **out,
@@ -436,20 +423,12 @@ int albba_graph_load(albba_ctx *ctx, const char *path, int C, int sigma, int pad
     }
     albd_ctx *d = ctx->d;
     int32_t *rp32 = NULL, *col = NULL;
-    void *buf[2] = {NULL, NULL};
     int rc = albd_malloc(d, sizeof(int32_t) * ((size_t)n + 1), (void **)&rp32);
     if (!rc) rc = albd_malloc(d, sizeof(int32_t) * (size_t)(nnz > 0 ? nnz : 1), (void **)&col);
-    if (!rc) rc = albd_pinned_alloc(d, LOAD_CHUNK, &buf[0]);
-    if (!rc) rc = albd_pinned_alloc(d, LOAD_CHUNK, &buf[1]);
-    /* a fresh pair of events: waiting on one never recorded returns at once */
-    if (!rc) rc = albd_event_record(d, 4);
-    if (!rc) rc = albd_event_record(d, 5);
-    if (!rc) rc = stream_to_device(d, f, rp32, sizeof(int32_t) * ((size_t)n + 1), buf);
-    if (!rc) rc = stream_to_device(d, f, col, sizeof(int32_t) * (size_t)nnz, buf);
-    if (!rc) rc = albd_sync(d);
+    const size_t rp_bytes = sizeof(int32_t) * ((size_t)n + 1);
+    if (!rc) rc = albba_file_to_device(d, f, (int64_t)sizeof hdr, rp32, rp_bytes);
+    if (!rc) rc = albba_file_to_device(d, f, (int64_t)(sizeof hdr + rp_bytes), col, sizeof(int32_t) * (size_t)nnz);
     fclose(f);
-    albd_pinned_free(d, buf[0]);
-    albd_pinned_free(d, buf[1]);
     const double t1 = albba_now_ms();
     int64_t *wp = NULL;
     int32_t *wc = NULL;
@@ -460,7 +439,7 @@ int albba_graph_load(albba_ctx *ctx, const char *path, int C, int sigma, int pad
     if (rc || bad) {
         char buf2[512];
         snprintf(buf2, sizeof buf2, "%s", bad ? "row pointers or column indices out of range" :
-                 (rc == ALBBA_EIO ? albba_last_error() : albd_error()));
+                 (rc == ALBBA_EIO ? "short read" : albd_error()));
         albd_free(d, wp);
         albd_free(d, wc);
         return albba_fail(bad ? ALBBA_EINVAL : rc, "graph_load: %s", buf2);
@@ -482,7 +461,6 @@ int albba_graph_load(albba_ctx *ctx, const char *path, int C, int sigma, int pad
     in.sigma = sigma;
     in.pad = pad;
     in.symmetric = 0; /* the .cbd path leaves isSymmetric unset: W is built as directed */
-    in.on_device = 1;
     albd_build_report r;
     memset(&r, 0, sizeof r);
     rc = albd_build_graph(d, &in, &G->g, build_alloc, G, &r);
@@ -586,8 +564,8 @@ int albba_graph_generate(albba_ctx *ctx, const albba_gen_params *p, int C, int s
             free(hrp); free(hcol); albd_free(d, rp); albd_free(d, col);
             return albba_fail(ALBBA_ENOMEM, "graph_generate: host copy");
         }
-        if ((rc = albd_d2h(d, hrp, rp, sizeof(int64_t) * ((size_t)g.n + 1))) ||
-            (rc = albd_d2h(d, hcol, col, sizeof(int32_t) * (size_t)m))) {
+        if ((rc = albba_d2h(d, hrp, rp, sizeof(int64_t) * ((size_t)g.n + 1))) ||
+            (rc = albba_d2h(d, hcol, col, sizeof(int32_t) * (size_t)m))) {
             char buf[512];
             snprintf(buf, sizeof buf, "%s", albd_error());
             free(hrp); free(hcol); albd_free(d, rp); albd_free(d, col);
@@ -619,7 +597,6 @@ int albba_graph_generate(albba_ctx *ctx, const albba_gen_params *p, int C, int s
     in.sigma = sigma;
     in.pad = pad;
     in.symmetric = 1;
-    in.on_device = 1;
     albd_build_report r;
     memset(&r, 0, sizeof r);
     rc = albd_build_graph(d, &in, &G->g, build_alloc, G, &r);
@@ -682,18 +659,18 @@ int albba_graph_layout(albba_ctx *ctx, const albba_graph *G, albba_sellcs **out)
     }
     albd_ctx *d = ctx->d;
     int rc = 0;
-    if ((rc = albd_d2h(d, s->row_order, g->row_order, sizeof(int32_t) * (size_t)g->n)) ||
-        (rc = albd_d2h(d, s->pos_of, g->pos_of, sizeof(int32_t) * (size_t)g->n)) ||
-        (rc = albd_d2h(d, s->slice_widths, g->slice_width, sizeof(int32_t) * (size_t)ns)) ||
-        (rc = albd_d2h(d, s->slice_pointers, g->slice_ptr, sizeof(int64_t) * (size_t)(ns + 1))) ||
-        (rc = albd_d2h(d, s->vop_pointers, g->vop_ptr, sizeof(int64_t) * (size_t)(ns + 1))) ||
-        (rc = albd_d2h(d, s->vop_lengths, g->vop_len, (size_t)g->nvops)) ||
-        (rc = albd_d2h(d, s->column_indices, g->colidx, sizeof(int32_t) * (size_t)g->padded_nnz)) ||
-        (rc = albd_d2h(d, s->row_lengths, g->row_len, sizeof(int32_t) * (size_t)npos_raw)) ||
-        (rc = albd_d2h(d, s->push_ptr, g->push_ptr, sizeof(int64_t) * (size_t)(npos_raw + 1))) ||
-        (rc = albd_d2h(d, s->push_col, g->push_col, sizeof(int32_t) * (size_t)g->nnz)) ||
-        (directed && (rc = albd_d2h(d, s->pull_ptr, g->pull_ptr, sizeof(int64_t) * (size_t)(npos_raw + 1)))) ||
-        (directed && (rc = albd_d2h(d, s->pull_col, g->pull_col, sizeof(int32_t) * (size_t)g->nnz)))) {
+    if ((rc = albba_d2h(d, s->row_order, g->row_order, sizeof(int32_t) * (size_t)g->n)) ||
+        (rc = albba_d2h(d, s->pos_of, g->pos_of, sizeof(int32_t) * (size_t)g->n)) ||
+        (rc = albba_d2h(d, s->slice_widths, g->slice_width, sizeof(int32_t) * (size_t)ns)) ||
+        (rc = albba_d2h(d, s->slice_pointers, g->slice_ptr, sizeof(int64_t) * (size_t)(ns + 1))) ||
+        (rc = albba_d2h(d, s->vop_pointers, g->vop_ptr, sizeof(int64_t) * (size_t)(ns + 1))) ||
+        (rc = albba_d2h(d, s->vop_lengths, g->vop_len, (size_t)g->nvops)) ||
+        (rc = albba_d2h(d, s->column_indices, g->colidx, sizeof(int32_t) * (size_t)g->padded_nnz)) ||
+        (rc = albba_d2h(d, s->row_lengths, g->row_len, sizeof(int32_t) * (size_t)npos_raw)) ||
+        (rc = albba_d2h(d, s->push_ptr, g->push_ptr, sizeof(int64_t) * (size_t)(npos_raw + 1))) ||
+        (rc = albba_d2h(d, s->push_col, g->push_col, sizeof(int32_t) * (size_t)g->nnz)) ||
+        (directed && (rc = albba_d2h(d, s->pull_ptr, g->pull_ptr, sizeof(int64_t) * (size_t)(npos_raw + 1)))) ||
+        (directed && (rc = albba_d2h(d, s->pull_col, g->pull_col, sizeof(int32_t) * (size_t)g->nnz)))) {
         char buf[512];
         snprintf(buf, sizeof buf, "%s", albd_error());
         albba_sellcs_free(s);
@@ -1054,7 +1031,6 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
         return albba_fail(ALBBA_EINVAL, "bfs: learned policy needs a selector");
     albd_ctx *d = ctx->d;
     const int reps = opts.timing_reps > 0 ? opts.timing_reps : 1;
-    const int32_t rp = G->pos_of[root];
     int valid_mask = 0;
     for (int c = 0; c < ALBBA_NUM_CHOICES; ++c) valid_mask |= choice_ok(G, c) << c;
     albd_select_args sel = {policy == ALBBA_SWITCH_LEARNED ? albba_selector_dparams(opts.selector) : NULL,
@@ -1101,7 +1077,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
     int vo_queued = 0;
     int64_t frontier_prev = 0;
     /* init, then the select kernel turns the root into level 0's frontier */
-    if ((rc = albd_event_record(d, ev.start)) || (rc = albd_bfs_init(d, &G->g, &G->st, rp, root)))
+    if ((rc = albd_event_record(d, ev.start)) || (rc = albd_bfs_init(d, &G->g, &G->st, root)))
         return albba_fail(rc, "bfs: %s", albd_error());
     if (spec)
         rc = select_prep(G, &ls, &sel, &seq) ||
@@ -1350,9 +1326,7 @@ int albba_bfs_results(albba_ctx *ctx, albba_graph *G, int32_t *level, int32_t *p
 {
     if (!ctx || !G) return albba_fail(ALBBA_EINVAL, "bfs_results: null");
     int rc = 0;
-    if (level && (rc = albd_d2h(ctx->d, level, G->st.level, sizeof(int32_t) * (size_t)G->n)))
-        return albba_fail(rc, "bfs_results: %s", albd_error());
-    if (parent && (rc = albd_d2h(ctx->d, parent, G->st.parent, sizeof(int32_t) * (size_t)G->n)))
+    if ((rc = albba_d2h_pair(ctx->d, level, G->st.level, parent, G->st.parent, sizeof(int32_t) * (size_t)G->n)))
         return albba_fail(rc, "bfs_results: %s", albd_error());
     return ALBBA_OK;
 }

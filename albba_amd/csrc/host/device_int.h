@@ -19,7 +19,6 @@ struct albba_graph {
     int32_t sigma;       /* the layout's sigma as requested */
     int32_t order_flags; /* ALBBA_SELL_* row-order flags of the layout */
     int64_t nnz;
-    int32_t *pos_of;     /* host: vertex id -> position */
     int64_t device_bytes;
     void *scratch_visited; /* BEST-policy snapshots */
     void *scratch_ctr;
@@ -29,5 +28,16 @@ struct albba_graph {
     int32_t *list_copy;    /* host: a pull's word list, for that accounting */
     int needs_reset;       /* a BFS failed midway: pmin/pkey may be dirty */
 };
+
+/* host/transfer.c: as albd_d2h / albd_h2d, through the context's pinned
+ * stages and several threads where the copy is large */
+ALBBA_HIDDEN int albba_d2h(albd_ctx *d, void *dst, const void *src, size_t bytes);
+ALBBA_HIDDEN int albba_h2d(albd_ctx *d, void *dst, const void *src, size_t bytes);
+/* two device arrays of `bytes` each (a null destination: not that one) */
+ALBBA_HIDDEN int albba_d2h_pair(albd_ctx *d, void *dst0, const void *src0, void *dst1, const void *src1,
+                                size_t bytes);
+/* `bytes` of f at offset `off` (where f stands, if it cannot seek) into device
+ * memory; ALBBA_EIO when the file is shorter */
+ALBBA_HIDDEN int albba_file_to_device(albd_ctx *d, FILE *f, int64_t off, void *dst, size_t bytes);
 
 #endif
