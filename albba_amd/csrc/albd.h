@@ -349,18 +349,26 @@ ALBD_HIDDEN int albd_mail_wait(albd_ctx *c, const albd_state *st, unsigned int s
 ALBD_HIDDEN void albd_mail_stats(const albd_ctx *c, unsigned long *hits, unsigned long *misses);
 
 /* ---- batched BFS (batch.hip) ---- */
+/* most workgroups of a team */
+#define ALBD_BATCH_TEAM_MAX 64
+/* entries of an instance's found list: every position, and two unfilled
+ * reservations (2 048 entries) of every workgroup of the largest team */
+#define ALBD_BATCH_FOUND(npos) ((size_t)(npos) + ALBD_BATCH_TEAM_MAX * 2 * 2048)
+/* words of an instance's barrier slots: two sets of three counts */
+#define ALBD_BATCH_SLOTS (2 * 3 * ALBD_BATCH_TEAM_MAX)
 /* One instance: a device graph, its own scratch, a root.  The control block
- * ctl (32 words) must be zero before the launch: [0] team barrier,
- * [1] found-list length, [2] error flag, [4..19] ring of four level counters
- * (pulled vertices, out-edges, -, nonzero words), [24..31] results. */
+ * ctl (32 words) and the slots must be zero before the launch: [1], [3] found-
+ * list reservations, [2] error flag, [4..7] shared-queue entries and [8..11]
+ * listed vertices of four push levels, [24..31] results. */
 typedef struct albd_batch_item {
     albd_graph g;
     uint64_t *visited;           /* [nwords] */
     uint64_t *bm[3];             /* [nwords] frontier bitmaps, rotating */
-    int32_t *found;              /* [npos] frontier queues, level after level */
+    int32_t *found;              /* [ALBD_BATCH_FOUND(npos)] vertices found by pushes */
     unsigned long long *key;     /* [npos] (level, parent id), all ones at rest */
-    int32_t *level, *parent;     /* [n] results in vertex order */
+    int32_t *level, *parent;     /* [n] results in vertex order; push queues before */
     unsigned long long *ctl;     /* [32] see above */
+    unsigned long long *slot;    /* [ALBD_BATCH_SLOTS] the team barrier's arrivals */
     int32_t root;                /* vertex id */
     int32_t mapping;             /* pull: ALBD_MAP_LANE_ROW or ALBD_MAP_WAVE_ROW */
 } albd_batch_item;

@@ -11,40 +11,43 @@
 // its row's first frontier neighbour u does the same.  The key keeps the
 // smallest (level, parent) pair, so it holds the BFS level and the min-id
 // parent no matter in which order the team's waves run, and the old value
-// names the one discoverer.  The visited bitmap is only a filter; the
-// frontier bitmaps are exact (a pull relies on them for the min-id parent).
+// names the one discoverer.
 //
-// Frontier bitmaps B_L (vertices of level L) rotate over three buffers: at
-// level L the team reads B_L, sets B_{L+1} and clears B_{L-1}, which becomes
-// B_{L+2}.  A push level lists its discoveries (found list), which is the
-// next level's queue and lets the bitmap be cleared two levels later without
-// a full pass; a pulled bitmap is cleared by a full pass.  Discoverers set
-// the visited bits at once: a push needs no visited filter (the key decides),
-// a pull reads visited as the exact set of vertices found so far.
+// Push levels run as in the small-frontier kernel (push_lists.h): lists of
+// edges in LDS, a shared queue (in the result arrays, which are written at the
+// end only), one barrier that carries the counts, and no bitmaps.  What bounds
+// the batch is its grids' thousands of levels: bitmaps set by the discoverers,
+// a queue in memory with its reservations and a counting barrier cost the
+// largest grid of a 24-instance mix 16.9 us a level where these take 5.2 (the
+// launch 45 -> 14 ms; 96 instances 66 -> 25, 256 instances 111 -> 62 ms).
+//
+// The kernel has phases with nothing in common, and values that the compiler
+// hoisted out of one were spilled in the others: the thread's index is taken
+// anew in each (here_tid), the push levels' registers live in a loop of their
+// own, the descriptor comes through scalar loads and the selector's logarithm
+// is a call.  79 spilled registers -> 33 took the push levels from 5.9 to 4.5
+// us and one workgroup's RMAT s20 search from 63 to 50 ms.
+//
+// A pull needs the frontier bitmap and the visited one: the found list since
+// the last pull gives both (materialize), once per turn from push to pull.
+// Bitmaps rotate over three buffers: a pull reads one, sets the next and
+// clears the one before; all are clean while levels push.
 #include "dev_common.h"
+#include "push_lists.h"
 #include "select_dev.h"
 #include "../../../include/albba.h"
 
 namespace {
 
-constexpr int kBB = 512;              // threads per workgroup
-constexpr int kBWaves = kBB / 64;
-constexpr int kBChunk = kBB;          // queue entries staged per pass
-constexpr int kBPer = 4;              // edges per thread per window
-constexpr int kBWin = kBPer * kBB;    // edges per window
+constexpr int kBB = kListBlock; // threads per workgroup
+constexpr int kBWaves = kListWaves;
 
 struct BLds {
-    int64_t pre[kBChunk];
-    int64_t start[kBChunk];
-    uint32_t ou[kBChunk];
-    int64_t scan[kBWaves];
-    int32_t found[kBWin];
-    unsigned int nf;
-    unsigned long long bf;
-    unsigned long long red[4][kBWaves];
+    PushLds l;
+    unsigned long long red[3][kBWaves];
     unsigned int s_cnt[kBWaves];
     unsigned long long s_base;
-    int ok, choice;
+    int choice;
     float params[ALBBA_MLP_NPARAM];
     float xs[ALBBA_MLP_IN], h1[ALBBA_MLP_H1], h2[ALBBA_MLP_H2], ys[ALBBA_MLP_OUT];
 };
@@ -54,135 +57,144 @@ __device__ __forceinline__ unsigned int *err_flag(const albd_batch_item &it)
     return reinterpret_cast<unsigned int *>(&it.ctl[2]);
 }
 
-__device__ __forceinline__ long long *ring(const albd_batch_item &it, int L)
+// sums of one value per thread over the workgroup, to thread 0
+__device__ __forceinline__ unsigned long long block_sum(BLds &S, int row, unsigned long long x)
 {
-    return reinterpret_cast<long long *>(it.ctl) + 4 + 4 * (L & 3);
-}
-
-// per-wave counts -> one atomic per workgroup into the level's ring slot
-__device__ void add_counts(BLds &S, long long *slot, unsigned long long f, unsigned long long e,
-                           unsigned long long w)
-{
-    const int lane = lane_id(), wid = threadIdx.x >> 6;
-    f = wave_sum(f);
-    e = wave_sum(e);
-    w = wave_sum(w);
-    if (lane == 0) {
-        S.red[0][wid] = f;
-        S.red[1][wid] = e;
-        S.red[3][wid] = w;
-    }
+    x = wave_sum(x);
+    if (lane_id() == 0) S.red[row][threadIdx.x >> 6] = x;
     __syncthreads();
-    if (threadIdx.x < 4 && threadIdx.x != 2) {
-        unsigned long long t = 0;
-        for (int i = 0; i < kBWaves; ++i) t += S.red[threadIdx.x][i];
-        if (t) atomicAdd(reinterpret_cast<unsigned long long *>(&slot[threadIdx.x]), t);
-    }
-    __syncthreads();
-}
-
-// the LDS list of a push window -> the instance's found list at
-// found[base + ...] (one reservation per window on the level's counter)
-__device__ void flush_found(BLds &S, const albd_batch_item &it, unsigned long long *counter, int64_t base)
-{
-    __syncthreads();
-    const unsigned int nf = S.nf;
-    if (threadIdx.x == 0) S.bf = nf ? atomicAdd(counter, (unsigned long long)nf) : 0;
-    __syncthreads();
-    if (threadIdx.x == 0) S.nf = 0;
-    const unsigned long long bf = S.bf;
-    for (unsigned int i = threadIdx.x; i < nf; i += kBB) st_coherent(&it.found[base + bf + i], S.found[i]);
-    __syncthreads();
+    unsigned long long t = 0;
+    if (threadIdx.x == 0)
+        for (int i = 0; i < kBWaves; ++i) t += S.red[row][i];
+    return t;
 }
 
 // One BFS of one instance by a team of T workgroups (this one is `rank`).
-// The found list holds, level after level, the vertices each push found and
-// the rebuilt frontier of a push that follows a pull: the frontier queue of
-// level L is the range [fs_cur, fe_cur).  Returns false when a team barrier
-// gave up.
+// Returns false when a team barrier gave up.
 __device__ bool run_instance(BLds &S, const albd_batch_item &it, int rank, int T, bool learned,
                              uint32_t spin_limit)
 {
     const albd_graph &g = it.g;
-    const int tid = threadIdx.x, lane = lane_id(), wid = tid >> 6;
-    const int64_t gtid = (int64_t)rank * kBB + tid, gthreads = (int64_t)T * kBB;
+    const int tid = threadIdx.x;
+    const int64_t gthreads = (int64_t)T * kBB;
+    // the thread's number in the team, worked out where a phase begins
+    auto team_tid = [&]() -> int64_t { return (int64_t)rank * kBB + here_tid(); };
     const int64_t nwords = g.nwords;
-    unsigned long long *bar = &it.ctl[0];
-    unsigned int *err = err_flag(it);
+    PushLds &L = S.l;
+    const TeamSlots B{it.slot, err_flag(it), ALBD_BATCH_TEAM_MAX, T, rank, spin_limit};
+    unsigned int tag = 0;
     const bool leader = rank == 0 && tid == 0;
     if (leader) st_coherent(reinterpret_cast<long long *>(&it.ctl[ALBD_RES_T0]), (long long)wall_clock64());
-    for (int64_t i = gtid; i < nwords; i += gthreads) {
+    for (int64_t i = team_tid(); i < nwords; i += gthreads) {
         st_coherent(&it.visited[i], (uint64_t)0);
         st_coherent(&it.bm[0][i], (uint64_t)0);
         st_coherent(&it.bm[1][i], (uint64_t)0);
         st_coherent(&it.bm[2][i], (uint64_t)0);
     }
-    if (tid == 0) S.nf = 0;
-    if (!team_sync(bar, err, T, spin_limit, &S.ok)) return false;
+    list_reset(L);
+    // the found list's reservations: counters 0 and 1 in turn, from one
+    // materialize to the next
+    unsigned long long *next_reserve = &it.ctl[3];
+    PushMem M{nullptr, it.key, it.found, &it.ctl[1]};
+    const int64_t found_cap = (int64_t)ALBD_BATCH_FOUND(g.npos);
+    __syncthreads();
+    if (tid == 0) reserve_found(L, M, 0);
+    int32_t *qa = it.level, *qb = it.parent; // the shared queues
     const int32_t rp = g.pos_of[it.root];
     const int64_t rdeg = g.push_ptr[rp + 1] - g.push_ptr[rp];
     if (leader) {
-        // the root: level 0, its own parent, frontier B_0, found entry 0
-        const uint64_t bit = 1ull << (rp & 63);
+        // the root: level 0, its own parent, the queue and the found list
         st_coherent(&it.key[rp], (unsigned long long)(uint32_t)it.root);
-        atomicOr(reinterpret_cast<unsigned long long *>(&it.visited[rp >> 6]), bit);
-        atomicOr(reinterpret_cast<unsigned long long *>(&it.bm[0][rp >> 6]), bit);
-        st_coherent(&it.found[0], rp);
+        st_coherent(&qa[0], rp);
+        st_coherent(&it.found[L.chunk[0]], rp);
     }
-    if (!team_sync(bar, err, T, spin_limit, &S.ok)) return false;
+    int64_t F = rank == 0 ? 1 : 0; // in this workgroup's reservations
+    if (!team_barrier(L, B, ++tag)) return false;
 
     // team-uniform loop state
-    unsigned long long F = 1, mf = (unsigned long long)rdeg, nzw = 1, F_prev = 0;
+    unsigned long long Fr = 1, mf = (unsigned long long)rdeg, nzw = 1, F_prev = 0;
     unsigned long long reached = 1, redges = (unsigned long long)rdeg;
     int prev_choice = ALBBA_CHOICE_PUSH;
-    int64_t fs_cur = 0, fe_cur = 1, fs_prev = 0, fe_prev = 0; // found ranges of B_L, B_{L-1}
-    bool have_queue = true;                                   // B_L's range holds its vertices
-    bool cur_by_pull = false, prev_by_pull = false;           // how B_L, B_{L-1} were made
+    int64_t ns = 1;         // the shared queue's length
+    int cap = kListEdges;   // edges the workgroup's list takes
+    bool lists = true;      // the frontier is in the lists and the queue
+    bool bitmap = false;    // it is in bcur, and visited is up to date
+    bool old_dirty = false; // bold holds an older frontier
+    // the bitmaps (pointers that rotate: an index into the descriptor's array
+    // would put the descriptor into scratch memory)
+    uint64_t *bcur = it.bm[0], *bnext = it.bm[1], *bold = it.bm[2];
+    int listed = 0;         // edges of the workgroup's list
     long long pushes = 0, pulls = 0;
     const long long thr = (long long)(int)((double)g.n * 0.04);
-    int L = 0;
-    for (; F > 0; ++L) {
-        uint64_t *bcur = it.bm[L % 3], *bnext = it.bm[(L + 1) % 3], *bprev = it.bm[(L + 2) % 3];
-        long long *slot = ring(it, L);
-        // direction of this level (the same in every workgroup of the team).
-        // A batched pull visits every word of the instance with the team's few
-        // workgroups, so the learned selector is consulted only when the
-        // frontier is large by the heuristic's count or its out-edges reach
-        // 1/16 of the unexplored edges; otherwise the level pushes.
-        int choice = (long long)F > thr ? ALBBA_CHOICE_PULL_SB : ALBBA_CHOICE_PUSH;
-        const unsigned long long unexplored =
-            (unsigned long long)g.nnz > redges ? (unsigned long long)g.nnz - redges : 0ull;
-        if (learned && ((long long)F > thr || 16 * mf >= unexplored)) {
+    // Whether a level is anything but a plain push.  The heuristic pulls when
+    // the frontier is large by its count.  A batched pull visits every word of
+    // the instance with the team's few workgroups, so the learned selector is
+    // consulted only then, or when the frontier's out-edges reach 1/16 of the
+    // unexplored edges.
+    auto decide = [&](unsigned long long f, unsigned long long edges, unsigned long long seen) -> bool {
+        if ((long long)f > thr) return true;
+        const unsigned long long unexplored = (unsigned long long)g.nnz > seen ? (unsigned long long)g.nnz - seen : 0ull;
+        return learned && 16 * edges >= unexplored;
+    };
+    int Lv = 0;
+    while (Fr > 0) {
+        // direction of this level (the same in every workgroup of the team)
+        int choice = (long long)Fr > thr ? ALBBA_CHOICE_PULL_SB : ALBBA_CHOICE_PUSH;
+        const bool consult = learned && decide(Fr, mf, redges);
+        if ((consult || choice != ALBBA_CHOICE_PUSH) && !bitmap) {
+            // materialize: the vertices found since the last time into
+            // visited, those of this level into the frontier bitmap
+            __syncthreads(); // the reservation made since the last level
+            end_found(L, M, F, found_cap);
+            if (!team_barrier(L, B, ++tag)) return false;
+            int64_t total = (int64_t)ld_coherent(M.reserve);
+            if (total > found_cap) total = found_cap;
+            unsigned long long my_w = 0;
+            for (int64_t i = team_tid(); i < total; i += gthreads) {
+                const int32_t v = ld_coherent(&it.found[i]);
+                if (v < 0) continue;
+                const uint64_t bit = 1ull << (v & 63);
+                atomicOr(reinterpret_cast<unsigned long long *>(&it.visited[v >> 6]), bit);
+                if ((uint32_t)(ld_coherent(&it.key[v]) >> 32) == (uint32_t)Lv)
+                    my_w += atomicOr(reinterpret_cast<unsigned long long *>(&bcur[v >> 6]), bit) == 0 ? 1 : 0;
+            }
+            const unsigned long long w = block_sum(S, 0, my_w);
+            if (!team_barrier(L, B, ++tag, w)) return false;
+            nzw = uniform64(L.tot[0]);
+            bitmap = true;
+            // a fresh found list, by the other counter
+            if (leader) st_coherent(M.reserve, 0ull);
+            unsigned long long *t = M.reserve;
+            M.reserve = next_reserve;
+            next_reserve = t;
+            F = 0;
+            __syncthreads();
+            if (tid == 0) {
+                L.reserved = 0;
+                reserve_found(L, M, 0);
+            }
+            __syncthreads();
+        }
+        if (consult) {
             if (tid < 64)
-                level_features(S.xs, g.n, g.nnz, nwords, F, mf, nzw, reached, redges, L, prev_choice,
-                               F_prev);
+                level_features<true>(S.xs, g.n, g.nnz, nwords, Fr, mf, nzw, reached, redges, Lv,
+                                     prev_choice, F_prev);
             __syncthreads();
             const int c = mlp_argmin(S.params, S.xs, S.h1, S.h2, S.ys, 0xF, &S.choice);
             if (c >= 0) choice = c;
         }
-        const bool push = choice == ALBBA_CHOICE_PUSH;
-        // the slot two levels ahead is free: its last readers passed a barrier
-        if (leader)
-            for (int f = 0; f < 4; ++f) st_coherent(ring(it, L + 2) + f, 0ll);
-        // B_{L-1} goes back to zero (it becomes B_{L+2})
-        if (L >= 1) {
-            if (prev_by_pull) {
-                for (int64_t i = gtid; i < nwords; i += gthreads) st_coherent(&bprev[i], (uint64_t)0);
-            } else {
-                for (int64_t i = fs_prev + gtid; i < fe_prev; i += gthreads)
-                    st_coherent(&bprev[ld_coherent(&it.found[i]) >> 6], (uint64_t)0);
-            }
-        }
-        const unsigned long long lkey = (unsigned long long)(uint32_t)(L + 1) << 32;
-        unsigned long long my_f = 0, my_e = 0, my_w = 0;
-        if (push) {
-            ++pushes;
-            if (!have_queue) {
-                // B_L came from a pull: list its vertices from the bitmap,
-                // one reservation per block step
+        if (choice == ALBBA_CHOICE_PUSH) {
+            if (!lists) {
+                // the frontier came from a pull: list its vertices from the
+                // bitmap, one reservation per block step, and leave every
+                // bitmap clean
+                const int tid = here_tid(), lane = tid & 63, wid = tid >> 6;
+                unsigned long long mine = 0; // thread 0's
                 for (int64_t wb = (int64_t)rank * kBB; wb < nwords; wb += gthreads) {
                     const int64_t w = wb + tid;
                     const uint64_t word = w < nwords ? ld_coherent(&bcur[w]) : 0ull;
+                    if (word) st_coherent(&bcur[w], (uint64_t)0);
+                    if (old_dirty && w < nwords) st_coherent(&bold[w], (uint64_t)0);
                     unsigned long long wtot;
                     const unsigned long long ex =
                         wave_exclusive_scan<unsigned long long>((unsigned long long)__popcll(word), &wtot);
@@ -191,105 +203,103 @@ __device__ bool run_instance(BLds &S, const albd_batch_item &it, int rank, int T
                     if (tid == 0) {
                         unsigned long long tot = 0;
                         for (int i = 0; i < kBWaves; ++i) tot += S.s_cnt[i];
-                        S.s_base = tot ? atomicAdd(reinterpret_cast<unsigned long long *>(&slot[2]), tot) : 0ull;
+                        S.s_base = tot ? atomicAdd(&it.ctl[8 + (pushes & 3)], tot) : 0ull;
+                        mine += tot;
                     }
                     __syncthreads();
-                    unsigned long long o = (unsigned long long)fe_cur + S.s_base + ex;
+                    unsigned long long o = S.s_base + ex;
                     for (int i = 0; i < wid; ++i) o += S.s_cnt[i];
                     __syncthreads();
                     uint64_t kb = word;
                     while (kb) {
                         const int b = __ffsll((unsigned long long)kb) - 1;
                         kb &= kb - 1;
-                        st_coherent(&it.found[o++], (int32_t)(w * 64 + b));
+                        st_coherent(&qa[o++], (int32_t)(w * 64 + b));
                     }
                 }
-                if (!team_sync(bar, err, T, spin_limit, &S.ok)) return false;
-                fs_cur = fe_cur;
-                fe_cur += (int64_t)ld_coherent(&slot[2]);
+                if (!team_barrier(L, B, ++tag, mine)) return false;
+                ns = (int64_t)uniform64(L.tot[0]);
+                cap = kListEdges;
+                listed = 0;
+                lists = true;
+                old_dirty = false;
+            } else if (bitmap) {
+                // materialized for the selector, which pushes all the same
+                for (int64_t i = team_tid(); i < nwords; i += gthreads) st_coherent(&bcur[i], (uint64_t)0);
             }
-            // expansion: workgroup `rank` takes queue entries [q0, q1)
-            const int64_t qlen = fe_cur - fs_cur;
-            const int64_t per = (qlen + T - 1) / T;
-            const int64_t q0 = fs_cur + (int64_t)rank * per;
-            const int64_t q1 = q0 + per < fe_cur ? q0 + per : fe_cur;
-            for (int64_t base = q0; base < q1; base += kBChunk) { // uniform in the workgroup
-                const int cnt_e = (int)(q1 - base < kBChunk ? q1 - base : kBChunk);
-                int64_t a0 = 0, e0 = 0;
-                uint32_t o0 = 0;
-                if (tid < cnt_e) {
-                    const int32_t u = ld_coherent(&it.found[base + tid]);
-                    a0 = g.push_ptr[u];
-                    e0 = g.push_ptr[u + 1];
-                    o0 = (uint32_t)g.row_order[u];
+            bitmap = false;
+            // push levels, as long as nothing else is to be decided: the
+            // edges' registers live in this loop only
+            PushEdge e[kListPer];
+            load_list(L, g, M, listed, e);
+            do {
+                const int wid = here_tid() >> 6, lane = here_tid() & 63;
+                // the waves that poll: the last ones, which hold the fewest edges
+                const int poll = wid - (kBWaves - 3);
+                const int par = (int)(pushes & 1);
+                // this push level's counter of entries put on the shared
+                // queue; that of two push levels ahead, and the one of listing
+                // a bitmap, are free (their last users passed a barrier) and
+                // start from zero
+                unsigned long long *spill_ctr = &it.ctl[4 + (pushes & 3)];
+                if (leader) {
+                    st_coherent(&it.ctl[4 + ((pushes + 2) & 3)], 0ull);
+                    st_coherent(&it.ctl[8 + ((pushes + 2) & 3)], 0ull);
                 }
-                int64_t Te;
-                const int64_t ex = block_scan_excl<kBB>(e0 - a0, &Te, S.scan);
-                S.pre[tid] = ex;
-                S.start[tid] = a0;
-                S.ou[tid] = o0;
+                ++pushes;
+                if (tid == 0) L.cnt[par ^ 1] = L.edges[par ^ 1] = L.spill[par ^ 1] = 0;
+                bool won[kListPer], spilled = false;
+                uint32_t f[kListPer];
+                const uint32_t lvl = (uint32_t)(Lv + 1);
+                relax_edges<kListPer, false>(L, g, M, e, lvl, par, cap, spill_ctr, qb, won, f, spilled);
+                if (ns > 0) {
+                    __syncthreads(); // the reservation made since the last level
+                    store_found<kListPer>(L, it.found, e, won, f, F);
+                    push_shared(L, g, M, qa, ns, rank, T, lvl, par, cap, spill_ctr, qb, F, spilled);
+                }
+                // the shared queue's entries and the leader's zeros are in
+                // place before the arrival
+                if (spilled || (rank == 0 && wid == 0)) __builtin_amdgcn_s_waitcnt(0);
                 __syncthreads();
-                for (int64_t wb = 0; wb < Te; wb += kBWin) { // uniform
-                    int64_t e = wb + (int64_t)tid * kBPer;
-                    const int64_t e_end = e + kBPer < Te ? e + kBPer : Te;
-                    int lo = 0;
-                    if (e < e_end) {
-                        int hi = cnt_e;
-                        while (hi - lo > 1) {
-                            const int mid = (lo + hi) >> 1;
-                            if (S.pre[mid] <= e) lo = mid;
-                            else hi = mid;
-                        }
-                    }
-                    int32_t v[kBPer];
-                    uint32_t ou[kBPer];
-                    bool okv[kBPer];
-#pragma unroll
-                    for (int i = 0; i < kBPer; ++i) {
-                        okv[i] = e < e_end;
-                        v[i] = 0;
-                        ou[i] = 0;
-                        if (okv[i]) {
-                            while (lo + 1 < cnt_e && S.pre[lo + 1] <= e) ++lo;
-                            v[i] = g.push_col[S.start[lo] + (e - S.pre[lo])];
-                            ou[i] = S.ou[lo];
-                            ++e;
-                        }
-                    }
-                    // the key decides: no visited filter on the way
-                    bool won[kBPer];
-#pragma unroll
-                    for (int i = 0; i < kBPer; ++i) {
-                        won[i] = false;
-                        if (okv[i]) won[i] = atomicMin(&it.key[v[i]], lkey | ou[i]) == ~0ull;
-                    }
-#pragma unroll
-                    for (int i = 0; i < kBPer; ++i) {
-                        if (won[i]) {
-                            const uint64_t bit = 1ull << (v[i] & 63);
-                            const unsigned long long old =
-                                atomicOr(reinterpret_cast<unsigned long long *>(&bnext[v[i] >> 6]), bit);
-                            atomicOr(reinterpret_cast<unsigned long long *>(&it.visited[v[i] >> 6]), bit);
-                            my_w += old == 0 ? 1 : 0;
-                            my_e += (unsigned long long)(g.push_ptr[v[i] + 1] - g.push_ptr[v[i]]);
-                        }
-                    }
-#pragma unroll
-                    for (int i = 0; i < kBPer; ++i) {
-                        const unsigned int pf = wave_append(&S.nf, won[i]);
-                        if (won[i]) S.found[pf] = v[i];
-                    }
-                    flush_found(S, it, reinterpret_cast<unsigned long long *>(&slot[0]), fe_cur);
+                if (poll == 0) {
+                    if (lane < 3)
+                        L.arrive[lane] =
+                            lane == 0 ? (L.cnt[par] & 0xffffffffull) : (lane == 1 ? L.edges[par] : L.spill[par]);
+                    team_arrive(L, B, tag + 1);
                 }
-                __syncthreads(); // pre/start/ou are restaged
-            }
+                if (ns == 0) store_found<kListPer>(L, it.found, e, won, f, F);
+                const unsigned long long mine = uniform64(L.cnt[par]);
+                F += (int64_t)(mine & 0xffffffffull);
+                listed = (int)((mine >> 32) < (unsigned long long)cap ? (mine >> 32) : (unsigned long long)cap);
+                load_list(L, g, M, listed, e);
+                if (poll >= 0) team_poll(L, B, poll, tag + 1);
+                ++tag;
+                __syncthreads();
+                if (!L.ok) return false;
+                F_prev = Fr;
+                Fr = uniform64(L.tot[0]);
+                mf = uniform64(L.tot[1]);
+                ns = (int64_t)uniform64(L.tot[2]);
+                if (tid == 0) reserve_found(L, M, F);
+                cap = list_cap((int64_t)(mine >> 32), (int64_t)mf, T);
+                int32_t *t = qa;
+                qa = qb;
+                qb = t;
+                reached += Fr;
+                redges += mf;
+                ++Lv;
+            } while (Fr > 0 && !decide(Fr, mf, redges));
+            prev_choice = ALBBA_CHOICE_PUSH;
         } else {
             ++pulls;
+            const int lane = here_tid() & 63, wid = here_tid() >> 6;
+            unsigned long long my_f = 0, my_e = 0, my_w = 0;
+            if (old_dirty)
+                for (int64_t i = team_tid(); i < nwords; i += gthreads) st_coherent(&bold[i], (uint64_t)0);
+            const unsigned long long lkey = (unsigned long long)(uint32_t)(Lv + 1) << 32;
             // pull: workgroup `rank` takes words [w0, w1) in runs of 64; wave
             // wid takes every kBWaves-th run.  The wave's lanes test the 64
-            // words of a run at once (rows with a length, not visited: every
-            // vertex found so far has its visited bit, set by its
-            // discoverer), then the wave works through the words that have
+            // words of a run at once (rows with a length, not visited), then the wave works through the words that have
             // such rows; their unvisited lanes look for their row's first
             // neighbour in B_L (rows list neighbours by ascending id)
             const int64_t per = (nwords + T - 1) / T;
@@ -361,35 +371,27 @@ __device__ bool run_instance(BLds &S, const albd_batch_item &it, int rank, int T
                     }
                 }
             }
+            const unsigned long long f = block_sum(S, 0, my_f), me = block_sum(S, 1, my_e), mw = block_sum(S, 2, my_w);
+            if (!team_barrier(L, B, ++tag, f, me, mw)) return false;
+            F_prev = Fr;
+            Fr = uniform64(L.tot[0]);
+            mf = uniform64(L.tot[1]);
+            nzw = uniform64(L.tot[2]);
+            // the lists are of the frontier before
+            lists = false;
+            old_dirty = true;
+            uint64_t *t = bold;
+            bold = bcur;
+            bcur = bnext;
+            bnext = t;
+            reached += Fr;
+            redges += mf;
+            ++Lv;
+            prev_choice = ALBBA_CHOICE_PULL;
         }
-        add_counts(S, slot, my_f, my_e, my_w);
-        if (!team_sync(bar, err, T, spin_limit, &S.ok)) return false;
-        // B_{L+1} is complete: its size, out-edges, words and (push) list
-        mf = (unsigned long long)ld_coherent(&slot[1]);
-        nzw = (unsigned long long)ld_coherent(&slot[3]);
-        fs_prev = fs_cur;
-        fe_prev = fe_cur;
-        prev_by_pull = cur_by_pull;
-        F_prev = F;
-        if (push) {
-            // the level's appends, counted in its own ring slot: a
-            // workgroup past the barrier may already append for the next
-            // level while another still reads this one's count
-            F = (unsigned long long)ld_coherent(&slot[0]);
-            fs_cur = fe_cur;
-            fe_cur += (int64_t)F;
-        } else {
-            F = (unsigned long long)ld_coherent(&slot[0]);
-            fs_cur = fe_cur; // a pulled level lists nothing
-        }
-        have_queue = push;
-        cur_by_pull = !push;
-        reached += F;
-        redges += mf;
-        prev_choice = push ? ALBBA_CHOICE_PUSH : ALBBA_CHOICE_PULL;
     }
     // results in vertex order from the keys; the keys go back to all ones
-    for (int64_t v = gtid; v < g.n; v += gthreads) {
+    for (int64_t v = team_tid(); v < g.n; v += gthreads) {
         const int32_t p = g.pos_of[v];
         const unsigned long long k = ld_coherent(&it.key[p]);
         const bool hit = k != ~0ull;
@@ -397,17 +399,37 @@ __device__ bool run_instance(BLds &S, const albd_batch_item &it, int rank, int T
         it.parent[v] = hit ? (int32_t)(uint32_t)k : -1;
         if (hit) st_coherent(&it.key[p], ~0ull);
     }
-    if (!team_sync(bar, err, T, spin_limit, &S.ok)) return false;
+    if (!team_barrier(L, B, ++tag)) return false;
     if (leader) {
-        long long *res = reinterpret_cast<long long *>(it.ctl);
-        st_coherent(&res[ALBD_RES_LEVELS], (long long)L);
-        st_coherent(&res[ALBD_RES_REACHED], (long long)reached);
-        st_coherent(&res[ALBD_RES_EDGES], (long long)redges);
-        st_coherent(&res[ALBD_RES_PUSHES], pushes);
-        st_coherent(&res[ALBD_RES_PULLS], pulls);
-        st_coherent(&res[ALBD_RES_T1], (long long)wall_clock64());
+        long long *r = reinterpret_cast<long long *>(it.ctl);
+        st_coherent(&r[ALBD_RES_LEVELS], (long long)Lv);
+        st_coherent(&r[ALBD_RES_REACHED], (long long)reached);
+        st_coherent(&r[ALBD_RES_EDGES], (long long)redges);
+        st_coherent(&r[ALBD_RES_PUSHES], pushes);
+        st_coherent(&r[ALBD_RES_PULLS], pulls);
+        st_coherent(&r[ALBD_RES_T1], (long long)wall_clock64());
     }
     return true;
+}
+
+// The descriptor of an instance through the constant address space: nothing
+// writes it during the launch, so that its uniform fields come as scalar loads
+// into scalar registers (as ordinary memory, which the kernel's stores might
+// change, each pointer took a pair of vector registers, and the push loop
+// spilled).
+__device__ __forceinline__ albd_batch_item load_item(const albd_batch_item *items, int32_t i)
+{
+    typedef const __attribute__((address_space(4))) uint32_t *ConstWords;
+    constexpr int kWords = (int)(sizeof(albd_batch_item) / 4);
+    static_assert(sizeof(albd_batch_item) % 4 == 0, "copied by word");
+    union {
+        albd_batch_item it;
+        uint32_t w[kWords];
+    } u;
+    const ConstWords src = (ConstWords)(uintptr_t)&items[__builtin_amdgcn_readfirstlane(i)];
+#pragma unroll
+    for (int k = 0; k < kWords; ++k) u.w[k] = src[k];
+    return u.it;
 }
 
 __global__ __launch_bounds__(kBB, 4) void k_bfs_batch(albd_batch_args a)
@@ -415,10 +437,11 @@ __global__ __launch_bounds__(kBB, 4) void k_bfs_batch(albd_batch_args a)
     __shared__ BLds S;
     if (a.params) mlp_to_lds<kBB>(S.params, a.params);
     __syncthreads();
-    const int t = a.wg_team[blockIdx.x];
-    const int rank = (int)blockIdx.x - a.team_first[t], T = a.team_size[t];
+    const int t = __builtin_amdgcn_readfirstlane(a.wg_team[blockIdx.x]);
+    const int rank = (int)blockIdx.x - __builtin_amdgcn_readfirstlane(a.team_first[t]);
+    const int T = __builtin_amdgcn_readfirstlane(a.team_size[t]);
     for (int j = a.team_ptr[t]; j < a.team_ptr[t + 1]; ++j) {
-        const albd_batch_item &it = a.items[a.team_items[j]];
+        const albd_batch_item it = load_item(a.items, a.team_items[j]);
         if (!run_instance(S, it, rank, T, a.params != nullptr, a.spin_limit)) {
             if (threadIdx.x == 0)
                 st_coherent(reinterpret_cast<long long *>(it.ctl) + ALBD_RES_ERROR, 1ll);

@@ -20,6 +20,7 @@
 // finds pmin[v] still all ones sets v in the next bitmap; a word pass then
 // writes level/parent and builds the next queue.
 #include "dev_common.h"
+#include "push_lists.h"
 #include "select_dev.h"
 #include "../../../include/albba.h"
 
@@ -1114,8 +1115,8 @@ __global__ __launch_bounds__(kBlock) void k_push_expand(albd_graph g, albd_state
 // everything that is not the atomic or the barrier is off that chain:
 //   - a workgroup keeps the vertices it finds as its own part of the next
 //     frontier, as a list of their edges in LDS (no queue in memory between
-//     levels); vertices with more than kSmallDeg out-edges, and those beyond
-//     the list's kSmallEdges, go to a queue in memory that the workgroups
+//     levels); vertices with more than kListDeg out-edges, and those beyond
+//     the list's kListEdges, go to a queue in memory that the workgroups
 //     share evenly at the next level;
 //   - the edges' columns, filters, degrees and vertex ids -- data that no
 //     level changes, but for the keys, which are only a filter -- are loaded
@@ -1143,15 +1144,6 @@ __global__ __launch_bounds__(kBlock) void k_push_expand(albd_graph g, albd_state
 // workgroups on one XCD changed nothing at 0.6 M vertices (4.1 us) and cost at
 // 16.8 M (8.3 us with 32 workgroups): the misses go to memory either way.
 
-constexpr int kSmallBlock = 512;
-constexpr int kSmallWaves = kSmallBlock / 64;
-constexpr int kSmallPer = 2;                           // edges per thread per window
-constexpr int kSmallEdges = kSmallPer * kSmallBlock;   // edges per window, and of the LDS list
-constexpr int kSmallDeg = 32;                          // most out-edges of a listed vertex
-constexpr int kSmallSlack = 64, kSmallKeep = 32;       // see the levels' end
-constexpr int kSmallFound = 1024;                      // found-list entries reserved at a time
-static_assert(kSmallFound >= kSmallEdges, "a window finds at most one reservation more");
-
 struct SmallArgs {
     albd_graph g;
     albd_state st;
@@ -1162,198 +1154,31 @@ struct SmallArgs {
     uint32_t spin_limit;
 };
 
-struct SmallLds {
-    // the next level's own edges: entry in push_col (-1: none) and source id
-    int32_t ecol[kSmallEdges];
-    uint32_t eou[kSmallEdges];
-    // a staged part of the shared queue
-    int64_t pre[kSmallBlock], start[kSmallBlock];
-    uint32_t ou[kSmallBlock];
-    int64_t scan[kSmallWaves];
-    // per level parity: listed edges << 32 | found; their out-edges; spilled
-    unsigned long long cnt[2], edges[2], spill[2];
-    unsigned long long tot[3]; // the grid's sums of found, edges, spilled
-    int64_t chunk[2];          // found-list reservations in use, by number & 1
-    int64_t reserved;          // reservations made so far
-    int ok;
-};
-
-// One edge of a lane: target position, its row and id, the source's id and
-// the filters.
-struct SmallEdge {
-    bool act;
-    int32_t v, start, deg;
-    uint32_t ou, ro;
-    uint64_t vis;
-    unsigned long long pk;
-};
-
-__device__ __forceinline__ void small_target(const albd_graph &g, const albd_state &st, SmallEdge &e)
-{
-    e.vis = e.act ? st.visited[e.v >> 6] : ~0ull;
-    e.pk = e.act ? st.pkey[e.v] : 0ull;
-    const int64_t a = e.act ? g.push_ptr[e.v] : 0, b = e.act ? g.push_ptr[e.v + 1] : 0;
-    e.start = (int32_t)a;
-    e.deg = (int32_t)(b - a);
-    e.ro = e.act ? (uint32_t)g.row_order[e.v] : 0u;
-}
-
-// Relax a window of edges (every lane of the wave calls): won lanes are their
-// vertices' discoverers; f gets their numbers among the level's found.
-__device__ __forceinline__ void small_relax(SmallLds &S, const albd_state &st, const SmallEdge (&e)[kSmallPer],
-                                            uint32_t lvl, int par, int cap, unsigned long long *spill_ctr,
-                                            int32_t *qb, bool (&won)[kSmallPer], uint32_t (&f)[kSmallPer], bool &spilled)
-{
-    const int lane = lane_id();
-#pragma unroll
-    for (int i = 0; i < kSmallPer; ++i) {
-        won[i] = false;
-        // unvisited at the launch and not found at an earlier level of it
-        if (e[i].act && !((e[i].vis >> (e[i].v & 63)) & 1ull) && (uint32_t)(e[i].pk >> 32) >= lvl)
-            won[i] = atomicMin(&st.pkey[e[i].v], ((unsigned long long)lvl << 32) | e[i].ou) == ~0ull;
-    }
-#pragma unroll
-    for (int i = 0; i < kSmallPer; ++i) {
-        const uint64_t m = __ballot(won[i]);
-        f[i] = 0;
-        if (m == 0) continue; // wave-uniform
-        const int32_t deg = won[i] ? e[i].deg : 0;
-        const bool listed = deg > 0 && deg <= kSmallDeg;
-        // exclusive prefix of the listed degrees, bit by bit
-        uint32_t pre = 0, tot = 0;
-#pragma unroll
-        for (int b = 0; b < 6; ++b) {
-            const uint64_t mb = __ballot(listed && ((deg >> b) & 1));
-            pre += (uint32_t)__popcll(mb & lanemask_lt(lane)) << b;
-            tot += (uint32_t)__popcll(mb) << b;
-        }
-        static_assert(kSmallDeg < 64, "six bits hold a listed degree");
-        const unsigned long long es = wave_sum((unsigned long long)(uint32_t)deg);
-        unsigned long long base = 0;
-        if (lane == 0) {
-            base = atomicAdd(&S.cnt[par], ((unsigned long long)tot << 32) | (unsigned long long)__popcll(m));
-            if (es) atomicAdd(&S.edges[par], es);
-        }
-        base = __shfl(base, 0, 64);
-        f[i] = (uint32_t)base + (uint32_t)__popcll(m & lanemask_lt(lane));
-        const unsigned long long e0 = (base >> 32) + pre;
-        const bool fits = listed && e0 + (unsigned long long)deg <= (unsigned long long)cap;
-        if (listed)
-            for (int k = 0; k < deg; ++k) {
-                if (e0 + k >= (unsigned long long)cap) break;
-                S.ecol[e0 + k] = fits ? e[i].start + k : -1;
-                S.eou[e0 + k] = e[i].ro;
-            }
-        const bool sp = deg > 0 && !fits;
-        const uint64_t ms = __ballot(sp);
-        if (ms) {
-            unsigned long long q = 0;
-            if (lane == 0) {
-                q = atomicAdd(spill_ctr, (unsigned long long)__popcll(ms));
-                atomicAdd(&S.spill[par], (unsigned long long)__popcll(ms));
-            }
-            q = __shfl(q, 0, 64);
-            if (sp) st_coherent(&qb[q + __popcll(ms & lanemask_lt(lane))], e[i].v);
-            spilled = true;
-        }
-    }
-}
-
-// the workgroup's found vertices of one window -> its reservations; F: found
-// before this level
-__device__ __forceinline__ void small_store_found(const SmallLds &S, int32_t *found,
-                                                  const SmallEdge (&e)[kSmallPer], const bool (&won)[kSmallPer],
-                                                  const uint32_t (&f)[kSmallPer], int64_t F)
-{
-#pragma unroll
-    for (int i = 0; i < kSmallPer; ++i)
-        if (won[i]) {
-            const int64_t at = F + f[i];
-            st_coherent(&found[S.chunk[(at / kSmallFound) & 1] + at % kSmallFound], e[i].v);
-        }
-}
-
-// room for a window's found vertices after the first `at` (thread 0)
-__device__ __forceinline__ void small_reserve(SmallLds &S, albd_persist *P, int64_t at)
-{
-    while (S.reserved < at / kSmallFound + 2) {
-        S.chunk[S.reserved & 1] = (int64_t)atomicAdd(&P->reserve, (unsigned long long)kSmallFound);
-        ++S.reserved;
-    }
-}
-
-// arrival: the workgroup's counts of a level (three lanes of one wave)
-__device__ __forceinline__ void small_arrive(const SmallLds &S, albd_persist *P, int par, unsigned int tag)
-{
-    const int lane = lane_id();
-    if (lane < 3) {
-        const unsigned long long x = lane == 0 ? (S.cnt[par] & 0xffffffffull) : (lane == 1 ? S.edges[par] : S.spill[par]);
-        st_coherent(&P->slot[tag & 1][lane][blockIdx.x], ((unsigned long long)tag << 48) | x);
-    }
-}
-
-// wait for every workgroup's arrival with `tag`; the wave sums word `k`
-__device__ __forceinline__ void small_poll(SmallLds &S, albd_persist *P, int k, unsigned int tag,
-                                           uint32_t spin_limit)
-{
-    const int lane = lane_id();
-    const unsigned int G = gridDim.x;
-    const unsigned long long *slot = P->slot[tag & 1][k];
-    unsigned long long sum = 0;
-    bool ok = true;
-    for (uint32_t spins = 0;; ++spins) {
-        bool all = true;
-        sum = 0;
-        for (unsigned int i = lane; i < G; i += 64) {
-            const unsigned long long x = ld_coherent(&slot[i]);
-            all = all && (x >> 48) == tag;
-            sum += x & ((1ull << 48) - 1);
-        }
-        if (__ballot(!all) == 0) break;
-        if (spins >= spin_limit || ((spins & 63) == 63 && ld_coherent(&P->error) != 0)) {
-            ok = false;
-            break;
-        }
-    }
-    sum = wave_sum(sum);
-    if (lane == 0) {
-        S.tot[k] = sum;
-        if (!ok) {
-            atomicOr(&P->error, 1u);
-            S.ok = 0;
-        }
-    }
-}
-
-__global__ __launch_bounds__(kSmallBlock) void k_push_small(SmallArgs a)
+__global__ __launch_bounds__(kListBlock) void k_push_small(SmallArgs a)
 {
     const albd_graph &g = a.g;
     const albd_state &st = a.st;
-    __shared__ SmallLds S;
+    __shared__ PushLds S;
     albd_persist *P = st.persist;
-    // every vertex this launch finds, in reservations of kSmallFound entries
-    int32_t *found = reinterpret_cast<int32_t *>(st.prefix);
+    // every vertex this launch finds goes to the prefix array's memory
+    const PushMem M{st.visited, st.pkey, reinterpret_cast<int32_t *>(st.prefix), &P->reserve};
+    int32_t *found = M.found;
     const int64_t found_cap = 2 * (g.npos + 1);
     int32_t *qa = st.queue, *qb = st.queue_next;
     const int tid = threadIdx.x, lane = lane_id(), wid = tid >> 6;
     const unsigned int G = gridDim.x, w = blockIdx.x;
+    const TeamSlots B{&P->slot[0][0][0], &P->error, ALBD_PERSIST_BLOCKS, (int32_t)G, (int32_t)w, a.spin_limit};
     // the waves that poll the slots: the last ones, which hold the fewest edges
-    const int poll = wid - (kSmallWaves - 3);
-    if (tid < 2) {
-        S.cnt[tid] = S.edges[tid] = S.spill[tid] = 0;
-        S.chunk[tid] = 0;
-    }
-    if (tid == 0) {
-        S.ok = 1;
-        S.reserved = 0;
-        small_reserve(S, P, 0);
-    }
+    const int poll = wid - (kListWaves - 3);
+    list_reset(S);
+    __syncthreads();
+    if (tid == 0) reserve_found(S, M, 0);
     int64_t ns = (int64_t)st.ctr->queue_len; // the shared queue's length
     int64_t F = 0;                           // found by this workgroup before the level
-    SmallEdge e[kSmallPer];
+    PushEdge e[kListPer];
 #pragma unroll
-    for (int i = 0; i < kSmallPer; ++i) e[i].act = false;
-    int cap = kSmallEdges; // edges the list takes at this level
+    for (int i = 0; i < kListPer; ++i) e[i].act = false;
+    int cap = kListEdges; // edges the list takes at this level
     bool ok = true;
     __syncthreads();
     int k = 0;
@@ -1363,89 +1188,36 @@ __global__ __launch_bounds__(kSmallBlock) void k_push_small(SmallArgs a)
         const int par = k & 1;
         unsigned long long *spill_ctr = reinterpret_cast<unsigned long long *>(&st.level_log[4 * k + 2]);
         if (tid == 0) S.cnt[par ^ 1] = S.edges[par ^ 1] = S.spill[par ^ 1] = 0;
-        bool won[kSmallPer], spilled = false;
-        uint32_t f[kSmallPer];
-        // the workgroup's own edges, loaded while it waited
-        small_relax(S, st, e, lvl, par, cap, spill_ctr, qb, won, f, spilled);
+        bool won[kListPer], spilled = false;
+        uint32_t f[kListPer];
+        // the workgroup's own edges, loaded while it waited, then its share
+        // of the queue in memory
+        relax_edges<kListPer, false>(S, g, M, e, lvl, par, cap, spill_ctr, qb, won, f, spilled);
         if (ns > 0) {
-            // its share of the queue in memory: entries [q0, q1)
-            small_store_found(S, found, e, won, f, F);
-            const int64_t per = (ns + G - 1) / G;
-            const int64_t q0 = (int64_t)w * per, q1 = q0 + per < ns ? q0 + per : ns;
-            for (int64_t base = q0; base < q1; base += kSmallBlock) { // uniform in the workgroup
-                const int cnt_e = (int)(q1 - base < kSmallBlock ? q1 - base : kSmallBlock);
-                int64_t a0 = 0, a1 = 0;
-                uint32_t o0 = 0;
-                if (tid < cnt_e) {
-                    const int32_t u = ld_coherent(&qa[base + tid]);
-                    a0 = g.push_ptr[u];
-                    a1 = g.push_ptr[u + 1];
-                    o0 = (uint32_t)g.row_order[u];
-                }
-                int64_t T;
-                const int64_t ex = block_scan_excl<kSmallBlock>(a1 - a0, &T, S.scan);
-                S.pre[tid] = ex;
-                S.start[tid] = a0;
-                S.ou[tid] = o0;
-                for (int64_t wb = 0; wb < T; wb += kSmallEdges) { // uniform
-                    // every found of the earlier windows has its place
-                    __syncthreads();
-                    if (tid == 0) small_reserve(S, P, F + (int64_t)(S.cnt[par] & 0xffffffffull));
-                    __syncthreads();
-                    SmallEdge x[kSmallPer];
-#pragma unroll
-                    for (int i = 0; i < kSmallPer; ++i) {
-                        const int64_t en = wb + i * kSmallBlock + tid;
-                        x[i].act = en < T;
-                        x[i].v = 0;
-                        x[i].ou = 0;
-                        if (x[i].act) {
-                            int lo = 0, hi = cnt_e;
-                            while (hi - lo > 1) {
-                                const int mid = (lo + hi) >> 1;
-                                if (S.pre[mid] <= en) lo = mid;
-                                else hi = mid;
-                            }
-                            x[i].v = g.push_col[S.start[lo] + (en - S.pre[lo])];
-                            x[i].ou = S.ou[lo];
-                        }
-                    }
-#pragma unroll
-                    for (int i = 0; i < kSmallPer; ++i) small_target(g, st, x[i]);
-                    bool xw[kSmallPer];
-                    uint32_t xf[kSmallPer];
-                    small_relax(S, st, x, lvl, par, cap, spill_ctr, qb, xw, xf, spilled);
-                    small_store_found(S, found, x, xw, xf, F);
-                }
-                __syncthreads(); // the staged entries are replaced
-            }
+            __syncthreads(); // the reservation made since the last level
+            store_found<kListPer>(S, found, e, won, f, F);
+            push_shared(S, g, M, qa, ns, (int)w, (int)G, lvl, par, cap, spill_ctr, qb, F, spilled);
         }
         // the shared queue's entries are in place before the arrival
         if (spilled) __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        if (poll == 0) small_arrive(S, P, par, (unsigned int)(k + 1));
+        if (poll == 0) {
+            if (lane < 3)
+                S.arrive[lane] = lane == 0 ? (S.cnt[par] & 0xffffffffull) : (lane == 1 ? S.edges[par] : S.spill[par]);
+            team_arrive(S, B, (unsigned int)(k + 1));
+        }
         // off the chain: the found list, and everything about the next
         // level's own edges but the atomic
-        if (ns == 0) small_store_found(S, found, e, won, f, F);
-        const unsigned long long mine = S.cnt[par];
+        if (ns == 0) store_found<kListPer>(S, found, e, won, f, F);
+        const unsigned long long mine = uniform64(S.cnt[par]);
         F += (int64_t)(mine & 0xffffffffull);
-        const int T = (int)((mine >> 32) < (unsigned long long)cap ? (mine >> 32) : (unsigned long long)cap);
-#pragma unroll
-        for (int i = 0; i < kSmallPer; ++i) {
-            const int en = i * kSmallBlock + tid;
-            const int32_t at = en < T ? S.ecol[en] : -1;
-            e[i].act = at >= 0;
-            e[i].ou = e[i].act ? S.eou[en] : 0;
-            e[i].v = e[i].act ? g.push_col[at] : 0;
-        }
-#pragma unroll
-        for (int i = 0; i < kSmallPer; ++i) small_target(g, st, e[i]);
-        if (poll >= 0) small_poll(S, P, poll, (unsigned int)(k + 1), a.spin_limit);
+        load_list(S, g, M, (int)((mine >> 32) < (unsigned long long)cap ? (mine >> 32) : (unsigned long long)cap), e);
+        if (poll >= 0) team_poll(S, B, poll, (unsigned int)(k + 1));
         __syncthreads();
         ok = S.ok != 0;
         if (!ok) break;
-        const int64_t na = (int64_t)S.tot[0], edges = (int64_t)S.tot[1];
-        ns = (int64_t)S.tot[2];
+        const int64_t na = (int64_t)uniform64(S.tot[0]), edges = (int64_t)uniform64(S.tot[1]);
+        ns = (int64_t)uniform64(S.tot[2]);
         if (w == 0 && tid == 0) {
             st.level_log[4 * k] = na;
             st.level_log[4 * k + 1] = edges;
@@ -1457,29 +1229,20 @@ __global__ __launch_bounds__(kSmallBlock) void k_push_small(SmallArgs a)
             st.ctr->reached += (unsigned long long)na;
             st.ctr->reached_edges += (unsigned long long)edges;
         }
-        if (tid == 0) small_reserve(S, P, F);
-        // a workgroup that holds more than twice its part of the edges keeps
-        // half a part of what it finds next and shares the rest
-        const int64_t part = edges / G;
-        cap = (int64_t)(mine >> 32) > 2 * part + kSmallSlack
-                  ? (int)(part / 2 < kSmallKeep ? kSmallKeep : (part / 2 > kSmallEdges ? kSmallEdges : part / 2))
-                  : kSmallEdges;
+        if (tid == 0) reserve_found(S, M, F);
+        cap = list_cap((int64_t)(mine >> 32), edges, (int)G);
         int32_t *t = qa;
         qa = qb;
         qb = t;
     }
     if (ok) {
         const unsigned long long na = S.tot[0], edges = S.tot[1];
-        // the unused ends of the reservations hold no vertex
-        for (int64_t j = F + tid; j < S.reserved * kSmallFound; j += kSmallBlock) {
-            const int64_t at = S.chunk[(j / kSmallFound) & 1] + j % kSmallFound;
-            if (at < found_cap) st_coherent(&found[at], (int32_t)-1);
-        }
+        end_found(S, M, F, found_cap);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         // (the counts of this arrival are not used)
-        if (poll == 0) small_arrive(S, P, k & 1, (unsigned int)(k + 2));
-        if (poll >= 0) small_poll(S, P, poll, (unsigned int)(k + 2), a.spin_limit);
+        if (poll == 0) team_arrive(S, B, (unsigned int)(k + 2));
+        if (poll >= 0) team_poll(S, B, poll, (unsigned int)(k + 2));
         __syncthreads();
         ok = S.ok != 0;
         if (ok) {
@@ -1489,8 +1252,8 @@ __global__ __launch_bounds__(kSmallBlock) void k_push_small(SmallArgs a)
             int64_t total = (int64_t)ld_coherent(&P->reserve);
             if (total > found_cap) total = found_cap;
             unsigned long long my_words = 0;
-            for (int64_t b = ((int64_t)w * kSmallWaves + wid) * 64; b < total;
-                 b += (int64_t)G * kSmallBlock) { // uniform in the wave
+            for (int64_t b = ((int64_t)w * kListWaves + wid) * 64; b < total;
+                 b += (int64_t)G * kListBlock) { // uniform in the wave
                 const int64_t i = b + lane;
                 const int32_t v = i < total ? ld_coherent(&found[i]) : -1;
                 bool queued = false;
@@ -1804,13 +1567,14 @@ int albd_push_small(albd_ctx *c, const albd_graph *g, const albd_state *st, int3
     // that could not become resident would only make the barrier give up
     // after spin_limit polls (ctr->persist_error), never hang.
     int per_cu = 0;
-    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_push_small, kSmallBlock, 0));
+    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_push_small, kListBlock, 0));
     int64_t cap = (int64_t)per_cu * albd_num_cus(c);
     if (cap < 1) return albd_set_error_msg(ALBBA_EHIP, "small-frontier kernel cannot be resident");
     if (cap > ALBD_PERSIST_BLOCKS) cap = ALBD_PERSIST_BLOCKS;
     // the found list (2 (npos + 1) entries) holds every vertex and the up to
-    // two unfilled reservations of every workgroup
-    if (cap > g->npos / (2 * kSmallFound)) cap = g->npos / (2 * kSmallFound);
+    // two unfilled reservations of every workgroup (one workgroup's are in order,
+    // so that its vertices alone fit)
+    if (cap > g->npos / (2 * kFound)) cap = g->npos / (2 * kFound);
     if (cap < 1) cap = 1;
     // More workgroups shorten each one's part of a level but lengthen the
     // barrier: measured us per level with 16, 32 and 64 workgroups on grids
@@ -1821,7 +1585,7 @@ int albd_push_small(albd_ctx *c, const albd_graph *g, const albd_state *st, int3
     // the grid state, the levels' counters and the error flag were zeroed by
     // the level-begin kernel (LB_SMALL)
     SmallArgs a{*g, *st, level0, max_levels, edge_cap, vertex_cap, spin_limit};
-    hipLaunchKernelGGL(k_push_small, dim3(blocks), dim3(kSmallBlock), 0, albd_stream(c), a);
+    hipLaunchKernelGGL(k_push_small, dim3(blocks), dim3(kListBlock), 0, albd_stream(c), a);
     HIPCHK(hipGetLastError());
     return 0;
 }

@@ -87,6 +87,14 @@ __device__ __forceinline__ T wave_sum(T v)
     }
 }
 
+// a value that is the same in every lane, in scalar registers
+__device__ __forceinline__ unsigned long long uniform64(unsigned long long x)
+{
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(x >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+
 // ---------------------------------------------------------------------------
 // cross-workgroup communication inside one launch
 //
@@ -110,20 +118,6 @@ template <class T> __device__ __forceinline__ void st_coherent(T *p, T v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// append one entry per predicated lane to an LDS list: returns the slot of
-// this lane (valid where pred holds); works under any exec mask
-__device__ __forceinline__ unsigned int wave_append(unsigned int *counter, bool pred)
-{
-    const uint64_t m = __ballot(pred);
-    if (m == 0) return 0;
-    const int lane = lane_id();
-    const int leader = __ffsll((unsigned long long)__ballot(1)) - 1;
-    unsigned int base = 0;
-    if (lane == leader) base = atomicAdd(counter, (unsigned int)__popcll(m));
-    base = __shfl(base, leader, 64);
-    return base + (unsigned int)__popcll(m & lanemask_lt(lane));
-}
-
 // exclusive scan of one value per thread over a BLOCK-thread workgroup;
 // lds holds BLOCK/64 entries and is free again after the next barrier
 template <int BLOCK>
@@ -143,32 +137,3 @@ __device__ __forceinline__ int64_t block_scan_excl(int64_t v, int64_t *total, in
     *total = tot;
     return ex + off;
 }
-
-// Barrier over `members` co-resident workgroups sharing a counter that only
-// grows (zeroed before the launch).  Wave 0 of each workgroup arrives and
-// polls.  Gives up after spin_limit polls or once *error is set, so every
-// wave always reaches the end of the kernel; returns false then.
-__device__ __forceinline__ bool team_sync(unsigned long long *counter, unsigned int *error,
-                                          unsigned int members, unsigned int spin_limit, int *s_ok)
-{
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int ok = 1;
-        const unsigned long long arrived = atomicAdd(counter, 1ull);
-        const unsigned long long target = (arrived / members + 1) * members;
-        unsigned int spins = 0;
-        while (ld_coherent(counter) < target) {
-            if (++spins > spin_limit || ld_coherent(error) != 0) {
-                atomicOr(error, 1u);
-                ok = 0;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(2);
-        }
-        *s_ok = ok;
-    }
-    __syncthreads();
-    return *s_ok != 0;
-}
-

@@ -15,7 +15,12 @@
 //
 // Called by all 64 lanes of one wave with the same arguments: the seven
 // log2(1 + x) terms are computed one per lane (double precision, about a
-// hundred instructions each), then lane 0 writes xs.
+// hundred instructions each), then lane 0 writes xs.  CALL: the logarithm as a
+// call, for a kernel that needs it now and then in a loop: inlined, its
+// constants are hoisted out of the loop and fill the kernel's registers.
+__device__ __attribute__((noinline)) inline double log2_call(double x) { return log2(x); }
+
+template <bool CALL = false>
 __device__ inline void level_features(float *xs, int64_t n_, int64_t nnz, int64_t nwords,
                                       unsigned long long F, unsigned long long mf,
                                       unsigned long long nzw, unsigned long long reached,
@@ -37,7 +42,7 @@ __device__ inline void level_features(float *xs, int64_t n_, int64_t nnz, int64_
     case 6: num = (double)F; den = (double)(F_prev > 0 ? F_prev : 1); break;
     default: break;
     }
-    const double y = log2(1.0 + num / den);
+    const double y = CALL ? log2_call(1.0 + num / den) : log2(1.0 + num / den);
     const double lF = __shfl(y, 0), ln = __shfl(y, 1), lmf = __shfl(y, 2), lm = __shfl(y, 3),
                  ldeg = __shfl(y, 4), lmn = __shfl(y, 5), lgrow = __shfl(y, 6);
     if (lane == 0) {
@@ -173,7 +178,8 @@ __device__ inline int mlp_argmin_wave(const float *params, const float *xs, floa
 // it contains barriers), with the parameters in LDS as mlp_to_lds lays them
 // out.  The sums run in the same order as the training kernels' forward.
 // Returns the argmin over the choices in valid_mask to every thread, or -1 if
-// none is valid.
+// none is valid.  (Unrolled in part only: the batched kernel calls it a few
+// times per BFS and needs its registers elsewhere.)
 __device__ inline int mlp_argmin(const float *params, const float *xs, float *h1, float *h2,
                                  float *ys, int valid_mask, int *s_choice)
 {
@@ -183,21 +189,21 @@ __device__ inline int mlp_argmin(const float *params, const float *xs, float *h1
                 *W3T = B2 + H2, *B3 = W3T + O * H2;
     if (tid < H1) {
         float a = B1[tid];
-#pragma unroll
+#pragma unroll 4
         for (int i = 0; i < I; ++i) a = fmaf(W1T[i * H1 + tid], xs[i], a);
         h1[tid] = a > 0.f ? a : 0.f;
     }
     __syncthreads();
     if (tid < H2) {
         float a = B2[tid];
-#pragma unroll
+#pragma unroll 4
         for (int i = 0; i < H1; ++i) a = fmaf(W2T[i * H2 + tid], h1[i], a);
         h2[tid] = a > 0.f ? a : 0.f;
     }
     __syncthreads();
     if (tid < O) {
         float a = B3[tid];
-#pragma unroll
+#pragma unroll 4
         for (int i = 0; i < H2; ++i) a = fmaf(W3T[i * O + tid], h2[i], a);
         ys[tid] = a;
     }

@@ -11,16 +11,16 @@
  * Later runs (split_teams_hist) use the level count L and run time t of
  * every instance in the first run (the share split).  A level costs a team
  * of s workgroups lat(s) = LAT_A + LAT_B / s microseconds of latency however
- * little it holds (a 4-neighbour grid of 4.1 M vertices run alone: 47, 28,
- * 18, 15, 14 and 14 us per level with teams of 1, 2, 4, 8, 16 and 32
- * workgroups); the rest of t, measured at the old team size s0, is work that
- * divides over the team: t(s) = L lat(s) + (t - L lat(s0)) k s0 / s, where
- * k = (the graph's stored entries) / (the entries of the root's component),
- * at most 64, covers a later root in a larger component.  A bisection finds
- * the shortest makespan M for which every instance fits: an instance with
- * t(1) <= M / 4 shares a one-workgroup team (first-fit decreasing into
- * teams of total <= M / 2, a margin for the estimates), any other gets its
- * own team of the smallest s <= 8 with t(s) <= M (larger teams gain little
+ * little it holds (a 4-neighbour grid of 0.36 M vertices run alone: 12.2, 8.3,
+ * 5.0, 4.5 and 4.5 us per level with teams of 1, 2, 4, 8 and 16 workgroups;
+ * one of 4.1 M: 39.6, 23.3, 13.6, 9.0 and 5.7); the rest of t, measured at the
+ * old team size s0, is work that divides over the team: t(s) = L lat(s) + (t -
+ * L lat(s0)) k s0 / s, where k = (the graph's stored entries) / (the entries of
+ * the root's component), at most 64, covers a later root in a larger component.
+ * A bisection finds the shortest makespan M for which every instance fits: an
+ * instance with t(1) <= M / 4 shares a one-workgroup team (first-fit decreasing
+ * into teams of total <= M / 2, a margin for the estimates), any other gets its
+ * own team of the smallest s <= 16 with t(s) <= M (larger teams gain little
  * per level and poll their barrier harder), never smaller than the own team
  * it had in the share split, and the teams must fit the workgroups.  Workgroups left over go one at a time to the own team whose
  * instance would still take longest.  Other roots on the same graphs take
@@ -141,7 +141,8 @@ int albba_batch_create(albba_ctx *ctx, albba_graph *const *graphs, int32_t count
     }
     b->items = (albd_batch_item *)b->stage;
     memset(b->stage, 0, b->stage_bytes);
-    b->ctl = (unsigned long long *)bdalloc(b, sizeof(unsigned long long) * CTL_WORDS * (size_t)count, &rc);
+    /* the control blocks, then the barrier slots: zeroed together */
+    b->ctl = (unsigned long long *)bdalloc(b, sizeof(unsigned long long) * (CTL_WORDS + ALBD_BATCH_SLOTS) * (size_t)count, &rc);
     for (int32_t i = 0; i < count && !rc; ++i) {
         albba_graph *G = graphs[i];
         b->graphs[i] = G;
@@ -150,12 +151,13 @@ int albba_batch_create(albba_ctx *ctx, albba_graph *const *graphs, int32_t count
         it->g = G->g;
         it->visited = (uint64_t *)bdalloc(b, 8 * nw, &rc);
         for (int k = 0; k < 3; ++k) it->bm[k] = (uint64_t *)bdalloc(b, 8 * nw, &rc);
-        it->found = (int32_t *)bdalloc(b, 4 * np, &rc);
+        it->found = (int32_t *)bdalloc(b, 4 * ALBD_BATCH_FOUND(np), &rc);
         it->key = (unsigned long long *)bdalloc(b, 8 * np, &rc);
         it->level = (int32_t *)bdalloc(b, 4 * n, &rc);
         it->parent = (int32_t *)bdalloc(b, 4 * n, &rc);
         if (!rc) rc = albd_fill_u64(ctx->d, it->key, ~0ull, np);
         it->ctl = b->ctl + (size_t)i * CTL_WORDS;
+        it->slot = b->ctl + (size_t)count * CTL_WORDS + (size_t)i * ALBD_BATCH_SLOTS;
         it->mapping = ALBD_MAP_LANE_ROW;
     }
     if (!rc) rc = albd_sync(ctx->d);
@@ -193,7 +195,7 @@ static int32_t split_teams(albba_batch *b, int32_t W, int32_t *team_first, int32
     for (int32_t i = 0; i < N; ++i) {
         order[i] = i;
         double s = (double)W * inst_cost(b->graphs[i]) / total;
-        share[i] = s >= 64 ? 64 : (int32_t)s;
+        share[i] = s >= ALBD_BATCH_TEAM_MAX ? ALBD_BATCH_TEAM_MAX : (int32_t)s;
     }
     for (int32_t i = 1; i < N; ++i) { /* insertion sort by cost, descending */
         int32_t x = order[i], j = i - 1;
@@ -250,9 +252,9 @@ static int32_t split_teams(albba_batch *b, int32_t W, int32_t *team_first, int32
 }
 
 /* per-level latency of a team of s workgroups, microseconds */
-#define LAT_A 12.0
-#define LAT_B 35.0
-#define TEAM_MAX 8
+#define LAT_A 4.0
+#define LAT_B 8.0
+#define TEAM_MAX 16
 /* Other roots take other level counts and the estimates come from one run
  * under its own contention: only instances estimated at most SHARE_FRAC of
  * the makespan share workgroups, in teams filled to BIN_FRAC of it. */
@@ -494,7 +496,7 @@ static int batch_run(albba_batch *b, const int32_t *roots, const albba_bfs_opts 
     float ms = 0;
     /* descriptors and tables in one copy from the pinned staging buffer */
     (void)((rc = albd_h2d(d, dev, b->stage, bytes)) ||
-           (rc = albd_fill_u64(d, b->ctl, 0, (size_t)N * CTL_WORDS)) || (rc = albd_event_record(d, 4)) ||
+           (rc = albd_fill_u64(d, b->ctl, 0, (size_t)N * (CTL_WORDS + ALBD_BATCH_SLOTS))) || (rc = albd_event_record(d, 4)) ||
            (rc = albd_batch_launch(d, &a, used)) || (rc = albd_event_record(d, 5)) ||
            (rc = albd_event_elapsed(d, 4, 5, &ms)) ||
            (rc = albd_d2h(d, b->hctl, b->ctl, sizeof(unsigned long long) * (size_t)N * CTL_WORDS)));
