@@ -348,6 +348,37 @@ ALBD_HIDDEN albd_counters *albd_mail_next(albd_ctx *c, unsigned int *seq);
 ALBD_HIDDEN int albd_mail_wait(albd_ctx *c, const albd_state *st, unsigned int seq);
 ALBD_HIDDEN void albd_mail_stats(const albd_ctx *c, unsigned long *hits, unsigned long *misses);
 
+/* ---- a small graph's BFS in one workgroup (one_group.hip) ---- */
+#define ALBD_ONE_NPOS 8192
+#define ALBD_ONE_NNZ (1 << 18)
+typedef struct albd_one_args {
+    const float *params;  /* the learned policy's MLP, or NULL (heuristic)      */
+    int32_t root;         /* vertex id                                          */
+    int32_t valid_mask;   /* bit c set: choice c may run                        */
+    int64_t edge_cap, vertex_cap; /* of a run of small push levels (edge_cap 0:
+                             none)                                              */
+    int32_t slow_levels;  /* small levels that did not double before a run      */
+} albd_one_args;
+/* one level of the log; features only where run <= 1 */
+typedef struct albd_one_level {
+    int32_t frontier, choice;
+    int32_t entries;      /* push: frontier edges; pull: entries looked at      */
+    int32_t words;        /* push: queue of the next level; pull: words with an
+                             unvisited row                                      */
+    int32_t col_bypassed; /* column bypass: entries of empty frontier words     */
+    int32_t run;          /* number in a run of small push levels, from 1; or 0 */
+    float features[12];
+} albd_one_level;
+/* whether the graph's BFS fits one workgroup */
+ALBD_HIDDEN int albd_one_fits(const albd_graph *g);
+/* the context's pinned log of ALBD_ONE_NPOS levels, allocated at the first use */
+ALBD_HIDDEN int albd_one_log(albd_ctx *c, const albd_one_level **host, albd_one_level **dev);
+/* The whole BFS and its results (st->level, st->parent), asynchronous;
+ * albd_mail_wait(seq) completes it: reached, reached_edges and the number of
+ * levels (persist_levels) in the counters, the levels in *log. */
+ALBD_HIDDEN int albd_bfs_one(albd_ctx *c, const albd_graph *g, const albd_state *st, const albd_one_args *a,
+                             const albd_one_level **log, unsigned int *seq);
+
 /* ---- batched BFS (batch.hip) ---- */
 /* most workgroups of a team */
 #define ALBD_BATCH_TEAM_MAX 64

@@ -38,6 +38,7 @@ struct albd_ctx {
     albd_counters *dmail; // its device address
     unsigned int mail_seq;
     unsigned long mail_hits, mail_misses; // posts seen / waits that fell back
+    albd_one_level *one_log, *done_log;   // pinned level log and its device address, null until first used
     void *stage[ALBD_STAGES];             // pinned, null until first used
     hipEvent_t stage_ev[ALBD_STAGES];
     std::mutex stage_lock;
@@ -101,6 +102,7 @@ void albd_ctx_destroy(albd_ctx *c)
     (void)hipStreamDestroy(c->stream);
     (void)hipHostFree(c->hctr);
     (void)hipHostFree(c->mail);
+    if (c->one_log) (void)hipHostFree(c->one_log);
     drop_kept(c);
     for (int i = 0; i < ALBD_STAGES && c->stage[0]; ++i) {
         (void)hipHostFree(c->stage[i]);
@@ -266,6 +268,24 @@ int albd_mail_wait(albd_ctx *c, const albd_state *st, unsigned int seq)
             return albd_read_counters(c, st);
         }
     }
+}
+
+int albd_one_log(albd_ctx *c, const albd_one_level **host, albd_one_level **dev)
+{
+    if (!c->one_log) {
+        void *p = nullptr, *d = nullptr;
+        HIPCHK(hipHostMalloc(&p, sizeof(albd_one_level) * ALBD_ONE_NPOS, hipHostMallocMapped | hipHostMallocCoherent));
+        const hipError_t e = hipHostGetDevicePointer(&d, p, 0);
+        if (e != hipSuccess) {
+            (void)hipHostFree(p);
+            return albd_set_error(e, "level log", __FILE__, __LINE__);
+        }
+        c->one_log = (albd_one_level *)p;
+        c->done_log = (albd_one_level *)d;
+    }
+    *host = c->one_log;
+    *dev = c->done_log;
+    return 0;
 }
 
 void albd_mail_stats(const albd_ctx *c, unsigned long *hits, unsigned long *misses)

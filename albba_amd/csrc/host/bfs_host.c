@@ -1014,6 +1014,57 @@ static int script_at(const albba_graph *G, const albba_bfs_opts *o, int32_t leve
  * in the small-frontier kernel */
 #define SLOW_LEVELS 4
 
+/* The BFS of a small graph in one launch of one workgroup: the choices and
+ * statistics of the level loop below, without its 4 launches a level (RMAT
+ * s10: 146 -> 25 us).  bfs_run's policies that decide a level by itself
+ * (heuristic, learned) take it where the graph fits (albd_one_fits), unless
+ * levels are to be timed. */
+static int bfs_one(albba_graph *G, int32_t root, const albba_bfs_opts *opts, int valid_mask,
+                   int64_t push_vertex_cap, int64_t queue_max, albba_bfs_stats *stats, bfs_events ev)
+{
+    albd_ctx *d = G->ctx->d;
+    const albd_one_args a = {
+        opts->switch_policy == ALBBA_SWITCH_LEARNED ? albba_selector_dparams(opts->selector) : NULL,
+        root, valid_mask, opts->small_frontier_edges, push_vertex_cap, SLOW_LEVELS};
+    const albd_one_level *log = NULL;
+    unsigned int seq = 0;
+    float ms = 0;
+    int rc;
+    if ((rc = albd_event_record(d, ev.start)) || (rc = albd_bfs_one(d, &G->g, &G->st, &a, &log, &seq)) ||
+        (rc = albd_event_record(d, ev.end)) || (rc = albd_mail_wait(d, &G->st, seq)) ||
+        (!ev.defer && (rc = albd_event_elapsed(d, ev.start, ev.end, &ms))))
+        return albba_fail(rc, "bfs: %s", albd_error());
+    if (!stats) return ALBBA_OK;
+    const albd_counters *hc = albd_host_counters(d);
+    const int32_t levels = hc->persist_levels;
+    for (int32_t l = 0; l < levels && l < stats->capacity; ++l) {
+        const albd_one_level *e = log + l;
+        const int push = e->choice == ALBBA_CHOICE_PUSH;
+        if (stats->frontier) stats->frontier[l] = e->frontier;
+        if (stats->choice) stats->choice[l] = e->choice;
+        if (stats->features) {
+            float *f = stats->features + (size_t)l * ALBBA_NUM_FEATURES;
+            if (e->run <= 1) memcpy(f, e->features, sizeof e->features);
+            else memset(f, 0, sizeof e->features);
+        }
+        if (stats->choice_ms) memset(stats->choice_ms + (size_t)l * ALBBA_NUM_CHOICES, 0,
+                                     sizeof(float) * ALBBA_NUM_CHOICES);
+        if (stats->level_ms) stats->level_ms[l] = 0;
+        if (stats->kernel_ms) stats->kernel_ms[l] = 0;
+        if (stats->entries) stats->entries[l] = e->entries;
+        if (stats->words)
+            stats->words[l] = e->run ? e->frontier : (!push || e->entries <= queue_max ? e->words : 0);
+        if (stats->bypassed) stats->bypassed[l] = push ? 0 : (int64_t)G->g.nwords - e->words;
+        if (stats->col_bypassed) stats->col_bypassed[l] = e->col_bypassed;
+        if (stats->swept) stats->swept[l] = -1;
+    }
+    stats->num_levels = levels;
+    stats->reached = (int64_t)hc->reached;
+    stats->edges_in_component = (int64_t)hc->reached_edges;
+    if (!ev.defer) stats->bfs_ms = ms;
+    return ALBBA_OK;
+}
+
 static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs_opts *opts_in,
                    albba_bfs_stats *stats, bfs_events ev)
 {
@@ -1048,6 +1099,9 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
     const float qratio = policy == ALBBA_SWITCH_LEARNED ? albba_selector_queue_ratio(opts.selector) : 0.0f;
     const int64_t learned_qmax = qratio > 0.0f ? (int64_t)ceil((double)qratio * (double)G->n) : push_vertex_cap;
     const int64_t queue_max_policy = policy == ALBBA_SWITCH_LEARNED ? learned_qmax : push_vertex_cap;
+    if (!opts.time_levels && (policy == ALBBA_SWITCH_HEURISTIC || policy == ALBBA_SWITCH_LEARNED) &&
+        albd_one_fits(&G->g))
+        return bfs_one(G, root, &opts, valid_mask, push_vertex_cap, queue_max_policy, stats, ev);
     /* a scripted level lists the queue exactly when the script pushes next
      * (-1: never; past the script the heuristic's rule) */
 #define QUEUE_MAX(L)                                                                                   \
