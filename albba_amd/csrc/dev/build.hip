@@ -43,31 +43,6 @@ int grid_for(int64_t items, int per_block)
     return (int)b;
 }
 
-// Walk the entries of the 64 rows held by the lanes of one wave (row i of
-// the group: `start`, `len` in lane i), 64 entries per step, lanes taking
-// consecutive entries: f(i, j, active) for entry j of row i.  Every lane
-// calls f on every step (the shuffles inside need the whole wave); `active`
-// says whether its (i, j) is an entry.
-template <class F>
-__device__ __forceinline__ void wave_rows_foreach(int32_t len, F &&f)
-{
-    const int lane = lane_id();
-    unsigned long long tot;
-    const unsigned long long ex = wave_exclusive_scan<unsigned long long>((unsigned long long)len, &tot);
-    for (unsigned long long e0 = 0; e0 < tot; e0 += 64) {
-        const unsigned long long e = e0 + (unsigned long long)lane;
-        // the row of entry e: the last lane whose exclusive offset is <= e
-        int lo = 0;
-#pragma unroll
-        for (int step = 32; step > 0; step >>= 1) {
-            const unsigned long long x = __shfl(ex, lo + step, 64);
-            if (x <= e) lo += step;
-        }
-        const unsigned long long base = __shfl(ex, lo, 64);
-        f(lo, (int64_t)(e - base), e < tot);
-    }
-}
-
 // 1. lengths, longest row, checks.  Rows are in ascending order exactly
 // when every descent col[k-1] > col[k] sits at the start of a row: one flat
 // pass counts all descents (and checks the column range), one pass over the
@@ -536,32 +511,82 @@ __global__ __launch_bounds__(kBB) void k_widen_u32(const unsigned int *in, int64
         out[i] = in[i];
 }
 
-// 7. a transpose by one sort (the directed push CSR over positions, and
-// W = A^T of a loaded file): entry (r, c) becomes the key c << shift | r, a
-// radix sort orders the keys by column and, within a column, by row, and one
-// pass splits them into the transpose's columns and row pointers.  Atomic
-// placement into per-column cursors serialised on the hubs' columns (RMAT
-// s22: 20 ms for the fill of one directed build) and still needed a sort of
-// every row.
-__global__ __launch_bounds__(kBB) void k_transpose_keys(const int64_t *rp, const int32_t *col, int32_t n,
-                                                        int shift, unsigned long long *keys)
+// the row of entry e: the largest r with rp[r] <= e (one wave, 64 probes per
+// round)
+__device__ __forceinline__ int32_t row_of_entry(const int64_t *rp, int32_t n, int64_t e)
 {
     const int lane = lane_id();
-    const int64_t wave = ((int64_t)blockIdx.x * kBB + threadIdx.x) >> 6;
-    const int64_t nwaves = ((int64_t)gridDim.x * kBB) >> 6;
-    for (int64_t p0 = wave * 64; p0 < n; p0 += nwaves * 64) {
-        const int64_t p = p0 + lane;
-        int64_t start = 0;
-        int32_t l = 0;
-        if (p < n) {
-            start = rp[p];
-            l = (int32_t)(rp[p + 1] - start);
-        }
-        wave_rows_foreach(l, [&](int i, int64_t j, bool act) {
-            const int64_t s = __shfl(start, i, 64);
-            if (act)
-                keys[s + j] = ((unsigned long long)(uint32_t)col[s + j] << shift) | (unsigned long long)(p0 + i);
-        });
+    int64_t r = 0;
+    for (int64_t hi = n; hi - r > 1;) { // rp[r] <= e < rp[hi]
+        const int64_t step = (hi - r + 63) / 64, at = r + lane * step;
+        const int c = __popcll(__ballot(at < hi && rp[at] <= e)); // lane 0's holds
+        r += (c - 1) * step;
+        if (r + step < hi) hi = r + step;
+    }
+    return (int32_t)r;
+}
+
+// 7. a transpose by one sort (the directed push CSR over positions, and
+// W = A^T of a loaded file): entry (r, c) becomes the key c << shift | r, a
+// stable radix sort orders the keys by column alone, since they are listed row
+// by row, and one pass splits them into the transpose's columns and row
+// pointers.  Atomic placement into per-column cursors serialised on the hubs'
+// columns (RMAT s22: 20 ms for the fill of one directed build) and still needed
+// a sort of every row.
+//
+// The keys are listed by blocks of kKeyChunk entries, whatever rows they belong
+// to: waves that took 64 rows each waited for the one with the hubs (in
+// position order they are neighbours; RMAT s20: 2 106 us).  A row's number goes
+// to the place of its first entry in the chunk, and a running maximum carries
+// it over the row's entries (empty rows share that place with a later row).
+constexpr int kKeyChunk = kBB * 8;
+
+__global__ __launch_bounds__(kBB) void k_transpose_keys(const int64_t *rp, const int32_t *col, int32_t n,
+                                                        int64_t nnz, int shift, unsigned long long *keys)
+{
+    constexpr int kPer = kKeyChunk / kBB;
+    __shared__ int32_t s_row[kKeyChunk];
+    __shared__ int32_t s_range[2], s_top[kBB / 64];
+    const int tid = threadIdx.x, lane = lane_id(), wid = tid >> 6;
+    const int64_t e0 = (int64_t)blockIdx.x * kKeyChunk;
+    const int cnt = (int)(nnz - e0 < kKeyChunk ? nnz - e0 : kKeyChunk);
+    if (wid < 2) {
+        const int32_t r = row_of_entry(rp, n, wid == 0 ? e0 : e0 + cnt - 1);
+        if (lane == 0) s_range[wid] = r;
+    }
+    for (int i = tid; i < kKeyChunk; i += kBB) s_row[i] = 0;
+    __syncthreads();
+    const int32_t first = s_range[0], last = s_range[1];
+    for (int64_t r = (int64_t)first + 1 + tid; r <= last; r += kBB)
+        atomicMax(&s_row[rp[r] - e0], (int32_t)(r - first));
+    __syncthreads();
+    int32_t row[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        row[k] = s_row[tid * kPer + k];
+        if (k > 0 && row[k - 1] > row[k]) row[k] = row[k - 1];
+    }
+    // the maximum over the threads before this one
+    int32_t m = row[kPer - 1];
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int32_t y = __shfl_up(m, d, 64);
+        if (lane >= d && y > m) m = y;
+    }
+    if (lane == 63) s_top[wid] = m;
+    m = __shfl_up(m, 1, 64);
+    if (lane == 0) m = 0;
+    __syncthreads();
+    for (int i = 0; i < wid; ++i)
+        if (s_top[i] > m) m = s_top[i];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) s_row[tid * kPer + k] = first + (row[k] > m ? row[k] : m);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int i = k * kBB + tid;
+        if (i < cnt)
+            keys[e0 + i] = ((unsigned long long)(uint32_t)col[e0 + i] << shift) | (unsigned long long)(uint32_t)s_row[i];
     }
 }
 
@@ -659,18 +684,23 @@ int transpose_by_sort(albd_ctx *c, Temps &T, const int64_t *rp, const int32_t *c
         return 0;
     }
     const int shift = bits_for((uint64_t)(nrows > 1 ? nrows - 1 : 0));
-    int end_bit = shift + bits_for((uint64_t)(ncols > 1 ? ncols - 1 : 0));
-    if (end_bit < 1) end_bit = 1;
+    const int end_bit = shift + bits_for((uint64_t)(ncols > 1 ? ncols - 1 : 0));
     unsigned long long *keys = nullptr, *sorted = nullptr;
     int rc;
     if ((rc = T.get(nnz, &keys)) || (rc = T.get(nnz, &sorted))) return rc;
-    hipLaunchKernelGGL(k_transpose_keys, dim3(grid_for(nrows, kBB)), dim3(kBB), 0, s, rp, col, nrows, shift, keys);
+    hipLaunchKernelGGL(k_transpose_keys, dim3((unsigned int)((nnz + kKeyChunk - 1) / kKeyChunk)), dim3(kBB), 0, s, rp,
+                       col, nrows, nnz, shift, keys);
     HIPCHK(hipGetLastError());
-    size_t bytes = 0;
-    ROCCHK(rocprim::radix_sort_keys(nullptr, bytes, keys, sorted, (size_t)nnz, 0, end_bit, s));
-    unsigned char *tmp = nullptr;
-    if ((rc = T.get(bytes ? bytes : 1, &tmp))) return rc;
-    ROCCHK(rocprim::radix_sort_keys(tmp, bytes, keys, sorted, (size_t)nnz, 0, end_bit, s));
+    if (end_bit > shift) {
+        // by column only (RMAT s20: 3 passes for 6): the sort is stable
+        size_t bytes = 0;
+        ROCCHK(rocprim::radix_sort_keys(nullptr, bytes, keys, sorted, (size_t)nnz, shift, end_bit, s));
+        unsigned char *tmp = nullptr;
+        if ((rc = T.get(bytes ? bytes : 1, &tmp))) return rc;
+        ROCCHK(rocprim::radix_sort_keys(tmp, bytes, keys, sorted, (size_t)nnz, shift, end_bit, s));
+    } else {
+        sorted = keys; // one column
+    }
     hipLaunchKernelGGL(k_transpose_split, dim3(grid_for(nnz, kBB)), dim3(kBB), 0, s, sorted, nnz, shift, ncols, tp,
                        tc);
     HIPCHK(hipGetLastError());
