@@ -86,14 +86,18 @@ static int to_device(albd_ctx *d, void *dst, const void *src, int fd, int64_t of
 {
     const size_t piece = piece_bytes(bytes);
     const int64_t np = (int64_t)((bytes + piece - 1) / piece);
-    int rc = 0, bad = 0;
+    /* Every thread has to leave the loop at the same barrier: it leaves on
+     * what only the master writes, and not again before each thread has passed
+     * another barrier.  (On `bad`, which a thread may set as soon as it reads,
+     * a slower one could leave while the others waited for it: a hang.) */
+    int rc = 0, bad = 0, waited = 0, stop = 0;
 #pragma omp parallel num_threads(copy_threads())
     for (int64_t i = 0; i < np; ++i) {
         const int k = (int)(i % ALBD_STAGES);
 #pragma omp master
-        if (i >= ALBD_STAGES) rc = rc ? rc : albd_stage_wait(d, k);
+        if (i >= ALBD_STAGES) waited = albd_stage_wait(d, k);
 #pragma omp barrier
-        if (rc || bad) break;
+        if (waited) break;
         size_t lo, hi;
         part_of(PIECE_LEN(i), omp_get_thread_num(), omp_get_num_threads(), &lo, &hi);
         if (fd < 0) {
@@ -112,14 +116,18 @@ static int to_device(albd_ctx *d, void *dst, const void *src, int fd, int64_t of
         }
 #pragma omp barrier
 #pragma omp master
-        if (!bad)
-            rc = albd_h2d_async(d, (char *)dst + (size_t)i * piece, stage[k], PIECE_LEN(i)) || albd_stage_mark(d, k);
+        {
+            if (!bad)
+                rc = albd_h2d_async(d, (char *)dst + (size_t)i * piece, stage[k], PIECE_LEN(i)) ||
+                     albd_stage_mark(d, k);
+            stop = rc || bad;
+        }
 #pragma omp barrier
-        if (rc || bad) break;
+        if (stop) break;
     }
     const int rs = albd_sync(d);
     if (bad) return ALBBA_EIO;
-    return rc ? ALBBA_EHIP : rs;
+    return rc || waited ? ALBBA_EHIP : rs;
 }
 
 int albba_h2d(albd_ctx *d, void *dst, const void *src, size_t bytes)
