@@ -36,7 +36,9 @@ typedef struct albd_slot {
 } albd_slot;
 
 typedef struct albd_counters {
-    unsigned long long queue_len;    /* current frontier queue length         */
+    /* entries in the low half; in the high half their edges, where the
+     * queue's degree prefix is there too                                     */
+    unsigned long long queue_len;    /* current frontier queue                */
     unsigned long long qnext_len;    /* queue being built                     */
     unsigned long long active_len;   /* length of the current unvisited-word list */
     unsigned long long push_edges;   /* sum of degrees over the queue         */
@@ -293,24 +295,27 @@ ALBD_HIDDEN int albd_pull(albd_ctx *c, const albd_graph *g, const albd_state *st
                           int32_t level, int64_t items_bound);
 ALBD_HIDDEN int albd_cb_supported(const albd_graph *g);
 
-/* the push kernels of one level (scan, expansion, finalize), queued before
- * the level's direction is known: they return at once unless the select
- * kernel chose the push (spec = 1: its learned choice, 0: the heuristic's)
- * for a nonempty frontier of at most ALBD_SPEC_PUSH_MAX vertices, the bound
- * below which albd_push_scan takes its one-block scan.  The queue must hold
- * the frontier (the last level pushed); the finalize lists the next queue as
- * albd_push_finalize does with build_max. */
+/* the push kernels of one level (expansion, finalize), queued before the
+ * level's direction is known: they return at once unless the select kernel
+ * chose the push (spec = 1: its learned choice, 0: the heuristic's) for a
+ * nonempty frontier.  The queue must hold the frontier (the last level
+ * pushed); scan: it has no degree prefix, which is then made first, for at most
+ * ALBD_SPEC_PUSH_MAX vertices (the bound below which albd_push_scan takes its
+ * one-block scan; for more, the kernels return at once).  The finalize lists
+ * the next queue as albd_push_finalize does with build_max. */
 #define ALBD_SPEC_PUSH_MAX 8192
 ALBD_HIDDEN int albd_push_spec(albd_ctx *c, const albd_graph *g, const albd_state *st, int32_t level, int spec,
-                               int64_t build_max);
-/* push: queue from the front bitmap (when the last level was a pull) */
+                               int64_t build_max, int scan);
+/* push: queue and its degree prefix from the front bitmap (when the last
+ * level was a pull) */
 ALBD_HIDDEN int albd_front_to_queue(albd_ctx *c, const albd_graph *g, const albd_state *st);
-/* push: prefix of degrees over the queue (qlen known on the host) */
+/* push: prefix of degrees over a queue that has none (after the
+ * small-frontier kernel, or a trial run); qlen known on the host */
 ALBD_HIDDEN int albd_push_scan(albd_ctx *c, const albd_graph *g, const albd_state *st,
                                int64_t qlen);
 ALBD_HIDDEN int albd_push_expand(albd_ctx *c, const albd_graph *g, const albd_state *st);
 /* push: merge next into visited, write level/parent from pmin, and list
- * queue_next (ctr->qnext_len) while the level's frontier edges
+ * queue_next (ctr->qnext_len) and its degree prefix while the level's frontier edges
  * (ctr->frontier_edges) are at most build_max; else it stays empty */
 ALBD_HIDDEN int albd_push_finalize(albd_ctx *c, const albd_graph *g, const albd_state *st,
                                    int32_t level, int64_t build_max);

@@ -360,17 +360,15 @@ __global__ __launch_bounds__(pull_block<VAR>()) void k_pull(PullArgs a)
 // wave's count (lane 0's value counts); returns the wave's first slot.  Same
 // address device atomics serialise, so the word passes take one per block
 // step rather than one per wave.
-template <int NW = kWavesPerBlock>
-__device__ __forceinline__ unsigned long long block_reserve(unsigned long long *counter,
-                                                           unsigned int wave_count,
-                                                           unsigned int *s_cnt,
+template <int NW = kWavesPerBlock, class T = unsigned int>
+__device__ __forceinline__ unsigned long long block_reserve(unsigned long long *counter, T wave_count, T *s_cnt,
                                                            unsigned long long *s_base)
 {
     const int wid = threadIdx.x >> 6;
     if (lane_id() == 0) s_cnt[wid] = wave_count;
     __syncthreads();
     if (threadIdx.x == 0) {
-        unsigned int tot = 0;
+        T tot = 0;
         for (int i = 0; i < NW; ++i) tot += s_cnt[i];
         *s_base = tot ? atomicAdd(counter, (unsigned long long)tot) : 0ull;
     }
@@ -430,10 +428,13 @@ __global__ __launch_bounds__(kBlock) void k_bfs_reset(albd_graph g, albd_state s
         constexpr int kQ = (int)(offsetof(albd_counters, queue_len) / 8);
         unsigned long long *c = reinterpret_cast<unsigned long long *>(st.ctr);
         for (int i = threadIdx.x; i < (int)(sizeof(albd_counters) / 8); i += kBlock)
-            c[i] = i == kQ && deg > 0 ? 1ull : 0ull;
+            c[i] = i == kQ && deg > 0 ? 1ull | (unsigned long long)deg << 32 : 0ull;
         if (threadIdx.x == 0) {
             st.lp[rp] = pack_lp(0, ro);
-            if (deg > 0) st.queue[0] = rp;
+            if (deg > 0) {
+                st.queue[0] = rp;
+                st.prefix[0] = 0;
+            }
         }
     }
 }
@@ -725,24 +726,31 @@ __global__ __launch_bounds__(kBlock) void k_select_prep(albd_graph g, albd_state
     else prep_body<FROM_LIST, SUMMARY>(g, st, ls, blockIdx.x - 1, gridDim.x - 1);
 }
 
-// Words -> queue of positions with out-degree > 0.  FINALIZE (after a push):
-// the words are st.next; merge them into visited, write level/parent from
-// pmin and count the new frontier; the queue only while the level's
-// frontier edges (the select kernel's count) are at most build_max: a larger
-// push likely leads to a pull, which needs none, and a push after it lists
-// the bitmap.  Otherwise the words are st.front.
+// Words -> queue of positions with out-degree > 0, and the queue's degree
+// prefix.  FINALIZE (after a push): the words are st.next; merge them into
+// visited, write level/parent from pmin and count the new frontier; the queue
+// only while the level's frontier edges (the select kernel's count) are at most
+// build_max: a larger push likely leads to a pull, which needs none, and a push
+// after it lists the bitmap.  Otherwise the words are st.front.
 //
-// 1024-thread blocks: the list reservation is one same-address atomic per
-// block, and those serialise (256-thread blocks made the reservations the
-// larger part of a big push level's finalize).
+// A block reserves its entries and their edges by one atomic on a packed count
+// (edges in the high half), so that the queue's order and the prefix's agree
+// whichever block comes first: the push that follows needs no scan of its queue
+// (one launch of about 9 us a level, three past 8 192 vertices).
+//
+// 1024-thread blocks: the reservation is one same-address atomic per block, and
+// those serialise (256-thread blocks made the reservations the larger part of a
+// big push level's finalize).  A wave takes wpw words, one after the other: 64
+// where the words fill the chip, fewer on smaller graphs (RMAT s16, 1 024 words,
+// 64 a wave: one block, 21 us).
 constexpr int kQBlock = 1024;
 constexpr int kQWaves = kQBlock / 64;
 
 template <bool FINALIZE>
-__global__ __launch_bounds__(kQBlock) void k_words_to_queue(albd_graph g, albd_state st,
-                                                            int32_t level, Spec sp, long long build_max)
+__global__ __launch_bounds__(kQBlock) void k_words_to_queue(albd_graph g, albd_state st, int32_t level, Spec sp,
+                                                            long long build_max, int wpw)
 {
-    __shared__ unsigned int s_cnt[kQWaves];
+    __shared__ unsigned long long s_cnt[kQWaves];
     __shared__ unsigned long long s_base;
     if (!spec_go(st.ctr, sp)) return;
     const bool build = !FINALIZE || (long long)st.ctr->frontier_edges <= build_max;
@@ -750,52 +758,64 @@ __global__ __launch_bounds__(kQBlock) void k_words_to_queue(albd_graph g, albd_s
     const uint64_t *words = FINALIZE ? st.next : st.front;
     int32_t *q = FINALIZE ? st.queue_next : st.queue;
     unsigned long long *qlen = FINALIZE ? &st.ctr->qnext_len : &st.ctr->queue_len;
-    const int64_t ngroups = ((int64_t)g.nwords + 63) >> 6;
+    const int64_t ngroups = ((int64_t)g.nwords + wpw - 1) / wpw;
     unsigned long long cnt = 0, nzw = 0, edges = 0;
-    // block-uniform steps of one 64-word group per wave
+    // block-uniform steps of one group of wpw words per wave
     for (int64_t gb = (int64_t)blockIdx.x * kQWaves; gb < ngroups; gb += (int64_t)gridDim.x * kQWaves) {
-        const int64_t grp = gb + wid;
-        const int64_t w = grp * 64 + lane;
-        const uint64_t word = (grp < ngroups && w < g.nwords) ? words[w] : 0ull;
+        const int64_t w0 = (gb + wid) * wpw, w = w0 + lane;
+        const uint64_t word = (lane < wpw && w < g.nwords) ? words[w] : 0ull;
         if (FINALIZE && word) {
             st.visited[w] |= word; // only this lane touches word w here
             cnt += __popcll(word);
             nzw += 1;
         }
         const uint64_t nzmask = __ballot(word != 0);
-        uint64_t keepw = 0; // lane k holds the keep mask of word grp*64+k
+        uint64_t keepw = 0;    // lane k holds the keep mask of word w0 + k
+        uint32_t kept_edges = 0; // and the edges of those it keeps
         uint64_t mm = nzmask;
         while (mm) {
             const int k = __ffsll((unsigned long long)mm) - 1;
             mm &= mm - 1;
             const uint64_t bits = __shfl(word, k, 64);
-            const int64_t pp = (grp * 64 + k) * 64 + lane;
-            bool keep = false;
+            const int64_t pp = (w0 + k) * 64 + lane;
+            uint32_t d = 0;
             if ((bits >> lane) & 1ull) {
-                const int64_t d = g.push_ptr[pp + 1] - g.push_ptr[pp];
-                keep = d > 0;
+                d = (uint32_t)(g.push_ptr[pp + 1] - g.push_ptr[pp]);
                 if (FINALIZE) {
                     st.lp[pp] = pack_lp(level + 1, (int32_t)st.pmin[pp]);
                     st.pmin[pp] = 0xFFFFFFFFu;
-                    edges += (unsigned long long)d;
+                    edges += d;
                 }
             }
-            const uint64_t km = __ballot(keep);
-            if (lane == k) keepw = km;
+            if (!build) continue; // kernel-uniform
+            const uint64_t km = __ballot(d > 0);
+            const uint32_t ke = wave_sum(d);
+            if (lane == k) {
+                keepw = km;
+                kept_edges = ke;
+            }
         }
-        if (!build) continue; // kernel-uniform
+        if (!build) continue;
         unsigned long long total;
-        const unsigned long long excl =
-            wave_exclusive_scan<unsigned long long>((unsigned long long)__popcll(keepw), &total);
-        const unsigned long long base = block_reserve<kQWaves>(qlen, (unsigned int)total, s_cnt, &s_base);
+        const unsigned long long excl = wave_exclusive_scan<unsigned long long>(
+            (unsigned long long)kept_edges << 32 | (unsigned long long)__popcll(keepw), &total);
+        const unsigned long long base = block_reserve<kQWaves>(qlen, total, s_cnt, &s_base);
         uint64_t km = __ballot(keepw != 0);
         while (km) {
             const int k = __ffsll((unsigned long long)km) - 1;
             km &= km - 1;
             const uint64_t kw = __shfl(keepw, k, 64);
-            const unsigned long long off = __shfl(excl, k, 64);
-            if ((kw >> lane) & 1ull)
-                q[base + off + __popcll(kw & lanemask_lt(lane))] = (int32_t)((grp * 64 + k) * 64 + lane);
+            const unsigned long long off = base + __shfl(excl, k, 64);
+            const int64_t pp = (w0 + k) * 64 + lane;
+            const bool mine = (kw >> lane) & 1ull;
+            uint32_t tot;
+            const uint32_t ex = wave_exclusive_scan<uint32_t>(
+                mine ? (uint32_t)(g.push_ptr[pp + 1] - g.push_ptr[pp]) : 0u, &tot);
+            if (mine) {
+                const uint32_t at = (uint32_t)off + (uint32_t)__popcll(kw & lanemask_lt(lane));
+                q[at] = (int32_t)pp;
+                st.prefix[at] = (int64_t)(off >> 32) + ex;
+            }
         }
     }
     if (FINALIZE) {
@@ -910,6 +930,12 @@ __global__ __launch_bounds__(kBlock) void k_to_vertex_order(albd_graph g, albd_s
 // ---------------------------------------------------------------------------
 // push: degree prefix over the queue
 
+// the frontier queue's entries (their edges are in the high half)
+__device__ __forceinline__ int64_t queue_count(const albd_counters *ctr)
+{
+    return (int64_t)(ctr->queue_len & 0xffffffffull);
+}
+
 __device__ __forceinline__ int64_t out_degree(const albd_graph &g, int32_t u)
 {
     return g.push_ptr[u + 1] - g.push_ptr[u];
@@ -938,7 +964,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_small(albd_graph g, albd_state 
 {
     __shared__ int64_t lds[8];
     if (!spec_go(st.ctr, sp)) return;
-    const int64_t qlen = (int64_t)st.ctr->queue_len;
+    const int64_t qlen = queue_count(st.ctr);
     int64_t carry = 0;
     for (int64_t base = 0; base < qlen; base += kBlock) {
         const int64_t i = base + threadIdx.x;
@@ -948,16 +974,13 @@ __global__ __launch_bounds__(kBlock) void k_scan_small(albd_graph g, albd_state 
         if (i < qlen) st.prefix[i] = carry + ex;
         carry += tot;
     }
-    if (threadIdx.x == 0) {
-        st.prefix[qlen] = carry;
-        st.ctr->push_edges = carry;
-    }
+    if (threadIdx.x == 0) st.ctr->queue_len = (unsigned long long)carry << 32 | (unsigned long long)qlen;
 }
 
 __global__ __launch_bounds__(kBlock) void k_scan_p1(albd_graph g, albd_state st)
 {
     __shared__ int64_t lds[8];
-    const int64_t qlen = (int64_t)st.ctr->queue_len;
+    const int64_t qlen = queue_count(st.ctr);
     const int64_t cs = (qlen + gridDim.x - 1) / gridDim.x;
     const int64_t lo = cs * blockIdx.x, hi = lo + cs < qlen ? lo + cs : qlen;
     int64_t sum = 0;
@@ -974,7 +997,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_p1(albd_graph g, albd_state st)
 __global__ __launch_bounds__(kBlock) void k_scan_p2(albd_state st, int32_t nblocks)
 {
     __shared__ int64_t lds[8];
-    const int64_t qlen = (int64_t)st.ctr->queue_len;
+    const int64_t qlen = queue_count(st.ctr);
     int64_t carry = 0;
     for (int base = 0; base < nblocks; base += kBlock) {
         const int i = base + threadIdx.x;
@@ -986,15 +1009,14 @@ __global__ __launch_bounds__(kBlock) void k_scan_p2(albd_state st, int32_t nbloc
     }
     if (threadIdx.x == 0) {
         st.block_sums[nblocks] = carry;
-        st.prefix[qlen] = carry;
-        st.ctr->push_edges = carry;
+        st.ctr->queue_len = (unsigned long long)carry << 32 | (unsigned long long)qlen;
     }
 }
 
 __global__ __launch_bounds__(kBlock) void k_scan_p3(albd_state st)
 {
     __shared__ int64_t lds[8];
-    const int64_t qlen = (int64_t)st.ctr->queue_len;
+    const int64_t qlen = queue_count(st.ctr);
     const int64_t cs = (qlen + gridDim.x - 1) / gridDim.x;
     const int64_t lo = cs * blockIdx.x, hi = lo + cs < qlen ? lo + cs : qlen;
     int64_t carry = st.block_sums[blockIdx.x];
@@ -1043,9 +1065,9 @@ __global__ __launch_bounds__(kBlock) void k_push_expand(albd_graph g, albd_state
 {
     if (!spec_go(st.ctr, sp)) return;
     const int lane = lane_id();
-    const int64_t qlen = (int64_t)st.ctr->queue_len;
+    const int64_t qlen = queue_count(st.ctr), E = (int64_t)(st.ctr->queue_len >> 32);
+    if (blockIdx.x == 0 && threadIdx.x == 0) st.ctr->push_edges = (unsigned long long)E;
     if (qlen == 0) return;
-    const int64_t E = st.prefix[qlen];
     const int64_t gw = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
     const int64_t nw = ((int64_t)gridDim.x * kBlock) >> 6;
     const int64_t nchunks = (E + 63) >> 6;
@@ -1059,7 +1081,7 @@ __global__ __launch_bounds__(kBlock) void k_push_expand(albd_graph g, albd_state
         const int64_t e = e0 + lane;
         // v0 holds edge e0 and queue entries have degree >= 1, so the chunk's
         // edges belong to vertices v0 .. v0+63
-        const int64_t Pk = (v0 + 1 + lane <= qlen) ? st.prefix[v0 + 1 + lane] : LLONG_MAX;
+        const int64_t Pk = (v0 + 1 + lane < qlen) ? st.prefix[v0 + 1 + lane] : LLONG_MAX;
         const int64_t P0 = st.prefix[v0];
         int t = 0;
 #pragma unroll
@@ -1173,7 +1195,7 @@ __global__ __launch_bounds__(kListBlock) void k_push_small(SmallArgs a)
     list_reset(S);
     __syncthreads();
     if (tid == 0) reserve_found(S, M, 0);
-    int64_t ns = (int64_t)st.ctr->queue_len; // the shared queue's length
+    int64_t ns = queue_count(st.ctr); // the shared queue's length
     int64_t F = 0;                           // found by this workgroup before the level
     PushEdge e[kListPer];
 #pragma unroll
@@ -1295,10 +1317,16 @@ int grid_persistent(albd_ctx *c, int blocks_per_cu)
     return g < 8 ? 8 : g;
 }
 
-// blocks of k_words_to_queue (1024 threads) for `groups` 64-word groups
-int grid_for_qgroups(albd_ctx *c, int64_t groups)
+// words per wave of k_words_to_queue, and its blocks of kQWaves such waves
+int words_per_wave(const albd_graph *g)
 {
-    int64_t blocks = (groups + kQWaves - 1) / kQWaves;
+    return g->nwords >= 1 << 17 ? 64 : (g->nwords >= 1 << 14 ? 16 : 4);
+}
+
+int grid_for_queue(albd_ctx *c, const albd_graph *g)
+{
+    const int64_t per_block = (int64_t)kQWaves * words_per_wave(g);
+    int64_t blocks = ((int64_t)g->nwords + per_block - 1) / per_block;
     int64_t cap = (int64_t)albd_num_cus(c) * 2;
     if (blocks > cap) blocks = cap;
     return blocks < 1 ? 1 : (int)blocks;
@@ -1522,9 +1550,8 @@ int albd_pull_spec(albd_ctx *c, const albd_graph *g, const albd_state *st, int v
 
 int albd_front_to_queue(albd_ctx *c, const albd_graph *g, const albd_state *st)
 {
-    const int grid = grid_for_qgroups(c, ((int64_t)g->nwords + 63) / 64);
-    hipLaunchKernelGGL(k_words_to_queue<false>, dim3(grid), dim3(kQBlock), 0, albd_stream(c), *g, *st, 0, kNoSpec,
-                       LLONG_MAX);
+    hipLaunchKernelGGL(k_words_to_queue<false>, dim3(grid_for_queue(c, g)), dim3(kQBlock), 0, albd_stream(c), *g, *st,
+                       0, kNoSpec, LLONG_MAX, words_per_wave(g));
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -1618,27 +1645,27 @@ int albd_select_read(albd_ctx *c, const albd_graph *g, const albd_state *st,
 
 int albd_push_finalize(albd_ctx *c, const albd_graph *g, const albd_state *st, int32_t level, int64_t build_max)
 {
-    const int grid = grid_for_qgroups(c, ((int64_t)g->nwords + 63) / 64);
-    hipLaunchKernelGGL(k_words_to_queue<true>, dim3(grid), dim3(kQBlock), 0, albd_stream(c), *g, *st, level,
-                       kNoSpec, (long long)build_max);
+    hipLaunchKernelGGL(k_words_to_queue<true>, dim3(grid_for_queue(c, g)), dim3(kQBlock), 0, albd_stream(c), *g, *st,
+                       level, kNoSpec, (long long)build_max, words_per_wave(g));
     HIPCHK(hipGetLastError());
     return 0;
 }
 
 int albd_push_spec(albd_ctx *c, const albd_graph *g, const albd_state *st, int32_t level, int spec,
-                   int64_t build_max)
+                   int64_t build_max, int scan)
 {
-    // the frontier bound is the one below which albd_push_scan takes the
-    // one-block scan
-    const Spec sp{spec, ALBBA_CHOICE_PUSH, (unsigned long long)ALBD_SPEC_PUSH_MAX};
+    // with a scan, the frontier bound is the one below which albd_push_scan
+    // takes the one-block scan
+    const Spec sp{spec, ALBBA_CHOICE_PUSH, scan ? (unsigned long long)ALBD_SPEC_PUSH_MAX : ~0ull};
     hipStream_t s = albd_stream(c);
-    hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(kBlock), 0, s, *g, *st, sp);
-    HIPCHK(hipGetLastError());
+    if (scan) {
+        hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(kBlock), 0, s, *g, *st, sp);
+        HIPCHK(hipGetLastError());
+    }
     hipLaunchKernelGGL(k_push_expand, dim3(grid_persistent(c, 8)), dim3(kBlock), 0, s, *g, *st, sp);
     HIPCHK(hipGetLastError());
-    const int grid = grid_for_qgroups(c, ((int64_t)g->nwords + 63) / 64);
-    hipLaunchKernelGGL(k_words_to_queue<true>, dim3(grid), dim3(kQBlock), 0, s, *g, *st, level, sp,
-                       (long long)build_max);
+    hipLaunchKernelGGL(k_words_to_queue<true>, dim3(grid_for_queue(c, g)), dim3(kQBlock), 0, s, *g, *st, level, sp,
+                       (long long)build_max, words_per_wave(g));
     HIPCHK(hipGetLastError());
     return 0;
 }

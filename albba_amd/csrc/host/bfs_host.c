@@ -709,6 +709,8 @@ int albd_level_begin_flags(albd_ctx *c, const albd_graph *g, const albd_state *s
 
 typedef struct loop_state {
     int have_queue;       /* st.queue holds the frontier                */
+    int have_prefix;      /* st.prefix its degree prefix (not kept where
+                           * trial runs write the next one)             */
     int prev_push;        /* last level pushed (queue_next pending)     */
     int list_valid;       /* st.active is a superset of unvisited words */
     int list_pending;     /* last level built a list (length pending)   */
@@ -732,7 +734,7 @@ static void sum_counters(const albd_counters *h, level_sums *o)
     o->col_bypassed = (int64_t)h->col_bypassed;
     o->qnext_len = (int64_t)h->qnext_len;
     o->active_len = (int64_t)h->active_len;
-    o->queue_len = (int64_t)h->queue_len;
+    o->queue_len = (int64_t)(h->queue_len & 0xffffffffull);
     o->push_edges = (int64_t)h->push_edges;
 }
 
@@ -746,8 +748,9 @@ static int run_level(albba_graph *G, const loop_state *ls, int choice, int32_t l
     int rc = albd_level_begin_flags(d, &G->g, &G->st, LB_SLOTS);
     if (rc) return rc;
     if (choice == ALBBA_CHOICE_PUSH) {
-        if (!ls->have_queue && (rc = albd_front_to_queue(d, &G->g, &G->st))) return rc;
-        if ((rc = albd_push_scan(d, &G->g, &G->st, frontier))) return rc;
+        if (!ls->have_queue) rc = albd_front_to_queue(d, &G->g, &G->st);
+        else rc = ls->have_prefix ? 0 : albd_push_scan(d, &G->g, &G->st, frontier);
+        if (rc) return rc;
         if (mark && (rc = albd_event_record(d, 6))) return rc;
         if ((rc = albd_push_expand(d, &G->g, &G->st))) return rc;
         if (mark && (rc = albd_event_record(d, 7))) return rc;
@@ -834,8 +837,9 @@ static int run_main(albba_graph *G, const loop_state *ls, int choice, int32_t le
     albd_ctx *d = G->ctx->d;
     int rc;
     if (choice == ALBBA_CHOICE_PUSH) {
-        if (!ls->have_queue && (rc = albd_front_to_queue(d, &G->g, &G->st))) return rc;
-        if ((rc = albd_push_scan(d, &G->g, &G->st, frontier))) return rc;
+        if (!ls->have_queue) rc = albd_front_to_queue(d, &G->g, &G->st);
+        else rc = ls->have_prefix ? 0 : albd_push_scan(d, &G->g, &G->st, frontier);
+        if (rc) return rc;
         if (mark && (rc = albd_event_record(d, 6))) return rc;
         if ((rc = albd_push_expand(d, &G->g, &G->st))) return rc;
         if (mark && (rc = albd_event_record(d, 7))) return rc;
@@ -882,8 +886,8 @@ static int run_small(albba_graph *G, const loop_state *ls, int32_t level, int64_
 
 /* Pointer swaps and bookkeeping after a committed level (list length from
  * the level's counters: commit_counts); queue_built: a pushed level listed
- * the next frontier's queue. */
-static void commit_pointers(albba_graph *G, loop_state *ls, int choice, int queue_built)
+ * the next frontier's queue, prefix_built: with its degree prefix. */
+static void commit_pointers(albba_graph *G, loop_state *ls, int choice, int queue_built, int prefix_built)
 {
     uint64_t *t = G->st.front;
     G->st.front = G->st.next;
@@ -897,6 +901,7 @@ static void commit_pointers(albba_graph *G, loop_state *ls, int choice, int queu
         G->st.queue = G->st.queue_next;
         G->st.queue_next = q;
         ls->have_queue = queue_built;
+        ls->have_prefix = queue_built && prefix_built;
         ls->prev_push = 1;
     } else {
         ls->have_queue = 0;
@@ -1108,7 +1113,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
     (policy != ALBBA_SWITCH_SCRIPT || script_at(G, &opts, (L) + 1) < 0                                 \
          ? queue_max_policy                                                                            \
          : (script_at(G, &opts, (L) + 1) == ALBBA_CHOICE_PUSH ? INT64_MAX : (int64_t)-1))
-    loop_state ls = {1, 0, 0, 0, 0};
+    loop_state ls = {1, 0, 0, 0, 0, 0};
     int small_streak = 0; /* consecutive plain push levels that stayed small */
     int slow_streak = 0;  /* consecutive small levels that did not double */
     int32_t level = 0;
@@ -1121,10 +1126,13 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
     const int spec = policy == ALBBA_SWITCH_HEURISTIC || policy == ALBBA_SWITCH_LEARNED ||
                      policy == ALBBA_SWITCH_SCRIPT;
     const int use_sel = policy != ALBBA_SWITCH_HEURISTIC; /* kernels queued ahead read sel_choice */
+    ls.have_prefix = spec; /* the root's, from the reset */
     unsigned int seq = 0;
     /* kernels already queued for the coming level: the choice whose pull is
-     * queued, or -1; whether the push kernels are */
+     * queued, or -1; whether the push kernels are, and the largest frontier
+     * they take */
     int queued_pull = -1, queued_push = 0;
+    int64_t queued_push_max = INT64_MAX;
     /* the vertex-order pass queued behind the last posted level (it runs only
      * if that level's select kernel finds the frontier empty), and the
      * frontier of the level before the current one */
@@ -1138,7 +1146,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
              /* the root level is a push as a rule; the small-frontier
               * kernel needs two push levels before it */
              (!opts.time_levels && (queued_push = 1, albd_push_spec(d, &G->g, &G->st, 0, use_sel,
-                                                                    QUEUE_MAX(0)))) ||
+                                                                    QUEUE_MAX(0), 0))) ||
              albd_mail_wait(d, &G->st, seq);
     else
         rc = albd_select_read(d, &G->g, &G->st, &sel);
@@ -1228,7 +1236,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
                            opts.small_frontier_blocks, opts.time_levels, spec, &nlev);
         else if (spec) {
             const int ran = choice == queued_pull ||
-                            (queued_push && choice == ALBBA_CHOICE_PUSH && frontier <= ALBD_SPEC_PUSH_MAX);
+                            (queued_push && choice == ALBBA_CHOICE_PUSH && frontier <= queued_push_max);
             /* the finalize kernel applies queue_max to the select kernel's
              * edge count, queued ahead or not */
             queue_built = choice != ALBBA_CHOICE_PUSH || first_edges <= queue_max;
@@ -1254,7 +1262,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
             /* swap to the next level's state, post the select kernel with
              * the next level's preparation beside it, then wait for the
              * counters */
-            commit_pointers(G, &ls, choice, queue_built);
+            commit_pointers(G, &ls, choice, queue_built, !small);
             if ((rc = select_prep(G, &ls, &sel, &seq))) return albba_fail(rc, "bfs: %s", albd_error());
             /* Queue the likely next kernels now, so that the device does
              * not wait for the host to read the choice: after a pull the
@@ -1284,10 +1292,12 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
                     guess = -1;
             }
             if (guess == ALBBA_CHOICE_PUSH && !opts.time_levels) {
+                /* (the small-frontier kernel's queue has no prefix) */
                 if ((rc = albd_push_spec(d, &G->g, &G->st, level + nlev, use_sel,
-                                         QUEUE_MAX(level + nlev))))
+                                         QUEUE_MAX(level + nlev), !ls.have_prefix)))
                     return albba_fail(rc, "bfs: %s", albd_error());
                 queued_push = 1;
+                queued_push_max = ls.have_prefix ? INT64_MAX : ALBD_SPEC_PUSH_MAX;
             }
             if (guess >= 0 && guess != ALBBA_CHOICE_PUSH && !opts.time_levels) {
                 const int variant = guess == ALBBA_CHOICE_PULL_SB
@@ -1355,7 +1365,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
                 if (stats->swept) stats->swept[lv] = j == 0 ? swept : -1;
             }
         }
-        if (!spec) commit_pointers(G, &ls, choice, 1);
+        if (!spec) commit_pointers(G, &ls, choice, 1, 0);
         commit_counts(&ls, choice, &sums);
         /* (a run of levels says nothing about the growth at its end) */
         frontier_prev = small ? (int64_t)hc->frontier : frontier;
