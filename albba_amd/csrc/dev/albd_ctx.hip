@@ -274,10 +274,11 @@ int albd_one_log(albd_ctx *c, const albd_one_level **host, albd_one_level **dev)
 {
     if (!c->one_log) {
         void *p = nullptr, *d = nullptr;
-        HIPCHK(hipHostMalloc(&p, sizeof(albd_one_level) * ALBD_ONE_NPOS, hipHostMallocMapped | hipHostMallocCoherent));
-        const hipError_t e = hipHostGetDevicePointer(&d, p, 0);
+        hipError_t e = hipHostMalloc(&p, sizeof(albd_one_level) * ALBD_ONE_NPOS,
+                                     hipHostMallocMapped | hipHostMallocCoherent);
+        if (e == hipSuccess && (e = hipHostGetDevicePointer(&d, p, 0)) != hipSuccess) (void)hipHostFree(p);
         if (e != hipSuccess) {
-            (void)hipHostFree(p);
+            (void)hipGetLastError();
             return albd_set_error(e, "level log", __FILE__, __LINE__);
         }
         c->one_log = (albd_one_level *)p;

@@ -1086,6 +1086,8 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
     if (policy == ALBBA_SWITCH_LEARNED && !opts.selector)
         return albba_fail(ALBBA_EINVAL, "bfs: learned policy needs a selector");
     albd_ctx *d = ctx->d;
+    const albd_one_level *one_log = NULL;
+    albd_one_level *one_dev = NULL;
     const int reps = opts.timing_reps > 0 ? opts.timing_reps : 1;
     int valid_mask = 0;
     for (int c = 0; c < ALBBA_NUM_CHOICES; ++c) valid_mask |= choice_ok(G, c) << c;
@@ -1105,7 +1107,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
     const int64_t learned_qmax = qratio > 0.0f ? (int64_t)ceil((double)qratio * (double)G->n) : push_vertex_cap;
     const int64_t queue_max_policy = policy == ALBBA_SWITCH_LEARNED ? learned_qmax : push_vertex_cap;
     if (!opts.time_levels && (policy == ALBBA_SWITCH_HEURISTIC || policy == ALBBA_SWITCH_LEARNED) &&
-        albd_one_fits(&G->g))
+        albd_one_fits(&G->g) && !albd_one_log(d, &one_log, &one_dev)) /* (no log: the loop) */
         return bfs_one(G, root, &opts, valid_mask, push_vertex_cap, queue_max_policy, stats, ev);
     /* a scripted level lists the queue exactly when the script pushes next
      * (-1: never; past the script the heuristic's rule) */
