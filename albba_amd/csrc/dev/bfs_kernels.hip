@@ -20,6 +20,9 @@
 // finds pmin[v] still all ones sets v in the next bitmap; a word pass then
 // writes level/parent and builds the next queue.
 #include "dev_common.h"
+// one own edge a thread (512 threads of two: 4 096 x 4 096 grid 5.6 us a level
+// against 5.4; 256 of two or four 6.5)
+#define PUSH_LIST_BLOCK 1024
 #include "push_lists.h"
 #include "select_dev.h"
 #include "../../../include/albba.h"
@@ -1158,7 +1161,7 @@ __global__ __launch_bounds__(kBlock) void k_push_expand(albd_graph g, albd_state
 // one workgroup carried the first 4 096 levels of a 4 096 x 4 096 grid alone
 // and the kernel took 8.2 us per level instead of 5.5.
 //
-// Measured on grids of 0.6, 4.2 and 16.8 M vertices: 4.0, 4.6 and 5.5 us per
+// Measured on grids of 0.6, 4.2 and 16.8 M vertices: 4.1, 4.5 and 5.4 us per
 // level, where a queue in memory between the levels, with its reservations
 // and a counting barrier, took 11.8, 12.3 and 13.6.  Of the 4 us about 1.3
 // are the atomic and the appends, 2.0 the loads behind the barrier (two
@@ -1604,10 +1607,10 @@ int albd_push_small(albd_ctx *c, const albd_graph *g, const albd_state *st, int3
     if (cap > g->npos / (2 * kFound)) cap = g->npos / (2 * kFound);
     if (cap < 1) cap = 1;
     // More workgroups shorten each one's part of a level but lengthen the
-    // barrier: measured us per level with 16, 32 and 64 workgroups on grids
-    // of 0.6, 4.2 and 16.8 M vertices: 4.04, 4.30, 4.65; 6.22, 4.91, 4.64;
-    // 9.43, 6.84, 5.56 (96 workgroups: 5.12, 4.96, 5.42).
-    if (blocks <= 0) blocks = g->n < (1 << 20) ? 16 : (g->n < (1 << 21) ? 32 : 64);
+    // barrier: measured us per level with 16, 32 and 64 workgroups on grids of
+    // 0.6, 2.3, 4.2, 7.3 and 16.8 M vertices: 4.1, 4.4, 4.9; 4.8, 4.5, 4.8; 4.8,
+    // 4.5, 4.8; 6.9, 5.5, 5.1; 8.5, 6.5, 5.4 (96 workgroups: 5.2-5.6).
+    if (blocks <= 0) blocks = g->n < (1 << 20) ? 16 : (g->n < 5 << 20 ? 32 : 64);
     if (blocks > cap) blocks = (int32_t)cap;
     // the grid state, the levels' counters and the error flag were zeroed by
     // the level-begin kernel (LB_SMALL)

@@ -12,13 +12,21 @@
 #pragma once
 #include "dev_common.h"
 
-constexpr int kListBlock = 512;
+// The threads of a workgroup are the including file's choice (PUSH_LIST_BLOCK);
+// the list has 1 024 edges either way.
+#ifndef PUSH_LIST_BLOCK
+#error "PUSH_LIST_BLOCK: threads of a workgroup"
+#endif
+
+namespace {
+
+constexpr int kListBlock = PUSH_LIST_BLOCK;
 constexpr int kListWaves = kListBlock / 64;
-constexpr int kListPer = 2;                          // own edges per thread
+constexpr int kListPer = 1024 / kListBlock;          // own edges per thread
 constexpr int kListEdges = kListPer * kListBlock;    // edges of the LDS list
 constexpr int kListDeg = 32;                         // most out-edges of a listed vertex
 constexpr int kListSlack = 64, kListKeep = 32;       // see list_cap
-constexpr int kSharePer = 4;                         // shared-queue edges per thread and window
+constexpr int kSharePer = 2048 / kListBlock;         // shared-queue edges per thread and window
 constexpr int kShareEdges = kSharePer * kListBlock;
 constexpr int kFound = 2048;                         // found-list entries reserved at a time
 static_assert(kFound >= kListEdges && kFound >= kShareEdges, "a window finds at most one reservation more");
@@ -376,3 +384,5 @@ __device__ __forceinline__ bool team_barrier(PushLds &S, const TeamSlots &B, uns
     __syncthreads();
     return S.ok != 0;
 }
+
+} // namespace
