@@ -4,9 +4,10 @@
 #include <cstdio>
 #include <cstring>
 #include <cstddef>
+#include <map>
 #include <mutex>
+#include <new>
 #include <unordered_map>
-#include <vector>
 
 #include "../albd.h"
 #include "../../../include/albba.h"
@@ -42,14 +43,21 @@ struct albd_ctx {
     void *stage[ALBD_STAGES];             // pinned, null until first used
     hipEvent_t stage_ev[ALBD_STAGES];
     std::mutex stage_lock;
+    struct Block {
+        size_t bytes;
+        bool kept;
+    };
     struct Kept {
         void *p;
-        size_t bytes;
+        unsigned long long age;
     };
+    using BySize = std::multimap<size_t, Kept>;
     std::mutex mem_lock;
-    std::unordered_map<void *, size_t> sizes; // every block, in use or kept
-    std::vector<Kept> kept;                   // freed ones, oldest first
+    std::unordered_map<void *, Block> blocks;             // in use or kept
+    BySize kept;                                          // freed ones
+    std::map<unsigned long long, BySize::iterator> oldest; // the same by age
     size_t kept_bytes;
+    unsigned long long age;
 };
 
 int albd_device_count(int *count)
@@ -119,45 +127,52 @@ hipStream_t albd_stream(albd_ctx *c) { return c->stream; }
 // device memory
 //
 // Freed blocks are kept for the context's next allocations, up to
-// ALBD_KEEP_BYTES.  The driver clears what is given back before it hands it
-// out again, at about 70 GB/s: a program that loads graph after graph (RMAT
-// s20: 2.3 GB of arrays and temporaries each) ran at that rate, 68 ms a load
-// where the work takes 20, and freeing a graph's arrays took 3 ms.  A kept
-// block is used again only by this context, whose work is in the order of its
-// one stream, so no wait is needed when it is freed.
+// ALBD_KEEP_BYTES and ALBD_KEEP_BLOCKS.  The driver clears what is given back
+// before it hands it out again, at about 70 GB/s: a program that loads graph
+// after graph (RMAT s20: 2.3 GB of arrays and temporaries each) ran at that
+// rate, 68 ms a load where the work takes 20, and freeing a graph's arrays took
+// 3 ms.  A kept block is used again only by this context, whose work is in the
+// order of its one stream, so no wait is needed when it is freed.
+//
+// The host entries for them can run out of host memory; no exception leaves
+// these functions.
 
-static int free_now(albd_ctx *c, void *p)
+static void free_now(albd_ctx *c, void *p)
 {
-    HIPCHK(hipSetDevice(c->device));
-    HIPCHK(hipFree(p));
-    return 0;
+    (void)hipSetDevice(c->device);
+    if (hipFree(p) != hipSuccess) (void)hipGetLastError();
+}
+
+// one kept block back to the device (mem_lock held)
+static void drop_one(albd_ctx *c, albd_ctx::BySize::iterator k)
+{
+    void *p = k->second.p;
+    c->kept_bytes -= k->first;
+    c->oldest.erase(k->second.age);
+    c->kept.erase(k);
+    c->blocks.erase(p);
+    free_now(c, p);
 }
 
 // every kept block back to the device (mem_lock held)
 static void drop_kept(albd_ctx *c)
 {
-    for (auto &k : c->kept) {
-        c->sizes.erase(k.p);
-        (void)free_now(c, k.p);
-    }
-    c->kept.clear();
-    c->kept_bytes = 0;
+    while (!c->kept.empty()) drop_one(c, c->kept.begin());
 }
 
 int albd_malloc(albd_ctx *c, size_t bytes, void **p)
 {
     if (!bytes) bytes = 256;
+    *p = nullptr;
     std::lock_guard<std::mutex> guard(c->mem_lock);
     // the smallest kept block that fits without wasting over a quarter
-    size_t best = c->kept.size();
-    for (size_t i = 0; i < c->kept.size(); ++i)
-        if (c->kept[i].bytes >= bytes && c->kept[i].bytes <= bytes + bytes / 4 + 4096 &&
-            (best == c->kept.size() || c->kept[i].bytes < c->kept[best].bytes))
-            best = i;
-    if (best < c->kept.size()) {
-        *p = c->kept[best].p;
-        c->kept_bytes -= c->kept[best].bytes;
-        c->kept.erase(c->kept.begin() + (std::ptrdiff_t)best);
+    const auto k = c->kept.lower_bound(bytes);
+    if (k != c->kept.end() && k->first <= bytes + bytes / 4 + 4096) {
+        *p = k->second.p;
+        c->blocks.find(*p)->second.kept = false;
+        c->kept_bytes -= k->first;
+        c->oldest.erase(k->second.age);
+        c->kept.erase(k);
         return 0;
     }
     HIPCHK(hipSetDevice(c->device));
@@ -173,7 +188,13 @@ int albd_malloc(albd_ctx *c, size_t bytes, void **p)
         snprintf(g_err, sizeof g_err, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
         return ALBBA_EDEVMEM;
     }
-    c->sizes[*p] = bytes;
+    try {
+        c->blocks.emplace(*p, albd_ctx::Block{bytes, false});
+    } catch (const std::bad_alloc &) {
+        free_now(c, *p);
+        *p = nullptr;
+        return albd_set_error_msg(ALBBA_ENOMEM, "device block: no host memory for its entry");
+    }
     return 0;
 }
 
@@ -181,23 +202,28 @@ void albd_free(albd_ctx *c, void *p)
 {
     if (!p) return;
     std::lock_guard<std::mutex> guard(c->mem_lock);
-    const auto it = c->sizes.find(p);
-    if (it == c->sizes.end()) return;
-    const size_t bytes = it->second;
-    if (bytes > ALBD_KEEP_BYTES / 2) {
-        c->sizes.erase(it);
-        (void)free_now(c, p);
-        return;
+    const auto it = c->blocks.find(p);
+    if (it == c->blocks.end() || it->second.kept) return;
+    const size_t bytes = it->second.bytes;
+    if (bytes <= ALBD_KEEP_BYTES / 2) {
+        // the oldest ones make room
+        while (!c->oldest.empty() &&
+               (c->kept_bytes + bytes > ALBD_KEEP_BYTES || c->kept.size() >= ALBD_KEEP_BLOCKS))
+            drop_one(c, c->oldest.begin()->second);
+        auto k = c->kept.end();
+        try {
+            k = c->kept.emplace(bytes, albd_ctx::Kept{p, c->age});
+            c->oldest.emplace(c->age, k);
+            ++c->age;
+            c->kept_bytes += bytes;
+            it->second.kept = true;
+            return;
+        } catch (const std::bad_alloc &) {
+            if (k != c->kept.end()) c->kept.erase(k); // given back instead
+        }
     }
-    // the oldest ones make room
-    while (c->kept_bytes + bytes > ALBD_KEEP_BYTES) {
-        c->kept_bytes -= c->kept.front().bytes;
-        c->sizes.erase(c->kept.front().p);
-        (void)free_now(c, c->kept.front().p);
-        c->kept.erase(c->kept.begin());
-    }
-    c->kept.push_back({p, bytes});
-    c->kept_bytes += bytes;
+    c->blocks.erase(it);
+    free_now(c, p);
 }
 
 int albd_h2d(albd_ctx *c, void *dst, const void *src, size_t bytes)

@@ -1,0 +1,82 @@
+"""The host code between the C API and the device, run without a GPU: a HIP
+runtime in host memory (fake_hip.c) stands in for the real one, so that what
+the library allocates, launches and times can be counted.  Each test is a
+program of its own, since the stand-in has to be loaded ahead of the library.
+"""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+ROCM = "/opt/rocm/include"
+
+pytestmark = pytest.mark.skipif(not os.path.isdir(os.path.join(ROCM, "hip")), reason="no HIP headers")
+
+PRELUDE = """
+import ctypes as C, sys
+fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+import numpy as np
+import albba_amd as A
+
+def get(name, ctype=C.c_longlong, n=0):
+    return (ctype * n).in_dll(fake, name) if n else ctype.in_dll(fake, name)
+
+def kernels():
+    return C.string_at(C.addressof(get("fake_log", C.c_char, 1 << 22))).decode().split()
+
+def empty(n):
+    # no entries: the stand-in runs no kernel, so a built layout holds none
+    return A.Graph.from_arrays(np.zeros(n + 1, np.int64), np.zeros(0, np.int32), symmetric=True)
+
+def levels(frontier, edges):
+    get("fake_levels", C.c_int).value = len(frontier)
+    get("fake_frontier", n=65)[:len(frontier)] = frontier
+    get("fake_edges", n=65)[:len(edges)] = edges
+
+live = lambda d=0: get("fake_live_bytes", n=2)[d]
+blocks = lambda d=0: get("fake_live_blocks", n=2)[d]
+"""
+
+
+@pytest.fixture(scope="session")
+def fake_hip(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake_hip") / "fake_hip.so")
+    subprocess.run(["gcc", "-O1", "-fPIC", "-shared", "-std=gnu11", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+                    "-I" + ROCM, "-I" + os.path.join(ROOT, "include"), "-o", so, os.path.join(HERE, "fake_hip.c")],
+                   check=True)
+    return so
+
+
+@pytest.fixture
+def program(fake_hip):
+    def run(body):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body), fake_hip], cwd=ROOT,
+                           capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    return run
+
+
+def test_kept_blocks_are_few(program):
+    """Freed device blocks that a context keeps are bounded in number and
+    bytes: closing thousands of small graphs gives most of them back."""
+    program("""
+        ctx = A.Context(0)
+        gs = [A.DeviceGraph.build(ctx, empty(100), 64, 64, 1) for _ in range(600)]
+        for g in gs:
+            g.close()
+        assert blocks() <= 4096, blocks()
+        # and they are used again: a graph like the last one takes none from
+        # the device
+        A.DeviceGraph.build(ctx, empty(100), 64, 64, 1).close()
+        before = blocks()
+        g = A.DeviceGraph.build(ctx, empty(100), 64, 64, 1)
+        assert blocks() == before
+        g.close()
+        ctx.close()
+        assert blocks() == 0 and live() == 0
+    """)
