@@ -137,9 +137,8 @@ hipStream_t albd_stream(albd_ctx *c) { return c->stream; }
 // The host entries for them can run out of host memory; no exception leaves
 // these functions.
 
-static void free_now(albd_ctx *c, void *p)
+static void free_now(void *p)
 {
-    (void)hipSetDevice(c->device);
     if (hipFree(p) != hipSuccess) (void)hipGetLastError();
 }
 
@@ -151,7 +150,7 @@ static void drop_one(albd_ctx *c, albd_ctx::BySize::iterator k)
     c->oldest.erase(k->second.age);
     c->kept.erase(k);
     c->blocks.erase(p);
-    free_now(c, p);
+    free_now(p);
 }
 
 // every kept block back to the device (mem_lock held)
@@ -164,6 +163,8 @@ int albd_malloc(albd_ctx *c, size_t bytes, void **p)
 {
     if (!bytes) bytes = 256;
     *p = nullptr;
+    // callers launch on the device without making it current themselves
+    HIPCHK(hipSetDevice(c->device));
     std::lock_guard<std::mutex> guard(c->mem_lock);
     // the smallest kept block that fits without wasting over a quarter
     const auto k = c->kept.lower_bound(bytes);
@@ -175,7 +176,6 @@ int albd_malloc(albd_ctx *c, size_t bytes, void **p)
         c->kept.erase(k);
         return 0;
     }
-    HIPCHK(hipSetDevice(c->device));
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess && !c->kept.empty()) {
         (void)hipGetLastError();
@@ -191,7 +191,7 @@ int albd_malloc(albd_ctx *c, size_t bytes, void **p)
     try {
         c->blocks.emplace(*p, albd_ctx::Block{bytes, false});
     } catch (const std::bad_alloc &) {
-        free_now(c, *p);
+        free_now(*p);
         *p = nullptr;
         return albd_set_error_msg(ALBBA_ENOMEM, "device block: no host memory for its entry");
     }
@@ -201,6 +201,7 @@ int albd_malloc(albd_ctx *c, size_t bytes, void **p)
 void albd_free(albd_ctx *c, void *p)
 {
     if (!p) return;
+    (void)hipSetDevice(c->device);
     std::lock_guard<std::mutex> guard(c->mem_lock);
     const auto it = c->blocks.find(p);
     if (it == c->blocks.end() || it->second.kept) return;
@@ -223,7 +224,7 @@ void albd_free(albd_ctx *c, void *p)
         }
     }
     c->blocks.erase(it);
-    free_now(c, p);
+    free_now(p);
 }
 
 int albd_h2d(albd_ctx *c, void *dst, const void *src, size_t bytes)
@@ -299,6 +300,7 @@ int albd_mail_wait(albd_ctx *c, const albd_state *st, unsigned int seq)
 int albd_one_log(albd_ctx *c, const albd_one_level **host, albd_one_level **dev)
 {
     if (!c->one_log) {
+        HIPCHK(hipSetDevice(c->device));
         void *p = nullptr, *d = nullptr;
         hipError_t e = hipHostMalloc(&p, sizeof(albd_one_level) * ALBD_ONE_NPOS,
                                      hipHostMallocMapped | hipHostMallocCoherent);

@@ -80,3 +80,15 @@ def test_kept_blocks_are_few(program):
         ctx.close()
         assert blocks() == 0 and live() == 0
     """)
+
+
+def test_allocating_makes_the_device_current(program):
+    """Two devices in one thread: a call that allocates makes its context's
+    device the current one, also where the memory is a kept block."""
+    program("""
+        a, b = A.Context(0), A.Context(1)
+        for _ in range(3):
+            a.bench_copy(1 << 20, 1)
+            b.bench_copy(1 << 20, 1)
+        assert get("fake_wrong_device", C.c_int).value == 0
+    """)
