@@ -170,6 +170,7 @@ def lib() -> C.CDLL:
         "albba_ctx_create": (C.c_int, [C.c_int, C.POINTER(C.c_void_p)]),
         "albba_ctx_destroy": (None, [C.c_void_p]),
         "albba_ctx_synchronize": (C.c_int, [C.c_void_p]),
+        "albba_ctx_trim": (C.c_int, [C.c_void_p]),
         "albba_bench_copy": (C.c_int, [C.c_void_p, C.c_int64, C.c_int, C.POINTER(C.c_float)]),
         "albba_graph_upload": (C.c_int, [C.c_void_p, C.POINTER(_SELL), C.POINTER(C.c_void_p)]),
         "albba_graph_build": (C.c_int, [C.c_void_p, C.POINTER(_CSR), C.c_int, C.c_int, C.c_int,
@@ -434,6 +435,11 @@ class Context:
 
     def synchronize(self):
         _check(lib().albba_ctx_synchronize(self._p))
+
+    def trim(self):
+        """Give the device memory that the context keeps of closed graphs and
+        batches back to the device (albba_ctx_trim)."""
+        _check(lib().albba_ctx_trim(self._p))
 
     def bench_copy(self, nbytes: int, reps: int = 10) -> float:
         """Mean ms of one device-to-device copy of nbytes (copy kernel)."""

@@ -158,12 +158,14 @@ ALBD_HIDDEN void albd_ctx_destroy(albd_ctx *c);
 ALBD_HIDDEN int albd_ctx_device(const albd_ctx *c);
 ALBD_HIDDEN int albd_num_cus(const albd_ctx *c);
 /* freed blocks are kept for later allocations of the context, at most
- * ALBD_KEEP_BYTES in ALBD_KEEP_BLOCKS blocks, and given back with it or when
- * memory runs out (a graph has about 35 blocks, its build 60 more) */
+ * ALBD_KEEP_BYTES in ALBD_KEEP_BLOCKS blocks (a graph has about 35, its
+ * build 60 more), and given back with the context, by albd_trim, or when an
+ * allocation of any context on the device fails */
 #define ALBD_KEEP_BYTES ((size_t)4 << 30)
 #define ALBD_KEEP_BLOCKS 4096
 ALBD_HIDDEN int albd_malloc(albd_ctx *c, size_t bytes, void **p);
 ALBD_HIDDEN void albd_free(albd_ctx *c, void *p);
+ALBD_HIDDEN int albd_trim(albd_ctx *c); /* 1: there were some */
 ALBD_HIDDEN int albd_h2d(albd_ctx *c, void *dst, const void *src, size_t bytes);
 ALBD_HIDDEN int albd_d2h(albd_ctx *c, void *dst, const void *src, size_t bytes);
 ALBD_HIDDEN int albd_d2d(albd_ctx *c, void *dst, const void *src, size_t bytes); /* async */

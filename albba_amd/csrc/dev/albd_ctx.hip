@@ -58,7 +58,12 @@ struct albd_ctx {
     std::map<unsigned long long, BySize::iterator> oldest; // the same by age
     size_t kept_bytes;
     unsigned long long age;
+    albd_ctx *next; // of the process's contexts
 };
+
+// every context of the process.  contexts_lock comes before a mem_lock.
+static std::mutex contexts_lock;
+static albd_ctx *contexts;
 
 int albd_device_count(int *count)
 {
@@ -95,15 +100,24 @@ int albd_ctx_create(int device, albd_ctx **out)
                          hipHostMallocMapped | hipHostMallocCoherent));
     memset(c->mail, 0, sizeof(albd_counters));
     HIPCHK(hipHostGetDevicePointer((void **)&c->dmail, c->mail, 0));
+    {
+        std::lock_guard<std::mutex> all(contexts_lock);
+        c->next = contexts;
+        contexts = c;
+    }
     *out = c;
     return 0;
 }
 
-static void drop_kept(albd_ctx *c);
-
 void albd_ctx_destroy(albd_ctx *c)
 {
     if (!c) return;
+    {
+        std::lock_guard<std::mutex> all(contexts_lock);
+        albd_ctx **at = &contexts;
+        while (*at && *at != c) at = &(*at)->next;
+        if (*at) *at = c->next;
+    }
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     for (int i = 0; i < ALBD_NEVENTS; ++i) (void)hipEventDestroy(c->ev[i]);
@@ -111,7 +125,7 @@ void albd_ctx_destroy(albd_ctx *c)
     (void)hipHostFree(c->hctr);
     (void)hipHostFree(c->mail);
     if (c->one_log) (void)hipHostFree(c->one_log);
-    drop_kept(c);
+    albd_trim(c);
     for (int i = 0; i < ALBD_STAGES && c->stage[0]; ++i) {
         (void)hipHostFree(c->stage[i]);
         (void)hipEventDestroy(c->stage_ev[i]);
@@ -132,7 +146,9 @@ hipStream_t albd_stream(albd_ctx *c) { return c->stream; }
 // after graph (RMAT s20: 2.3 GB of arrays and temporaries each) ran at that
 // rate, 68 ms a load where the work takes 20, and freeing a graph's arrays took
 // 3 ms.  A kept block is used again only by this context, whose work is in the
-// order of its one stream, so no wait is needed when it is freed.
+// order of its one stream, so no wait is needed when it is freed.  When device
+// memory runs out, every context on the device gives its kept blocks back
+// (hipFree waits for what is still done with them).
 //
 // The host entries for them can run out of host memory; no exception leaves
 // these functions.
@@ -153,10 +169,23 @@ static void drop_one(albd_ctx *c, albd_ctx::BySize::iterator k)
     free_now(p);
 }
 
-// every kept block back to the device (mem_lock held)
-static void drop_kept(albd_ctx *c)
+int albd_trim(albd_ctx *c)
 {
+    (void)hipSetDevice(c->device);
+    std::lock_guard<std::mutex> guard(c->mem_lock);
+    const int any = c->kept.empty() ? 0 : 1;
     while (!c->kept.empty()) drop_one(c, c->kept.begin());
+    return any;
+}
+
+// the kept blocks of every context on the device back to it
+static bool trim_device(int device)
+{
+    std::lock_guard<std::mutex> all(contexts_lock);
+    bool any = false;
+    for (albd_ctx *c = contexts; c; c = c->next)
+        if (c->device == device) any |= albd_trim(c) != 0;
+    return any;
 }
 
 int albd_malloc(albd_ctx *c, size_t bytes, void **p)
@@ -165,22 +194,23 @@ int albd_malloc(albd_ctx *c, size_t bytes, void **p)
     *p = nullptr;
     // callers launch on the device without making it current themselves
     HIPCHK(hipSetDevice(c->device));
-    std::lock_guard<std::mutex> guard(c->mem_lock);
-    // the smallest kept block that fits without wasting over a quarter
-    const auto k = c->kept.lower_bound(bytes);
-    if (k != c->kept.end() && k->first <= bytes + bytes / 4 + 4096) {
-        *p = k->second.p;
-        c->blocks.find(*p)->second.kept = false;
-        c->kept_bytes -= k->first;
-        c->oldest.erase(k->second.age);
-        c->kept.erase(k);
-        return 0;
+    {
+        std::lock_guard<std::mutex> guard(c->mem_lock);
+        // the smallest kept block that fits without wasting over a quarter
+        const auto k = c->kept.lower_bound(bytes);
+        if (k != c->kept.end() && k->first <= bytes + bytes / 4 + 4096) {
+            *p = k->second.p;
+            c->blocks.find(*p)->second.kept = false;
+            c->kept_bytes -= k->first;
+            c->oldest.erase(k->second.age);
+            c->kept.erase(k);
+            return 0;
+        }
     }
     hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess && !c->kept.empty()) {
+    if (e != hipSuccess) {
         (void)hipGetLastError();
-        drop_kept(c);
-        e = hipMalloc(p, bytes);
+        if (trim_device(c->device)) e = hipMalloc(p, bytes);
     }
     if (e != hipSuccess) {
         (void)hipGetLastError();
@@ -189,6 +219,7 @@ int albd_malloc(albd_ctx *c, size_t bytes, void **p)
         return ALBBA_EDEVMEM;
     }
     try {
+        std::lock_guard<std::mutex> guard(c->mem_lock);
         c->blocks.emplace(*p, albd_ctx::Block{bytes, false});
     } catch (const std::bad_alloc &) {
         free_now(*p);

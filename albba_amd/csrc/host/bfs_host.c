@@ -67,6 +67,13 @@ int albba_ctx_synchronize(albba_ctx *c)
     return rc ? albba_fail(rc, "%s", albd_error()) : ALBBA_OK;
 }
 
+int albba_ctx_trim(albba_ctx *c)
+{
+    if (!c) return albba_fail(ALBBA_EINVAL, "ctx_trim: null");
+    (void)albd_trim(c->d);
+    return ALBBA_OK;
+}
+
 albd_ctx *albba_ctx_dev(albba_ctx *c) { return c ? c->d : NULL; }
 
 int albba_bench_copy(albba_ctx *c, int64_t bytes, int reps, float *ms)

@@ -344,6 +344,13 @@ ALBBA_API int albba_device_count(int *count);
 ALBBA_API int albba_ctx_create(int device, albba_ctx **out);
 ALBBA_API void albba_ctx_destroy(albba_ctx *ctx);
 ALBBA_API int albba_ctx_synchronize(albba_ctx *ctx);
+/* A context keeps the device memory of freed graphs, batches and temporaries
+ * for its next ones: at most 4 GiB in at most 4096 blocks, none of them over
+ * 2 GiB.  It goes back to the device with the context, when an allocation of
+ * any context of the process on the device fails, and by this call: for a
+ * program that gives the device to another library or process meanwhile.  (The
+ * pinned host memory of a context, under 20 MB, stays with it.) */
+ALBBA_API int albba_ctx_trim(albba_ctx *ctx);
 /* Upload a SELL layout (+ push CSR) and allocate the BFS state on the
  * context's device. */
 ALBBA_API int albba_graph_upload(albba_ctx *ctx, const albba_sellcs *s, albba_graph **out);

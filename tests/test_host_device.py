@@ -82,6 +82,39 @@ def test_kept_blocks_are_few(program):
     """)
 
 
+def test_kept_blocks_go_to_other_contexts(program):
+    """A context that runs out of device memory gets the blocks that the
+    device's other contexts keep; trim gives a context's own back."""
+    program("""
+        get("fake_capacity").value = 1 << 30
+        a, b = A.Context(0), A.Context(0)
+        other = A.Context(1)
+        other.bench_copy(300 << 20, 1)
+        a.bench_copy(400 << 20, 1)
+        assert live() >= 800 << 20
+        b.bench_copy(300 << 20, 1)
+        assert live(1) >= 600 << 20  # another device's are left alone
+        a.bench_copy(400 << 20, 1)
+        # what does not fit an empty device fails as before
+        try:
+            b.bench_copy(600 << 20, 1)
+            raise SystemExit("1.2 GB on a device of 1 GB")
+        except A.AlbbaError as e:
+            assert e.code == -7
+        b.trim()
+        assert live() == 0
+        a.bench_copy(200 << 20, 1)
+        assert live() == 400 << 20
+        a.trim()
+        assert live() == 0
+        a.close()
+        assert A.lib().albba_ctx_trim(None) == -1
+        b.bench_copy(500 << 20, 1)
+        b.close()
+        assert live() == 0
+    """)
+
+
 def test_allocating_makes_the_device_current(program):
     """Two devices in one thread: a call that allocates makes its context's
     device the current one, also where the memory is a kept block."""
