@@ -391,11 +391,16 @@ ALBD_HIDDEN int albd_bfs_one(albd_ctx *c, const albd_graph *g, const albd_state 
 /* ---- batched BFS (batch.hip) ---- */
 /* most workgroups of a team */
 #define ALBD_BATCH_TEAM_MAX 64
-/* entries of an instance's found list: every position, and two unfilled
- * reservations (2 048 entries) of every workgroup of the largest team */
-#define ALBD_BATCH_FOUND(npos) ((size_t)(npos) + ALBD_BATCH_TEAM_MAX * 2 * 2048)
-/* words of an instance's barrier slots: two sets of three counts */
-#define ALBD_BATCH_SLOTS (2 * 3 * ALBD_BATCH_TEAM_MAX)
+/* found-list entries that a workgroup may have reserved and not filled */
+#define ALBD_BATCH_SLACK (2 * 2048)
+/* entries of an instance's found list for a team of T: every position, and the
+ * unfilled reservations of every workgroup (one workgroup's reservations are in
+ * order, so that its vertices alone fit) */
+#define ALBD_BATCH_FOUND(npos, T) ((size_t)(npos) + ((T) > 1 ? (size_t)(T) * ALBD_BATCH_SLACK : 0))
+/* words of an instance's barrier slots: two sets of three counts, each of whole
+ * 128-byte lines (one workgroup has no barrier) */
+#define ALBD_BATCH_STRIDE(T) (((T) + 15) / 16 * 16)
+#define ALBD_BATCH_SLOTS(T) ((T) > 1 ? (size_t)(2 * 3 * ALBD_BATCH_STRIDE(T)) : 0)
 /* One instance: a device graph, its own scratch, a root.  The control block
  * ctl (32 words) and the slots must be zero before the launch: [1], [3] found-
  * list reservations, [2] error flag, [4..7] shared-queue entries and [8..11]
@@ -404,11 +409,11 @@ typedef struct albd_batch_item {
     albd_graph g;
     uint64_t *visited;           /* [nwords] */
     uint64_t *bm[3];             /* [nwords] frontier bitmaps, rotating */
-    int32_t *found;              /* [ALBD_BATCH_FOUND(npos)] vertices found by pushes */
+    int32_t *found;              /* [ALBD_BATCH_FOUND(npos, its largest team)] vertices found by pushes */
     unsigned long long *key;     /* [npos] (level, parent id), all ones at rest */
     int32_t *level, *parent;     /* [n] results in vertex order; push queues before */
     unsigned long long *ctl;     /* [32] see above */
-    unsigned long long *slot;    /* [ALBD_BATCH_SLOTS] the team barrier's arrivals */
+    unsigned long long *slot;    /* [ALBD_BATCH_SLOTS(its largest team)] the team barrier's arrivals */
     int32_t root;                /* vertex id */
     int32_t mapping;             /* pull: ALBD_MAP_LANE_ROW or ALBD_MAP_WAVE_ROW */
 } albd_batch_item;

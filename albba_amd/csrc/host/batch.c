@@ -39,12 +39,14 @@ struct albba_batch {
     int32_t wcap;                 /* resident workgroups of the batch kernel */
     albba_graph **graphs;
     albd_batch_item *items;       /* host copies (pinned, head of `stage`) */
-    unsigned long long *ctl;      /* device: count * CTL_WORDS */
+    unsigned long long *ctl;      /* device: count * CTL_WORDS, then the instances' slots */
+    size_t ctl_words;             /* both */
     unsigned long long *hctl;     /* host mirror (pinned) */
     void **allocs;                /* device allocations to free */
     int32_t nallocs;
     int32_t *team_of;             /* instance -> team, team sizes of the last run */
     int32_t *team_size_of;
+    int32_t *team_max;            /* largest team of each instance (see largest_team) */
     /* host work arrays of a run, sized at creation for `wcap` workgroups, so
      * that a run allocates no host memory */
     int32_t *order, *share, *cnt, *team_first, *team_size, *team_ptr, *team_items, *wg_team;
@@ -73,6 +75,36 @@ static void *bdalloc(albba_batch *b, size_t bytes, int *rc)
     return p;
 }
 
+static double inst_cost(const albba_graph *G) { return (double)G->g.nnz + (double)G->g.n; }
+
+/* per-level latency of a team of s workgroups, microseconds (see est_us), and
+ * the largest team that an instance gets for its latency */
+#define LAT_A 4.0
+#define LAT_B 8.0
+#define TEAM_MAX 16
+
+/* an instance's share of W workgroups by its cost */
+static int32_t share_of(const albba_graph *G, double total, int32_t W)
+{
+    const double s = (double)W * inst_cost(G) / (total > 0 ? total : 1);
+    return s >= ALBD_BATCH_TEAM_MAX ? ALBD_BATCH_TEAM_MAX : (int32_t)s;
+}
+
+/* The largest team that an instance may get: its share of all workgroups, or
+ * for its latency TEAM_MAX.  A team's unfilled reservations take 16 KB of found
+ * list a workgroup, so that the latency team is held to what the graph's own
+ * positions take as much as, or to an even part of the workgroups: a batch of N
+ * instances needs at most its graphs' lists twice and 16 KB for each of
+ * 2 * wcap workgroups more, not N times what the largest team needs. */
+static int32_t largest_team(const albba_graph *G, double total, int32_t wcap, int32_t N)
+{
+    const int64_t own = G->g.npos / ALBD_BATCH_SLACK, even = wcap / N;
+    const int64_t fit = own > even ? own : even;
+    const int32_t lat = fit > TEAM_MAX ? TEAM_MAX : (int32_t)fit, share = share_of(G, total, wcap);
+    const int32_t t = share > lat ? share : lat;
+    return t > 1 ? t : 1;
+}
+
 void albba_batch_free(albba_batch *b)
 {
     if (!b) return;
@@ -83,6 +115,7 @@ void albba_batch_free(albba_batch *b)
     free(b->graphs);
     free(b->team_of);
     free(b->team_size_of);
+    free(b->team_max);
     free(b->order); free(b->share); free(b->cnt); free(b->team_first); free(b->team_size);
     free(b->team_ptr); free(b->team_items); free(b->wg_team); free(b->load);
     free(b->hist_levels); free(b->hist_team); free(b->own); free(b->hist_us); free(b->hist_scale); free(b->est);
@@ -109,6 +142,7 @@ int albba_batch_create(albba_ctx *ctx, albba_graph *const *graphs, int32_t count
     b->allocs = (void **)albba_calloc(N * 12 + 1, sizeof(void *));
     b->team_of = (int32_t *)albba_calloc(N, sizeof(int32_t));
     b->team_size_of = (int32_t *)albba_calloc(N, sizeof(int32_t));
+    b->team_max = (int32_t *)albba_calloc(N, sizeof(int32_t));
     b->order = (int32_t *)albba_calloc(N, sizeof(int32_t));
     b->share = (int32_t *)albba_calloc(N, sizeof(int32_t));
     b->cnt = (int32_t *)albba_calloc(W + 1, sizeof(int32_t));
@@ -126,7 +160,7 @@ int albba_batch_create(albba_ctx *ctx, albba_graph *const *graphs, int32_t count
     b->est = (double *)albba_calloc(N, sizeof(double));
     b->tab_off = tab_offset(count);
     b->stage_bytes = b->tab_off + sizeof(int32_t) * tab_words(count, wcap, (int32_t)T);
-    if (!b->graphs || !b->allocs || !b->team_of || !b->team_size_of || !b->order || !b->share ||
+    if (!b->graphs || !b->allocs || !b->team_of || !b->team_size_of || !b->team_max || !b->order || !b->share ||
         !b->cnt || !b->load || !b->team_first || !b->team_size || !b->team_ptr || !b->team_items ||
         !b->wg_team || !b->hist_levels || !b->hist_team || !b->own || !b->hist_us || !b->hist_scale || !b->est) {
         albba_batch_free(b);
@@ -142,7 +176,15 @@ int albba_batch_create(albba_ctx *ctx, albba_graph *const *graphs, int32_t count
     b->items = (albd_batch_item *)b->stage;
     memset(b->stage, 0, b->stage_bytes);
     /* the control blocks, then the barrier slots: zeroed together */
-    b->ctl = (unsigned long long *)bdalloc(b, sizeof(unsigned long long) * (CTL_WORDS + ALBD_BATCH_SLOTS) * (size_t)count, &rc);
+    double total = 0;
+    for (int32_t i = 0; i < count; ++i) total += inst_cost(graphs[i]);
+    b->ctl_words = N * CTL_WORDS;
+    for (int32_t i = 0; i < count; ++i) {
+        b->team_max[i] = largest_team(graphs[i], total, wcap, count);
+        b->ctl_words += ALBD_BATCH_SLOTS(b->team_max[i]);
+    }
+    b->ctl = (unsigned long long *)bdalloc(b, sizeof(unsigned long long) * b->ctl_words, &rc);
+    unsigned long long *slot = b->ctl + N * CTL_WORDS;
     for (int32_t i = 0; i < count && !rc; ++i) {
         albba_graph *G = graphs[i];
         b->graphs[i] = G;
@@ -151,13 +193,14 @@ int albba_batch_create(albba_ctx *ctx, albba_graph *const *graphs, int32_t count
         it->g = G->g;
         it->visited = (uint64_t *)bdalloc(b, 8 * nw, &rc);
         for (int k = 0; k < 3; ++k) it->bm[k] = (uint64_t *)bdalloc(b, 8 * nw, &rc);
-        it->found = (int32_t *)bdalloc(b, 4 * ALBD_BATCH_FOUND(np), &rc);
+        it->found = (int32_t *)bdalloc(b, 4 * ALBD_BATCH_FOUND(np, b->team_max[i]), &rc);
         it->key = (unsigned long long *)bdalloc(b, 8 * np, &rc);
         it->level = (int32_t *)bdalloc(b, 4 * n, &rc);
         it->parent = (int32_t *)bdalloc(b, 4 * n, &rc);
         if (!rc) rc = albd_fill_u64(ctx->d, it->key, ~0ull, np);
         it->ctl = b->ctl + (size_t)i * CTL_WORDS;
-        it->slot = b->ctl + (size_t)count * CTL_WORDS + (size_t)i * ALBD_BATCH_SLOTS;
+        it->slot = slot;
+        if (!rc) slot += ALBD_BATCH_SLOTS(b->team_max[i]);
         it->mapping = ALBD_MAP_LANE_ROW;
     }
     if (!rc) rc = albd_sync(ctx->d);
@@ -170,8 +213,6 @@ int albba_batch_create(albba_ctx *ctx, albba_graph *const *graphs, int32_t count
     *out = b;
     return ALBBA_OK;
 }
-
-static double inst_cost(const albba_graph *G) { return (double)G->g.nnz + (double)G->g.n; }
 
 /* Split W workgroups into teams and give every instance a team.  Fills
  * team_first/team_size (teams), team_ptr/team_items (instances per team),
@@ -187,15 +228,13 @@ static int32_t split_teams(albba_batch *b, int32_t W, int32_t *team_first, int32
     const int32_t N = b->count;
     double total = 0;
     for (int32_t i = 0; i < N; ++i) total += inst_cost(b->graphs[i]);
-    if (total <= 0) total = 1;
     int32_t *order = b->order, *share = b->share, *cnt = b->cnt;
     double *load = b->load;
     memset(load, 0, sizeof(double) * (size_t)W);
     memset(cnt, 0, sizeof(int32_t) * ((size_t)W + 1));
     for (int32_t i = 0; i < N; ++i) {
         order[i] = i;
-        double s = (double)W * inst_cost(b->graphs[i]) / total;
-        share[i] = s >= ALBD_BATCH_TEAM_MAX ? ALBD_BATCH_TEAM_MAX : (int32_t)s;
+        share[i] = share_of(b->graphs[i], total, W); /* at most team_max: W <= wcap */
     }
     for (int32_t i = 1; i < N; ++i) { /* insertion sort by cost, descending */
         int32_t x = order[i], j = i - 1;
@@ -251,10 +290,6 @@ static int32_t split_teams(albba_batch *b, int32_t W, int32_t *team_first, int32
     return T;
 }
 
-/* per-level latency of a team of s workgroups, microseconds */
-#define LAT_A 4.0
-#define LAT_B 8.0
-#define TEAM_MAX 16
 /* Other roots take other level counts and the estimates come from one run
  * under its own contention: only instances estimated at most SHARE_FRAC of
  * the makespan share workgroups, in teams filled to BIN_FRAC of it. */
@@ -275,14 +310,21 @@ static double est_us(const albba_batch *b, int32_t i, int32_t s)
     return L * lat_us(s) + work * b->hist_scale[i] * (double)s0 / (double)s;
 }
 
-/* the smallest team size <= TEAM_MAX with instance i done within M, or 0;
+/* the largest team that instance i gets for its latency */
+static int32_t latency_team(const albba_batch *b, int32_t i)
+{
+    return b->team_max[i] < TEAM_MAX ? b->team_max[i] : TEAM_MAX;
+}
+
+/* the smallest team size <= latency_team with instance i done within M, or 0;
  * never below the instance's own team in the share split (a work-heavy
  * instance slows by far more than its team shrinks: an RMAT s20 instance
  * that took 4.6 ms on 12 workgroups took 218 ms on one beside busy grids) */
 static int32_t team_for(const albba_batch *b, int32_t i, double M)
 {
     const int32_t s0 = b->hist_team[i] >= 2 ? b->hist_team[i] : 1;
-    for (int32_t s = s0; s <= (s0 > TEAM_MAX ? s0 : TEAM_MAX); ++s)
+    const int32_t most = latency_team(b, i);
+    for (int32_t s = s0; s <= (s0 > most ? s0 : most); ++s)
         if (est_us(b, i, s) <= M) return s;
     return 0;
 }
@@ -343,7 +385,7 @@ static int32_t split_teams_hist(albba_batch *b, int32_t W, int32_t *team_first, 
     for (int32_t i = 0; i < N; ++i) {
         b->est[i] = est_us(b, i, 1);
         order[i] = i;
-        const double best = est_us(b, i, TEAM_MAX) < b->est[i] ? est_us(b, i, TEAM_MAX) : b->est[i];
+        const double most = est_us(b, i, latency_team(b, i)), best = most < b->est[i] ? most : b->est[i];
         if (best > lo) lo = best;
         hi += b->est[i];
     }
@@ -383,7 +425,7 @@ static int32_t split_teams_hist(albba_batch *b, int32_t W, int32_t *team_first, 
             if (!b->own[i]) continue;
             const int32_t t = inst_team[i], s = team_size[t];
             const double e = est_us(b, i, s);
-            if (s < TEAM_MAX && est_us(b, i, s + 1) < e && e > worst) {
+            if (s < latency_team(b, i) && est_us(b, i, s + 1) < e && e > worst) {
                 worst = e;
                 tb = t;
             }
@@ -496,7 +538,7 @@ static int batch_run(albba_batch *b, const int32_t *roots, const albba_bfs_opts 
     float ms = 0;
     /* descriptors and tables in one copy from the pinned staging buffer */
     (void)((rc = albd_h2d(d, dev, b->stage, bytes)) ||
-           (rc = albd_fill_u64(d, b->ctl, 0, (size_t)N * (CTL_WORDS + ALBD_BATCH_SLOTS))) || (rc = albd_event_record(d, 4)) ||
+           (rc = albd_fill_u64(d, b->ctl, 0, b->ctl_words)) || (rc = albd_event_record(d, 4)) ||
            (rc = albd_batch_launch(d, &a, used)) || (rc = albd_event_record(d, 5)) ||
            (rc = albd_event_elapsed(d, 4, 5, &ms)) ||
            (rc = albd_d2h(d, b->hctl, b->ctl, sizeof(unsigned long long) * (size_t)N * CTL_WORDS)));

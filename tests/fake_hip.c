@@ -124,13 +124,15 @@ typedef struct {
     int device;
 } head_t;
 #define HEAD 4096
+#define BIG (1u << 20)
 
 API hipError_t hipMalloc(void **p, size_t bytes)
 {
     *p = NULL;
     if (fake_live_bytes[current] + (long long)bytes > fake_capacity) return hipErrorOutOfMemory;
-    char *m = (char *)mmap(NULL, bytes + HEAD, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
-    if (m == MAP_FAILED) return hipErrorOutOfMemory;
+    /* (large ones by mmap, so that what is not touched takes no memory) */
+    char *m = bytes < BIG ? (char *)calloc(1, bytes + HEAD) : (char *)mmap(NULL, bytes + HEAD, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+    if (!m || m == MAP_FAILED) return hipErrorOutOfMemory;
     ((head_t *)m)->bytes = bytes;
     ((head_t *)m)->device = current;
     fake_live_bytes[current] += (long long)bytes;
@@ -144,7 +146,8 @@ API hipError_t hipFree(void *p)
     head_t *h = (head_t *)((char *)p - HEAD);
     fake_live_bytes[h->device] -= (long long)h->bytes;
     --fake_live_blocks[h->device];
-    munmap(h, h->bytes + HEAD);
+    if (h->bytes < BIG) free(h);
+    else munmap(h, h->bytes + HEAD);
     return hipSuccess;
 }
 API hipError_t hipHostMalloc(void **p, size_t bytes, unsigned f)
