@@ -84,7 +84,7 @@ __device__ bool run_instance(BLds &S, const albd_batch_item &it, int rank, int T
     auto team_tid = [&]() -> int64_t { return (int64_t)rank * kBB + here_tid(); };
     const int64_t nwords = g.nwords;
     PushLds &L = S.l;
-    const TeamSlots B{it.slot, err_flag(it), ALBD_BATCH_STRIDE(T), T, rank, spin_limit};
+    const TeamSlots B{it.slot, err_flag(it), ALBD_BATCH_TEAM_MAX, T, rank, spin_limit};
     unsigned int tag = 0;
     const bool leader = rank == 0 && tid == 0;
     if (leader) st_coherent(reinterpret_cast<long long *>(&it.ctl[ALBD_RES_T0]), (long long)wall_clock64());
