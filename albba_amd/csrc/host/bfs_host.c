@@ -718,6 +718,8 @@ typedef struct loop_state {
     int have_queue;       /* st.queue holds the frontier                */
     int have_prefix;      /* st.prefix its degree prefix (not kept where
                            * trial runs write the next one)             */
+    int unlisted;         /* BEST: the level loop would not have listed the
+                           * queue                                      */
     int prev_push;        /* last level pushed (queue_next pending)     */
     int list_valid;       /* st.active is a superset of unvisited words */
     int list_pending;     /* last level built a list (length pending)   */
@@ -859,6 +861,30 @@ static int run_main(albba_graph *G, const loop_state *ls, int choice, int32_t le
     const int64_t bound = ls->list_valid ? ls->list_len : G->g.nwords;
     if ((rc = albd_pull(d, &G->g, &G->st, variant, level, bound))) return rc;
     return mark ? albd_event_record(d, 7) : 0;
+}
+
+/* What a trial of `choice` finds in place when the level loop runs it (not
+ * timed): the state after the select kernel, the preparation that the loop
+ * queues behind it for every choice (zero next, unvisited-word list, frontier
+ * summary), and for a push the queue's degree prefix, which the last push
+ * listed and another trial has overwritten -- or no queue, where the loop would
+ * not have listed it and the push starts from the bitmap.  *ls is the trial's
+ * own. */
+static int trial_prep(albba_graph *G, loop_state *ls, int choice, int32_t level, int64_t frontier)
+{
+    albd_ctx *d = G->ctx->d;
+    int rc;
+    if ((rc = albd_d2d(d, G->st.visited, G->scratch_visited, sizeof(uint64_t) * (size_t)G->g.nwords)) ||
+        (rc = albd_d2d(d, G->st.ctr, G->scratch_ctr, sizeof(albd_counters))) ||
+        (rc = albd_level_begin_flags(d, &G->g, &G->st, LB_SLOTS)) || (rc = prep_level(G, ls, level)))
+        return rc;
+    if (choice != ALBBA_CHOICE_PUSH || !ls->have_queue) return 0;
+    if (ls->unlisted) {
+        ls->have_queue = 0;
+        return albd_fill_u64(d, &G->st.ctr->queue_len, 0, 1);
+    }
+    ls->have_prefix = 1;
+    return albd_push_scan(d, &G->g, &G->st, frontier);
 }
 
 /* Push levels in the single-workgroup kernel, starting with the level whose
@@ -1122,7 +1148,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
     (policy != ALBBA_SWITCH_SCRIPT || script_at(G, &opts, (L) + 1) < 0                                 \
          ? queue_max_policy                                                                            \
          : (script_at(G, &opts, (L) + 1) == ALBBA_CHOICE_PUSH ? INT64_MAX : (int64_t)-1))
-    loop_state ls = {1, 0, 0, 0, 0, 0};
+    loop_state ls = {1, 0, 0, 0, 0, 0, 0};
     int small_streak = 0; /* consecutive plain push levels that stayed small */
     int slow_streak = 0;  /* consecutive small levels that did not double */
     int32_t level = 0;
@@ -1135,7 +1161,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
     const int spec = policy == ALBBA_SWITCH_HEURISTIC || policy == ALBBA_SWITCH_LEARNED ||
                      policy == ALBBA_SWITCH_SCRIPT;
     const int use_sel = policy != ALBBA_SWITCH_HEURISTIC; /* kernels queued ahead read sel_choice */
-    ls.have_prefix = spec; /* the root's, from the reset */
+    ls.have_prefix = policy != ALBBA_SWITCH_BEST; /* the root's, from the reset */
     unsigned int seq = 0;
     /* kernels already queued for the coming level: the choice whose pull is
      * queued, or -1; whether the push kernels are, and the largest frontier
@@ -1188,15 +1214,13 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
                     /* a choice 4x slower than the best so far cannot win:
                      * one trial is enough to rank it */
                     if (r == 1 && t[0] > 4.0f * best) { nr = 1; break; }
-                    /* the state after the select kernel, the preparation the
-                     * deployed loop queues behind it for every choice (zero
-                     * next, unvisited-word list, frontier summary), then the
-                     * choice's own kernels -- the only part that is timed, as
-                     * only that part differs between choices when deployed */
-                    if ((rc = albd_d2d(d, G->st.visited, G->scratch_visited, sizeof(uint64_t) * (size_t)G->g.nwords)) ||
-                        (rc = albd_d2d(d, G->st.ctr, G->scratch_ctr, sizeof(albd_counters))) ||
-                        (rc = albd_level_begin_flags(d, &G->g, &G->st, LB_SLOTS)) || (rc = prep_level(G, &ls, level)) ||
-                        (rc = albd_event_record(d, 4)) || (rc = run_main(G, &ls, c, level, frontier, 0, INT64_MAX)) ||
+                    /* the choice's own kernels are the only part that is
+                     * timed, as only that part differs between choices when
+                     * deployed; a push lists the next queue where the
+                     * deployed one does */
+                    loop_state t_ls = ls;
+                    if ((rc = trial_prep(G, &t_ls, c, level, frontier)) || (rc = albd_event_record(d, 4)) ||
+                        (rc = run_main(G, &t_ls, c, level, frontier, 0, queue_max)) ||
                         (rc = albd_event_record(d, 5)) || (rc = albd_event_elapsed(d, 4, 5, &t[r])))
                         return albba_fail(rc, "bfs: %s", albd_error());
                 }
@@ -1374,7 +1398,11 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
                 if (stats->swept) stats->swept[lv] = j == 0 ? swept : -1;
             }
         }
-        if (!spec) commit_pointers(G, &ls, choice, 1, 0);
+        if (!spec) {
+            /* (a BEST or FIXED push lists the queue whatever its size) */
+            commit_pointers(G, &ls, choice, 1, policy != ALBBA_SWITCH_BEST);
+            ls.unlisted = choice == ALBBA_CHOICE_PUSH && first_edges > queue_max;
+        }
         commit_counts(&ls, choice, &sums);
         /* (a run of levels says nothing about the growth at its end) */
         frontier_prev = small ? (int64_t)hc->frontier : frontier;

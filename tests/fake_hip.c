@@ -25,6 +25,8 @@ API int fake_wrong_device;               /* launches on a stream of another than
 API int fake_levels, fake_level;
 API long long fake_frontier[MAX_LEVELS + 1], fake_edges[MAX_LEVELS + 1];
 API char fake_log[1 << 22];              /* kernel names, one a line */
+API long long fake_build_max[MAX_LEVELS * 64]; /* of the push finalizes, in turn */
+API int fake_finalizes;
 static size_t log_len;
 
 API void fake_log_reset(void)
@@ -115,6 +117,8 @@ API hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args
     /* a pull costs ten of the others, so that a push is the fastest choice */
     now += strstr(name, "k_pull") ? 10 : 1;
     if (strstr(name, "k_select")) select_level(args);
+    if (strstr(name, "k_words_to_queueILb1") && fake_finalizes < MAX_LEVELS * 64)
+        fake_build_max[fake_finalizes++] = *(const long long *)args[4];
     return hipSuccess;
 }
 

@@ -148,3 +148,46 @@ def test_batch_memory_of_small_graphs(program, count):
         b.close()
         ctx.close()
     """)
+
+
+# a BFS that pushes on every level: a frontier beyond the one-block scan, one
+# with too many edges for its queue to be listed, and the push after that
+PUSHES = "levels([1, 10, 9000, 11000, 11500, 50], [5, 9000, 30000, 11000, 11900, 100])"
+
+
+def test_best_times_a_push_as_it_is_deployed(program):
+    """The BEST policy's time of a push covers the kernels that the same push
+    costs in the level loop (every kernel takes 1 ms here): no scan of a queue
+    that was listed with its prefix, and no queue listed where the loop lists
+    none."""
+    program(f"""
+        g = A.DeviceGraph.build(A.Context(0), empty(300000), 64, 4096, 1)
+        {PUSHES}
+        done = get("fake_finalizes", C.c_int)
+        loop = g.bfs(0, policy=A.SWITCH_HEURISTIC, time_levels=True, small_frontier_edges=0, results=False)
+        caps = list(get("fake_build_max", n=4096)[:done.value])
+        done.value = 0
+        best = g.bfs(0, policy=A.SWITCH_BEST, timing_reps=1, results=False)
+        assert list(loop["choice"]) == [A.CHOICE_PUSH] * 6 == list(best["choice"])
+        assert list(best["choice_ms"][:, A.CHOICE_PUSH]) == list(loop["level_ms"]), (best["choice_ms"], loop["level_ms"])
+        # the trial of each level, with the loop's limit, then the committed
+        # push, which lists every queue
+        assert list(get("fake_build_max", n=4096)[:done.value]) == [x for c in caps for x in (c, 2**63 - 1)]
+    """)
+
+
+def test_fixed_pushes_scan_no_queue(program):
+    """A queue that the last push listed has its degree prefix: the pushes of
+    the FIXED policy do not scan it again."""
+    program(f"""
+        g = A.DeviceGraph.build(A.Context(0), empty(300000), 64, 4096, 1)
+        {PUSHES}
+        fake.fake_log_reset()
+        r = g.bfs(0, policy=A.SWITCH_FIXED, fixed_choice=A.CHOICE_PUSH, results=False)
+        assert r["num_levels"] == 6
+        assert not [k for k in kernels() if "k_scan" in k]
+        # a pull in front of a push: the queue and its prefix come from the bitmap
+        fake.fake_log_reset()
+        g.bfs(0, policy=A.SWITCH_SCRIPT, script=[0, 1, 0, 0, 2, 0], results=False)
+        assert not [k for k in kernels() if "k_scan" in k]
+    """)
