@@ -121,8 +121,9 @@ ALBBA_API void sellcs_preprocess(const SparseMatrixCSR *csr, SparseMatrixSELLCS 
 ALBBA_API void free_sellcs_struct(SparseMatrixSELLCS *sellcs);
 /* bfs/src/bfs.h:13 -- BFS from vertex 0 on the GPU.  Fills frontier[level]
  * (frontier size per level), *num_iter, *num_vex, *bfs_time (ms, level loop
- * only), *conv_time (ms, SELL build) and iter_times[level] (ms); sets *nnzx
- * to 0 at the end as the reference loop does.  bfs_x is not touched. */
+ * only), *conv_time (ms, SELL build, on the device as a rule: without the
+ * upload of the CSR) and iter_times[level] (ms); sets *nnzx to 0 at the end
+ * as the reference loop does.  bfs_x is not touched. */
 ALBBA_API void run_custom_bfs_test(const SparseMatrixCSR *matrix, elem_t *bfs_x,
                                    int *colidx_x, int *nnzx, int *frontier,
                                    int *num_vex, double *conv_time,

@@ -191,3 +191,18 @@ def test_fixed_pushes_scan_no_queue(program):
         g.bfs(0, policy=A.SWITCH_SCRIPT, script=[0, 1, 0, 0, 2, 0], results=False)
         assert not [k for k in kernels() if "k_scan" in k]
     """)
+
+
+def test_conv_time_is_the_layout_build(program):
+    """conv_time of the reference's entry point is the SELL build: what the
+    device build reports for the same matrix (kernels take 1 ms here), without
+    the upload and the BFS state around it."""
+    program("""
+        g = empty(1000)
+        sigma = 16384  # the reference's sigma_window
+        want = A.DeviceGraph.build(A.Context(0), g, 64, sigma, 1).build_report["build_ms"]
+        assert want >= 5 and want == int(want)
+        levels([1], [0])
+        r = A.run_custom_bfs_test(1000, np.zeros(1001, np.int32), np.zeros(0, np.int32))
+        assert r["conv_time"] == want, (r["conv_time"], want)
+    """)
