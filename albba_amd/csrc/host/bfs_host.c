@@ -354,11 +354,11 @@ int albba_graph_build_ex(albba_ctx *ctx, const albba_csr *cg, int C, int sigma, 
     G->sigma = sigma;
     G->order_flags = flags;
     albd_ctx *d = ctx->d;
-    const double t0 = albba_now_ms();
     int64_t *rp = NULL;
     int32_t *col = NULL;
     int rc = albd_malloc(d, sizeof(int64_t) * ((size_t)cg->n + 1), (void **)&rp);
     if (!rc) rc = albd_malloc(d, sizeof(int32_t) * (size_t)(cg->nnz > 0 ? cg->nnz : 1), (void **)&col);
+    const double t0 = albba_now_ms();
     if (!rc) rc = albba_h2d(d, rp, cg->row_ptr, sizeof(int64_t) * ((size_t)cg->n + 1));
     if (!rc) rc = albba_h2d(d, col, cg->col, sizeof(int32_t) * (size_t)cg->nnz);
     const double t1 = albba_now_ms();

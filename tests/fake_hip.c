@@ -10,6 +10,7 @@
 #include <stdlib.h>
 #include <string.h>
 #include <sys/mman.h>
+#include <unistd.h>
 
 #include "../albba_amd/csrc/albd.h"
 
@@ -21,6 +22,7 @@
 API long long fake_capacity = 1ll << 40; /* bytes of one device */
 API long long fake_live_bytes[DEVICES], fake_live_blocks[DEVICES];
 API long long fake_pinned_max = 1ll << 40; /* larger pinned blocks fail */
+API int fake_malloc_us;                  /* what an allocation takes */
 API int fake_wrong_device;               /* launches on a stream of another than the current device */
 API int fake_levels, fake_level;
 API long long fake_frontier[MAX_LEVELS + 1], fake_edges[MAX_LEVELS + 1];
@@ -133,6 +135,7 @@ typedef struct {
 API hipError_t hipMalloc(void **p, size_t bytes)
 {
     *p = NULL;
+    if (fake_malloc_us) usleep((useconds_t)fake_malloc_us);
     if (fake_live_bytes[current] + (long long)bytes > fake_capacity) return hipErrorOutOfMemory;
     /* (large ones by mmap, so that what is not touched takes no memory) */
     char *m = bytes < BIG ? (char *)calloc(1, bytes + HEAD) : (char *)mmap(NULL, bytes + HEAD, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);

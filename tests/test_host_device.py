@@ -206,3 +206,13 @@ def test_conv_time_is_the_layout_build(program):
         r = A.run_custom_bfs_test(1000, np.zeros(1001, np.int32), np.zeros(0, np.int32))
         assert r["conv_time"] == want, (r["conv_time"], want)
     """)
+
+
+def test_upload_time_is_the_copy(program):
+    """upload_ms of a build is the CSR's way to the device, without the
+    allocation of its arrays (here 50 ms each)."""
+    program("""
+        get("fake_malloc_us", C.c_int).value = 50000
+        t = A.DeviceGraph.build(A.Context(0), empty(10), 64, 64, 1).build_report["upload_ms"]
+        assert t < 50, t
+    """)
