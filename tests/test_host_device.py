@@ -216,3 +216,25 @@ def test_upload_time_is_the_copy(program):
         t = A.DeviceGraph.build(A.Context(0), empty(10), 64, 64, 1).build_report["upload_ms"]
         assert t < 50, t
     """)
+
+
+def test_without_pinned_memory(program):
+    """Where the pinned level log and the copies' stages cannot be allocated, a
+    small graph's BFS runs in the level loop and results come by plain copies;
+    where they can again, in one workgroup."""
+    program("""
+        ctx = A.Context(0)
+        get("fake_pinned_max").value = 1 << 18
+        g = A.DeviceGraph.build(ctx, empty(5000), 64, 64, 1)
+        big = A.DeviceGraph.build(ctx, empty(1 << 20), 64, 64, 1)
+        levels([1, 3], [2, 0])
+        fake.fake_log_reset()
+        r = g.bfs(0)
+        assert r["num_levels"] == 2 and r["level"].size == 5000
+        assert [k for k in kernels() if "k_bfs_reset" in k] and not [k for k in kernels() if "k_bfs_one" in k]
+        assert big.bfs(0)["parent"].size == 1 << 20
+        get("fake_pinned_max").value = 1 << 40
+        fake.fake_log_reset()
+        g.bfs(0)
+        assert [k for k in kernels() if "k_bfs_one" in k] and not [k for k in kernels() if "k_bfs_reset" in k]
+    """)
