@@ -266,8 +266,10 @@ ALBD_HIDDEN int albd_bfs_init(albd_ctx *c, const albd_graph *g, const albd_state
 /* if_done: queued before the host knew the BFS had ended; the kernel runs only
  * if the last select kernel found the frontier empty */
 ALBD_HIDDEN int albd_to_vertex_order(albd_ctx *c, const albd_graph *g, const albd_state *st, int if_done);
-/* zero st->next (and, flag 1, the per-level slot counters) */
-ALBD_HIDDEN int albd_level_begin(albd_ctx *c, const albd_graph *g, const albd_state *st);
+/* zero st->next and, by flag, the per-level slot counters (ALBD_LB_SLOTS) or
+ * what the small-frontier kernel counts in (ALBD_LB_SMALL) */
+enum { ALBD_LB_SLOTS = 1, ALBD_LB_SMALL = 8 };
+ALBD_HIDDEN int albd_level_begin(albd_ctx *c, const albd_graph *g, const albd_state *st, int flags);
 
 /* pull variants */
 enum { ALBD_PULL_ALL = 0, ALBD_PULL_LIST = 1, ALBD_PULL_LIST_CB = 2 };
@@ -339,12 +341,10 @@ ALBD_HIDDEN int albd_push_small(albd_ctx *c, const albd_graph *g, const albd_sta
                                 int32_t max_levels, int32_t blocks, uint32_t spin_limit);
 /* end of a level: sum the slot counters into ctr->frontier*, update the
  * running totals, compute the 12 features and the next level's choice
- * (MLP argmin when sel->params is set, else the reference heuristic) */
-ALBD_HIDDEN int albd_select(albd_ctx *c, const albd_graph *g, const albd_state *st,
-                            const albd_select_args *sel);
-/* albd_select, then the counters on the host (albd_host_counters): the
- * kernel posts them into a pinned host-coherent mailbox and the host polls
- * it, instead of a copy and a stream synchronisation (synchronous) */
+ * (MLP argmin when sel->params is set, else the reference heuristic), then the
+ * counters on the host (albd_host_counters): the kernel posts them into a
+ * pinned host-coherent mailbox and the host polls it, instead of a copy and a
+ * stream synchronisation (synchronous) */
 ALBD_HIDDEN int albd_select_read(albd_ctx *c, const albd_graph *g, const albd_state *st,
                                  const albd_select_args *sel);
 /* the launch half of albd_select_read (asynchronous); albd_mail_wait(seq)

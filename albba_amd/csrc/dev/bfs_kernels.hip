@@ -590,23 +590,22 @@ __global__ __launch_bounds__(kSelectBlock) void k_select(albd_graph g, albd_stat
 }
 
 // Zero st.next (the select kernel has moved the counters and zeroed the
-// slots).  LB_SLOTS: zero the slots too (trial runs of one level);
-// LB_SMALL: the small-frontier kernel follows; zero its grid state, its
+// slots).  ALBD_LB_SLOTS: zero the slots too (trial runs of one level);
+// ALBD_LB_SMALL: the small-frontier kernel follows; zero its grid state, its
 // levels' counters and the error flag here instead of in launches of their own.
-enum { LB_SLOTS = 1, LB_SMALL = 8 };
 
 __global__ __launch_bounds__(kBlock) void k_level_begin(albd_state st, int32_t nwords, int flags)
 {
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < nwords;
          i += (int64_t)gridDim.x * kBlock)
         st.next[i] = 0;
-    if (flags & LB_SLOTS) {
+    if (flags & ALBD_LB_SLOTS) {
         unsigned long long *slots = reinterpret_cast<unsigned long long *>(st.slots);
         for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
              i < (int64_t)(ALBD_NSLOT * sizeof(albd_slot) / 8); i += (int64_t)gridDim.x * kBlock)
             slots[i] = 0;
     }
-    if (flags & LB_SMALL) {
+    if (flags & ALBD_LB_SMALL) {
         const int64_t i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x, step = (int64_t)gridDim.x * kBlock;
         unsigned long long *p = reinterpret_cast<unsigned long long *>(st.persist);
         static_assert(sizeof(albd_persist) % 8 == 0, "cleared by word");
@@ -1425,7 +1424,7 @@ int albd_to_vertex_order(albd_ctx *c, const albd_graph *g, const albd_state *st,
     return 0;
 }
 
-int albd_level_begin_flags(albd_ctx *c, const albd_graph *g, const albd_state *st, int flags)
+int albd_level_begin(albd_ctx *c, const albd_graph *g, const albd_state *st, int flags)
 {
     int64_t blocks = ((int64_t)g->nwords + kBlock - 1) / kBlock;
     int64_t cap = (int64_t)albd_num_cus(c) * 8;
@@ -1433,11 +1432,6 @@ int albd_level_begin_flags(albd_ctx *c, const albd_graph *g, const albd_state *s
                        dim3(kBlock), 0, albd_stream(c), *st, g->nwords, flags);
     HIPCHK(hipGetLastError());
     return 0;
-}
-
-int albd_level_begin(albd_ctx *c, const albd_graph *g, const albd_state *st)
-{
-    return albd_level_begin_flags(c, g, st, 0);
 }
 
 int albd_build_active(albd_ctx *c, const albd_graph *g, albd_state *st, int from_list,
@@ -1613,17 +1607,9 @@ int albd_push_small(albd_ctx *c, const albd_graph *g, const albd_state *st, int3
     if (blocks <= 0) blocks = g->n < (1 << 20) ? 16 : (g->n < 5 << 20 ? 32 : 64);
     if (blocks > cap) blocks = (int32_t)cap;
     // the grid state, the levels' counters and the error flag were zeroed by
-    // the level-begin kernel (LB_SMALL)
+    // the level-begin kernel (ALBD_LB_SMALL)
     SmallArgs a{*g, *st, level0, max_levels, edge_cap, vertex_cap, spin_limit};
     hipLaunchKernelGGL(k_push_small, dim3(blocks), dim3(kListBlock), 0, albd_stream(c), a);
-    HIPCHK(hipGetLastError());
-    return 0;
-}
-
-int albd_select(albd_ctx *c, const albd_graph *g, const albd_state *st, const albd_select_args *sel)
-{
-    hipLaunchKernelGGL(k_select, dim3(1), dim3(kSelectBlock), 0, albd_stream(c), *g, *st, *sel,
-                       (albd_counters *)nullptr, 0u);
     HIPCHK(hipGetLastError());
     return 0;
 }

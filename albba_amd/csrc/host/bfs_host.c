@@ -709,11 +709,6 @@ void albba_bfs_opts_default(albba_bfs_opts *o)
     o->small_frontier_edges = 65536;
 }
 
-/* k_level_begin flags; the select kernel moves the queue/list counters from
- * one level to the next and zeroes the slots */
-enum { LB_SLOTS = 1, LB_SMALL = 8 };
-int albd_level_begin_flags(albd_ctx *c, const albd_graph *g, const albd_state *st, int flags);
-
 typedef struct loop_state {
     int have_queue;       /* st.queue holds the frontier                */
     int have_prefix;      /* st.prefix its degree prefix (not kept where
@@ -727,21 +722,16 @@ typedef struct loop_state {
 } loop_state;
 
 typedef struct level_sums {
-    int64_t next_count, next_edges, next_words, scanned, words, bypassed, col_bypassed;
-    int64_t qnext_len, active_len, queue_len, push_edges;
+    int64_t scanned, words, bypassed, col_bypassed, active_len, queue_len, push_edges;
 } level_sums;
 
 static void sum_counters(const albd_counters *h, level_sums *o)
 {
     /* the select kernel has summed the slot counters of the level */
-    o->next_count = (int64_t)h->frontier;
-    o->next_edges = (int64_t)h->frontier_edges;
-    o->next_words = (int64_t)h->frontier_words;
     o->scanned = (int64_t)h->scanned;
     o->words = (int64_t)h->words;
     o->bypassed = (int64_t)h->bypassed;
     o->col_bypassed = (int64_t)h->col_bypassed;
-    o->qnext_len = (int64_t)h->qnext_len;
     o->active_len = (int64_t)h->active_len;
     o->queue_len = (int64_t)(h->queue_len & 0xffffffffull);
     o->push_edges = (int64_t)h->push_edges;
@@ -754,7 +744,7 @@ static int run_level(albba_graph *G, const loop_state *ls, int choice, int32_t l
 {
     albd_ctx *d = G->ctx->d;
     /* slots too: trial runs of one level start from zero each time */
-    int rc = albd_level_begin_flags(d, &G->g, &G->st, LB_SLOTS);
+    int rc = albd_level_begin(d, &G->g, &G->st, ALBD_LB_SLOTS);
     if (rc) return rc;
     if (choice == ALBBA_CHOICE_PUSH) {
         if (!ls->have_queue) rc = albd_front_to_queue(d, &G->g, &G->st);
@@ -876,7 +866,7 @@ static int trial_prep(albba_graph *G, loop_state *ls, int choice, int32_t level,
     int rc;
     if ((rc = albd_d2d(d, G->st.visited, G->scratch_visited, sizeof(uint64_t) * (size_t)G->g.nwords)) ||
         (rc = albd_d2d(d, G->st.ctr, G->scratch_ctr, sizeof(albd_counters))) ||
-        (rc = albd_level_begin_flags(d, &G->g, &G->st, LB_SLOTS)) || (rc = prep_level(G, ls, level)))
+        (rc = albd_level_begin(d, &G->g, &G->st, ALBD_LB_SLOTS)) || (rc = prep_level(G, ls, level)))
         return rc;
     if (choice != ALBBA_CHOICE_PUSH || !ls->have_queue) return 0;
     if (ls->unlisted) {
@@ -892,12 +882,10 @@ static int trial_prep(albba_graph *G, loop_state *ls, int choice, int32_t level,
  * number of levels run in *nlev; afterwards the state is that of one
  * finished push level (queue_next holds the last frontier's queue). */
 static int run_small(albba_graph *G, const loop_state *ls, int32_t level, int64_t frontier,
-                     int64_t edge_cap, int64_t vertex_cap, int32_t blocks, int mark, int prepped,
-                     int *nlev)
+                     int64_t edge_cap, int64_t vertex_cap, int32_t blocks, int mark, int *nlev)
 {
     albd_ctx *d = G->ctx->d;
-    (void)prepped; /* the counters moved in the select kernel either way */
-    int rc = albd_level_begin_flags(d, &G->g, &G->st, LB_SMALL);
+    int rc = albd_level_begin(d, &G->g, &G->st, ALBD_LB_SMALL);
     if (rc) return rc;
     if (!ls->have_queue && (rc = albd_front_to_queue(d, &G->g, &G->st))) return rc;
     if (mark && (rc = albd_event_record(d, 6))) return rc;
@@ -1266,7 +1254,7 @@ static int bfs_run(albba_ctx *ctx, albba_graph *G, int32_t root, const albba_bfs
         if (opts.time_levels && (rc = albd_event_record(d, 2))) return albba_fail(rc, "bfs: %s", albd_error());
         if (small)
             rc = run_small(G, &ls, level, frontier, opts.small_frontier_edges, push_vertex_cap,
-                           opts.small_frontier_blocks, opts.time_levels, spec, &nlev);
+                           opts.small_frontier_blocks, opts.time_levels, &nlev);
         else if (spec) {
             const int ran = choice == queued_pull ||
                             (queued_push && choice == ALBBA_CHOICE_PUSH && frontier <= queued_push_max);
