@@ -174,7 +174,8 @@ int albd_trim(albd_ctx *c)
     (void)hipSetDevice(c->device);
     std::lock_guard<std::mutex> guard(c->mem_lock);
     const int any = c->kept.empty() ? 0 : 1;
-    while (!c->kept.empty()) drop_one(c, c->kept.begin());
+    // oldest first: by size, a context of an RMAT s17 graph took 0.4 ms more
+    while (!c->oldest.empty()) drop_one(c, c->oldest.begin()->second);
     return any;
 }
 
