@@ -20,8 +20,8 @@
 // finds pmin[v] still all ones sets v in the next bitmap; a word pass then
 // writes level/parent and builds the next queue.
 #include "dev_common.h"
-// one own edge a thread (512 threads of two: 4 096 x 4 096 grid 5.6 us a level
-// against 5.4; 256 of two or four 6.5)
+// one own edge a thread (512 threads of two: 4 096 x 4 096 grid, a root of 7 120
+// levels, 5.6 us a level against 5.4; 256 of two or four 6.5)
 #define PUSH_LIST_BLOCK 1024
 #include "push_lists.h"
 #include "select_dev.h"
@@ -1160,9 +1160,11 @@ __global__ __launch_bounds__(kBlock) void k_push_expand(albd_graph g, albd_state
 // one workgroup carried the first 4 096 levels of a 4 096 x 4 096 grid alone
 // and the kernel took 8.2 us per level instead of 5.5.
 //
-// Measured on grids of 0.6, 4.2 and 16.8 M vertices: 4.1, 4.5 and 5.4 us per
-// level, where a queue in memory between the levels, with its reservations
-// and a counting barrier, took 11.8, 12.3 and 13.6.  Of the 4 us about 1.3
+// Measured on grids of 0.6, 4.2 and 16.8 M vertices, one root each: 4.2, 4.4
+// and 5.4 us per level, where a queue in memory between the levels, with its
+// reservations and a counting barrier, took 11.8, 12.3 and 13.6.  (32 roots of
+// the largest: 5.4 from the ones with most levels, 7 410, to 6.4 from those with
+// fewest, 4 536, whose levels are wider.)  Of the 4 us about 1.3
 // are the atomic and the appends, 2.0 the loads behind the barrier (two
 // dependent misses) and 0.7 what the barrier waits beyond them.  Keeping all
 // workgroups on one XCD changed nothing at 0.6 M vertices (4.1 us) and cost at
